@@ -96,6 +96,21 @@ std::vector<fk_abi_param> gemm_params() {
           FK_PA(S, ldc, 2, "u32"),     FK_P(S, act, "u32")};
 }
 
+// The forms of the GEMM of few rows (fk_skinny.h): row and column blocks of a
+// tile, the wavefronts its k is split among.
+struct SkinnyForm {
+  const char *name;
+  uint32_t mb, nb, waves;
+};
+const SkinnyForm skinny_forms[] = {{"m1n1", 1, 1, 8}, {"m1n2", 1, 2, 8}, {"m2n1", 2, 1, 8}, {"m2n2", 2, 2, 8},
+                                   {"m2n4", 2, 4, 4}, {"m4n2", 4, 2, 8}, {"m4n4", 4, 4, 4}, {"m4n8", 4, 8, 4},
+                                   {"m8n4", 8, 4, 4}, {"m8n8", 8, 8, 4}};
+const char *const skinny_modes[] = {"store", "add", "store_keys", "silu_mul", "qkv_rope", "qkv_rope_paged"};
+
+bool skinny_pairs(const char *mode) {
+  return std::strcmp(mode, "silu_mul") == 0 || std::strncmp(mode, "qkv_rope", 8) == 0;
+}
+
 std::vector<Entry> build() {
   std::vector<Entry> out;
   auto add = [&](const std::string &entry, uint32_t threads, std::vector<fk_abi_buffer> b,
@@ -299,6 +314,25 @@ std::vector<Entry> build() {
          buf("rope", "read", "f32")},
         p, sizeof(SP));
   }
+  for (const SkinnyForm &f : skinny_forms)
+    for (const char *mode : skinny_modes) {
+      if (f.nb == 1 && skinny_pairs(mode)) continue;
+      using S = fk_skinny_params;
+      std::vector<fk_abi_param> p = gemm_params();
+      p.insert(p.end(), {FK_P(S, live, "u32"), FK_P(S, run_chunks, "u32"), FK_P(S, run, "u32"), FK_P(S, apart, "u32"),
+                         FK_PX(S, r.kv_heads, "kv_heads", "u32"), FK_PX(S, r.rope_rows, "rope_rows", "u32"),
+                         FK_PX(S, r.length, "length", "u32"), FK_PX(S, r.slots, "slots", "u32"),
+                         FK_PX(S, r.cache_bf16, "cache_bf16", "u32"), FK_PX(S, r.staged, "staged", "u32"),
+                         FK_PX(S, pg.block_size, "block_size", "u32"), FK_PX(S, pg.table_len, "table_len", "u32"),
+                         FK_PX(S, pg.blocks, "blocks", "u32")});
+      const char *ct = skinny_pairs(mode) ? "f16" : "f32";
+      add(std::string("fk_skinny_") + mode + "_" + f.name, 64 * f.waves,
+          {buf("a", "read", "f16"), buf("b0", "read", "f16"), buf("b1", "read", "f16"), buf("b2", "read", "f16"),
+           buf("c0", "write", ct), buf("c1", "read_write", ct), buf("c2", "read_write", ct), buf("r0", "read", "f32"),
+           buf("position", "read", "u32"), buf("slot", "read", "u32"), buf("rope", "read", "f32"),
+           buf("keys", "write", "u64")},
+          p, sizeof(S));
+    }
   {
     using S = fk_prefill_gather_params;
     add("fk_prefill_gather", 256, {buf("table", "read", "f16"), buf("tokens", "read", "u32"), buf("x", "write", "f32")},
@@ -786,6 +820,61 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
       need.push_back({"rope", 0});
       for (Need &n : need)
         if (std::strcmp(n.name, "c1") == 0 || std::strcmp(n.name, "c2") == 0) n.bytes = pool;
+    }
+  } else if (std::strncmp(entry, "fk_skinny_", 10) == 0) {
+    fk_skinny_params p;
+    std::memcpy(&p, params, sizeof p);
+    const char *form = std::strrchr(entry, '_') + 1;
+    const std::string mode(entry + 10, form - 1);
+    const SkinnyForm *f = nullptr;
+    for (const SkinnyForm &s : skinny_forms)
+      if (std::strcmp(s.name, form) == 0) f = &s;
+    const bool silu = mode == "silu_mul", paged = mode == "qkv_rope_paged", qkv = paged || mode == "qkv_rope";
+    const fk_gemm_params &g = p.g;
+    const uint32_t cols = g.n_anchors >= 1 && g.n_anchors <= 3 ? g.first_col[g.n_anchors] : 0;
+    bool shape = f && g.m && g.m % 256 == 0 && g.k && g.k % 64 == 0 && cols && p.live && p.run_chunks && p.apart &&
+                 (uint64_t)g.m * g.k * 2 < 0xfffffff0u && (silu ? g.n_anchors == 1 && g.ldc[0] == cols && cols % 128 == 0
+                                                                : g.first_col[0] == 0);
+    for (uint32_t j = 0; shape && !silu && j < g.n_anchors; j++)
+      shape = g.first_col[j + 1] > g.first_col[j] && (g.first_col[j + 1] - g.first_col[j]) % 256 == 0 &&
+              g.ldc[j] >= g.first_col[j + 1] - g.first_col[j];
+    // SiLU·mul: the pair's 2 cols weight rows.
+    const uint64_t tiles_n = shape ? (uint64_t)(silu ? 2 * cols : cols) / (16 * f->nb) : 0;
+    const uint64_t tiles_m = shape ? ((uint64_t)p.live + f->mb - 1) / f->mb : 0;
+    if (!shape || (uint64_t)groups != (tiles_n + 7) / 8 * 8 * tiles_m)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u rows, k %u, %u anchors over %u columns, %u chunks of rows in %u threadgroups",
+                 entry, g.m, g.k, g.n_anchors, cols, p.live, groups);
+    const uint64_t m = g.m;
+    need.push_back({"a", m * g.k * 2});
+    static const char *bn[3] = {"b0", "b1", "b2"}, *cn[3] = {"c0", "c1", "c2"};
+    for (uint32_t j = 0; j < g.n_anchors; j++) {
+      const uint64_t wide = silu ? 2ull * cols : g.first_col[j + 1] - g.first_col[j];
+      need.push_back({bn[j], wide * g.k * 2});
+      if (!qkv || j == 0) need.push_back({cn[j], m * g.ldc[j] * (silu || qkv ? 2 : 4)});
+    }
+    if (mode == "add") {
+      if (g.n_anchors != 1) return bad(err, cap, FK_ERR_ARG, "%s: %u anchors", entry, g.n_anchors);
+      need.push_back({"r0", m * g.ldc[0] * 4});
+    }
+    if (mode == "store_keys") {
+      if (g.n_anchors != 1 || g.ldc[0] != cols)
+        return bad(err, cap, FK_ERR_ARG, "%s: %u anchors, %u columns in rows of %u", entry, g.n_anchors, cols, g.ldc[0]);
+      need.push_back({"keys", m * tiles_n * 8});
+    }
+    if (qkv) {
+      if (g.n_anchors != 3 || p.r.kv_heads == 0 || p.r.rope_rows == 0 || g.ldc[1] != p.r.kv_heads * 64 ||
+          g.ldc[2] != p.r.kv_heads * 64 || (paged ? !p.pg.block_size || !p.pg.table_len || !p.pg.blocks || p.r.staged
+                                                  : !p.r.staged && (!p.r.length || !p.r.slots)))
+        return bad(err, cap, FK_ERR_ARG, "%s: %u anchors, %u kv heads of rows of %u and %u", entry, g.n_anchors,
+                   p.r.kv_heads, g.ldc[1], g.ldc[2]);
+      const uint64_t cache = p.r.staged ? m * p.r.kv_heads * 128
+                             : paged    ? (uint64_t)p.pg.blocks * p.r.kv_heads * p.pg.block_size * 128
+                                        : (uint64_t)p.r.slots * p.r.kv_heads * p.r.length * 128;
+      need.push_back({"c1", cache});
+      need.push_back({"c2", cache});
+      need.push_back({"position", m * 4});
+      need.push_back({"slot", m * 4 * (paged ? p.pg.table_len : 1)});
+      need.push_back({"rope", (uint64_t)p.r.rope_rows * 256});
     }
   } else if (std::strncmp(entry, "fk_prefill_attend_g", 19) == 0 ||
              std::strncmp(entry, "fk_prefill_attend_f16_g", 23) == 0) {

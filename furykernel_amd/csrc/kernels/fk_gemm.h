@@ -267,11 +267,7 @@ __device__ __forceinline__ void gemm_tile(const _Float16 *__restrict__ a, const 
   if (MODE == FK_GEMM_SILU_MUL) {
     uint16_t *out = reinterpret_cast<uint16_t *>(c0);
     const uint32_t ncols = p.ldc[0];
-    // silu(g) u = g / (1 + e^-g) · u, or gelu(g) u = 0.5 g (1 + tanh(y)) u
-    // with tanh(y) = 1 - 2 / (1 + e^2y), with the hardware's exp and
-    // reciprocal (a few ulp of binary32), then rounded once to f16 (2^-11):
-    // the f16 rounding bounds the error.  An exponential overflowing gives
-    // the limits (silu 0, tanh 1).  The activation is a branch on the
+    // The activation (fk::act_hw) is a branch on the
     // launch's uniform parameter around the whole epilogue, each side
     // unrolled, so a tile pays for its own activation's exponentials only.
     auto act_mul_tiles = [&](auto gelu_tag) {
@@ -287,15 +283,7 @@ __device__ __forceinline__ void gemm_tile(const _Float16 *__restrict__ a, const 
           for (int r = 0; r < 4; r++) {
             const float gt = acc[i][j][r];
             const float u = acc[i][j + 4][r];
-            float a;
-            if constexpr (GELU) {
-              const float y = 0.7978845608028654f * (gt + ((0.044715f * gt) * gt) * gt);
-              const float th = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __expf(2.0f * y));
-              a = (0.5f * gt) * (1.0f + th);
-            } else {
-              a = gt * __builtin_amdgcn_rcpf(1.0f + __expf(-gt));
-            }
-            h[r] = fk::to_f16(a * u);
+            h[r] = fk::to_f16(fk::act_hw<GELU>(gt) * u);
           }
           uint2 w;
           w.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);

@@ -7,3 +7,4 @@
 #include "fk_step.h"
 #include "fk_gemm.h"
 #include "fk_prefill.h"
+#include "fk_skinny.h"

@@ -26,4 +26,20 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void *base, size_
 // binary32 -> binary16, to nearest even (v_cvt_f16_f32).
 __device__ __forceinline__ uint16_t to_f16(float x) { return __builtin_bit_cast(uint16_t, (_Float16)x); }
 
+// The gated MLP's activation of a matrix product's element, on its way to f16:
+// silu(g) = g / (1 + e^-g), or gelu(g) = 0.5 g (1 + tanh(y)) with tanh(y) =
+// 1 - 2 / (1 + e^2y), with the hardware's exp and reciprocal (a few ulp of
+// binary32): the f16 rounding after it (2^-11) bounds the error.  An
+// exponential overflowing gives the limits (silu 0, tanh 1).
+template <bool GELU>
+__device__ __forceinline__ float act_hw(float g) {
+  if constexpr (GELU) {
+    const float y = 0.7978845608028654f * (g + ((0.044715f * g) * g) * g);
+    const float th = 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + __expf(2.0f * y));
+    return (0.5f * g) * (1.0f + th);
+  } else {
+    return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));
+  }
+}
+
 }  // namespace fk

@@ -105,6 +105,15 @@ class GemmQkvParams(ctypes.Structure):
                                       ("cache_bf16", ctypes.c_uint32), ("staged", ctypes.c_uint32)]
 
 
+class SkinnyParams(ctypes.Structure):
+    """fk_skinny_params: the GEMM's, the rows it makes, then the QKV
+    epilogue's RoPE, caches and paging."""
+    _fields_ = GemmParams._fields_ + [("live", ctypes.c_uint32), ("run_chunks", ctypes.c_uint32),
+                                      ("run", ctypes.c_uint32), ("apart", ctypes.c_uint32)] + \
+        GemmQkvParams._fields_[len(GemmParams._fields_):] + \
+        [("block_size", ctypes.c_uint32), ("table_len", ctypes.c_uint32), ("blocks", ctypes.c_uint32)]
+
+
 class PrefillGatherParams(ctypes.Structure):
     _fields_ = [("rows", ctypes.c_uint32), ("width", ctypes.c_uint32), ("table_rows", ctypes.c_uint32),
                 ("table_f16", ctypes.c_uint32), ("factor", ctypes.c_float)]
@@ -322,6 +331,24 @@ STEP_GEMV_ENTRIES = tuple(f"{shape}_p{pro}_e{epi}" for shape, pairs in STEP_GEMV
 STEP_GEMV_BUFFERS = ("w0", "w1", "w2", "y0", "y1", "y2", "src", "src2", "gamma", "table", "token", "res", "res_table",
                      "res_token", "epi_out", "arg")
 
+# The GEMM of few rows (fk_skinny.h): fk_skinny_<mode>_<form>, a form being the
+# (16-row, 16-column) blocks of a tile and the wavefronts its k is split
+# among; forms of one column block have no pairs of columns (gate and up, a
+# head's RoPE pairs).
+SKINNY_FORMS = {"m1n1": (1, 1, 8), "m1n2": (1, 2, 8), "m2n1": (2, 1, 8), "m2n2": (2, 2, 8), "m2n4": (2, 4, 4),
+                "m4n2": (4, 2, 8), "m4n4": (4, 4, 4), "m4n8": (4, 8, 4), "m8n4": (8, 4, 4), "m8n8": (8, 8, 4)}
+SKINNY_PAIR_MODES = ("silu_mul", "qkv_rope", "qkv_rope_paged")
+SKINNY_MODES = ("store", "add", "store_keys") + SKINNY_PAIR_MODES
+SKINNY_BUFFERS = ("a", "b0", "b1", "b2", "c0", "c1", "c2", "r0", "position", "slot", "rope", "keys")
+_SKINNY = re.compile(r"^fk_skinny_(\w+)_(m\dn\d)$")
+
+
+def skinny_entry(entry: str) -> tuple[str, tuple]:
+    """(mode, (row blocks, column blocks, wavefronts)) of a fk_skinny entry."""
+    m = _SKINNY.match(entry)
+    return m.group(1), SKINNY_FORMS[m.group(2)]
+
+
 # Keys a block of the prefill attention stages (fk_attend.h): ring lengths are
 # multiples of it.
 ATTEND_KEYS = 64
@@ -345,6 +372,9 @@ ABIS: dict[str, KernelAbi] = {
     "fk_gemm_f16_qkv_rope_paged": KernelAbi("fk_gemm_f16_qkv_rope_paged", ("a", "b0", "b1", "b2", "c0", "c1", "c2",
                                                                            "r0", "position", "table", "rope"),
                                             GemmQkvPagedParams, 256),
+    **{f"fk_skinny_{mode}_{form}": KernelAbi(f"fk_skinny_{mode}_{form}", SKINNY_BUFFERS, SkinnyParams, 64 * w)
+       for form, (_, nb, w) in SKINNY_FORMS.items() for mode in SKINNY_MODES
+       if nb > 1 or mode not in SKINNY_PAIR_MODES},
     "fk_prefill_gather": KernelAbi("fk_prefill_gather", ("table", "tokens", "x"), PrefillGatherParams, 256),
     "fk_prefill_norm_pack": KernelAbi("fk_prefill_norm_pack", ("x", "gamma", "y"), PrefillNormParams, 256),
     **{f"fk_prefill_norm_pack_w{w}": KernelAbi(f"fk_prefill_norm_pack_w{w}", ("x", "gamma", "y"), PrefillNormParams,
@@ -750,6 +780,13 @@ def launch_reads(entry: str, params: dict) -> set[str]:
         if entry == "fk_gemm_f16_store_keys":
             need.add("keys")
         return need
+    if entry.startswith("fk_skinny_"):
+        mode, _ = skinny_entry(entry)
+        n = params.get("n_anchors", 1)
+        need = {"a"} | {f"b{j}" for j in range(n)} | {f"c{j}" for j in range(n)}
+        if mode in ("qkv_rope", "qkv_rope_paged"):
+            need |= {"position", "slot", "rope"}
+        return need | {"add": {"r0"}, "store_keys": {"keys"}}.get(mode, set())
     if entry == "fk_rmsnorm_f32" or entry.startswith("fk_prefill_norm_pack"):
         return set(abi.buffers) - ({"gamma"} if not params.get("has_gamma") else set())
     if entry.startswith(("fk_prefill_attend_g", "fk_prefill_attend_f16_g")):

@@ -41,13 +41,14 @@ the sequence rows of a step).
 from __future__ import annotations
 
 from collections import defaultdict
+from dataclasses import dataclass
 from typing import Optional
 
 import numpy as np
 
-from .kernels import ATTEND_KEYS, NORM_PACK_HELD
+from .kernels import ATTEND_KEYS, NORM_PACK_HELD, SKINNY_FORMS, SKINNY_PAIR_MODES
 from .layout import SLAB, pack, pair
-from .lower import ACT, Launch, Lowered, LoweringError, rope_table
+from .lower import ACT, BufferSpec, Launch, Lowered, LoweringError, rope_table
 from .program.check import CheckedProgram
 from .program.graph import (
     CACHE_BF16, F16, F32, GELU_TANH, SILU, U32, Add, ArgMax, Attend, Gather, GeluMul, Input, KvStore, Linear, Paged, Ring,
@@ -61,8 +62,19 @@ QBLOCK = 32                        # rows an attention threadgroup takes
 HEAD_DIM = 64                      # the attention kernel's head dimension
 
 
+@dataclass(frozen=True)
+class LiveRows:
+    """The rows of a step whose outputs are read, in chunks of 16: chunk c is
+    rows first + i apart (i = 0 .. 15), first = (c div run_chunks) run +
+    (c mod run_chunks) 16 apart.  The rest only fill the step's tiles out."""
+    chunks: int
+    run_chunks: int
+    run: int
+    apart: int = 1
+
+
 def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Optional[int] = None,
-                  scratch_slot: bool = False) -> Lowered:
+                  scratch_slot: bool = False, live: Optional[LiveRows] = None) -> Lowered:
     """The launches of every step of the plan for a step of `rows` rows (a
     multiple of 256: the sequences' rows one after another, each sequence's
     run a multiple of 32 rows; `run_rows` rows each where the plan stages
@@ -70,7 +82,8 @@ def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Opti
     holds one slot more (and each paged pool one block more) past the
     program's: rows that only fill a step out to its tiles store there, so
     that a step's real rows may be any number (``PrefillSession``,
-    ``DecodeRows``)."""
+    ``DecodeRows``).  `live`: which rows those are (default: every row);
+    where few enough, the GEMMs make them alone."""
     if rows <= 0 or rows % SLAB:
         raise LoweringError(f"a step of {rows} rows; the prefill kernels take multiples of {SLAB}")
     run_rows = rows if run_rows is None else run_rows
@@ -80,7 +93,72 @@ def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Opti
     _Prefill(out, run_rows, scratch_slot).run()
     _fuse_qkv_rope(out)
     _fuse_argmax(out)
+    _skinny_gemms(out, live or LiveRows(rows // 16, rows // 16, rows))
     return out
+
+
+def skinny_form(chunks: int, m: int, n: int, k: int, pairs: bool) -> Optional[str]:
+    """The form of fk_skinny that a GEMM of `chunks` live chunks of 16 rows
+    (of a step of m) by n weight rows of k columns takes, or None where the
+    256 × 256 tiles of fk_gemm are faster (MI355X, 256 CUs; µs, f16):
+
+    - A launch of 256 × 256 tiles costs its rounds of 256 tiles, whatever
+      its rows: 46 a round at k 2048, 151 at 8192.  A round of skinny's
+      largest tiles (128 × 128, k split in 4) costs about half of that (25
+      and 66), so skinny takes over at half as many rounds more: at n 2048,
+      1408 rows take 25 against 46 (k 2048) and 66 against 152 (k 8192); at
+      n 16384, 208 rows 28 against 44, but 352 rows (two rounds) 49 against
+      47 and 704 (three) 74 against 51.
+    - Of its forms, the largest tile of which there are 140 or more (half
+      the chip busy): a larger one reads its operands fewer times, a smaller
+      one fills more CUs.  At k 8192 and n 2048: 16 rows 12.2 (m1n1), 112
+      rows 18.3 (m2n2; m4n2's 128 tiles 25.6), 208 rows 22.9 (m4n2), 352
+      rows 32 (m4n4), 704 rows 44 (m8n4; m8n8's 96 tiles 61).
+    - A k shorter than 1024 leaves a wavefront under four steps to
+      overlap."""
+    if k < 1024 or m * k * 2 >= 0xfffffff0:
+        return None
+    tiles = (m // SLAB) * (n // SLAB)
+    largest = -(-chunks // 8) * (n // 128)
+    if 2 * -(-largest // 256) > 3 * -(-tiles // 256):
+        return None
+    best = None
+    for form, (mb, nb, _) in SKINNY_FORMS.items():
+        if mb >= 2 * chunks or (pairs and nb == 1):
+            continue
+        if best is None or -(-chunks // mb) * (n // (16 * nb)) >= 140:
+            best = form
+    return best
+
+
+def _skinny_gemms(out: Lowered, live: LiveRows) -> None:
+    """Each GEMM of too few live rows for fk_gemm's tiles, as the form of
+    fk_skinny that ``skinny_form`` picks: the same epilogue on the live rows
+    alone."""
+    for i, gm in enumerate(out.launches):
+        if not gm.entry.startswith("fk_gemm_f16_"):
+            continue
+        p = gm.params
+        mode = gm.entry[len("fk_gemm_f16_"):]
+        n = 2 * p["ldc"][0] if mode == "silu_mul" else p["first_col"][p["n_anchors"]]
+        form = skinny_form(live.chunks, p["m"], n, p["k"], mode in SKINNY_PAIR_MODES)
+        if form is None:
+            continue
+        mb, nb, waves = SKINNY_FORMS[form]
+        bind = dict(gm.bind)
+        if "table" in bind:
+            bind["slot"] = bind.pop("table")
+        if mode == "store_keys":
+            # a key a tile's columns
+            parts = n // (16 * nb)
+            out.buffers[bind["keys"]] = BufferSpec(bind["keys"], "u64", p["m"] * parts)
+            for am in out.launches:
+                if am.entry == "fk_prefill_argmax_keys" and am.bind["keys"] == bind["keys"]:
+                    am.params["parts"] = parts
+        groups = -(-(n // (16 * nb)) // 8) * 8 * -(-live.chunks // mb)
+        out.launches[i] = Launch(gm.step, f"fk_skinny_{mode}_{form}", groups, 64 * waves, bind,
+                                 dict(p, live=live.chunks, run_chunks=live.run_chunks, run=live.run,
+                                      apart=live.apart))
 
 
 def _fuse_argmax(out: Lowered) -> None:
@@ -635,7 +713,7 @@ class _RowsSession:
     layout and rounding), with that slot after them."""
 
     def _setup(self, device, kernels, dims, program, sequence_rows: int, rows: int, run_rows: int,
-               positions, slots, real, scratch: bool, paging=None, tables=None) -> None:
+               positions, slots, real, scratch: bool, live: LiveRows, paging=None, tables=None) -> None:
         from .engine import Engine
         from .program.check import check_program
         from .program.plan import PlanOptions, plan
@@ -644,7 +722,7 @@ class _RowsSession:
         self.program = program
         self.checked = check_program(self.program)
         self.plan = plan(PlanOptions(sequence_rows=sequence_rows), self.checked)
-        self.lowered = lower_prefill(self.checked, self.plan, rows, run_rows=run_rows, scratch_slot=scratch)
+        self.lowered = lower_prefill(self.checked, self.plan, rows, run_rows=run_rows, scratch_slot=scratch, live=live)
         self.engine = Engine(device, kernels, self.lowered)
         self.rows, self.run_rows = rows, run_rows
         self.real = np.asarray(real, np.int64)
@@ -765,8 +843,9 @@ class PrefillSession(_RowsSession):
         # makes the plan stage the KV stores.
         program = decoder_step(dims, "prefill", embed, layers, position_bound=position_bound or seq_rows,
                                rope_rotated=rope_rotated, paging=paging)
-        self._setup(device, kernels, dims, program, seq_rows, rows, run, positions, slots, real, pad, paging,
-                    rows_tables)
+        chunks = -(-seq_rows // 16)
+        self._setup(device, kernels, dims, program, seq_rows, rows, run, positions, slots, real, pad,
+                    LiveRows(seqs * chunks, chunks, run), paging, rows_tables)
         if paging is not None:
             self.tables = tables
 
@@ -786,7 +865,9 @@ class DecodeRows(_RowsSession):
         self.embed = embed
         rows, pos, sl, real = decode_placement(positions, slots, dims.slots)
         program = decoder_step(dims, "decode", embed, layers, position_bound=dims.context)
-        self._setup(device, kernels, dims, program, 1, rows, QBLOCK, pos, sl, real, True)
+        chunks = -(-len(real) // 16)
+        self._setup(device, kernels, dims, program, 1, rows, QBLOCK, pos, sl, real, True,
+                    LiveRows(chunks, chunks, rows, QBLOCK))
 
 
 def decode_placement(positions, slots, n_slots: int) -> tuple:

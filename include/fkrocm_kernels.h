@@ -338,6 +338,20 @@ typedef struct fk_gemm_qkv_paged_params {
   fk_paging pg;
 } fk_gemm_qkv_paged_params;
 
+/* fk_skinny_*: the GEMM of a step of few rows (fk_skinny.h), the epilogues of
+ * fk_gemm_f16_*.  Its rows go by chunks of 16: chunk c holds rows first +
+ * i apart, i = 0 .. 15, first = (c / run_chunks) run + (c mod run_chunks) 16
+ * apart; rows past g.m are neither read nor stored. */
+typedef struct fk_skinny_params {
+  fk_gemm_params g;
+  uint32_t live;       /* chunks of rows the launch makes */
+  uint32_t run_chunks; /* chunks of a run that are live */
+  uint32_t run;        /* rows from run to run */
+  uint32_t apart;      /* rows from row to row of a chunk */
+  fk_gemm_rope_params r; /* the QKV epilogue's; paged: `length`, `slots`, `staged` unused */
+  fk_paging pg;          /* paged */
+} fk_skinny_params;
+
 typedef struct fk_prefill_gather_params {
   uint32_t rows;
   uint32_t width;      /* a multiple of 4 */

@@ -1,0 +1,96 @@
+"""Which GEMMs of a step go to the kernel of few rows (fk_skinny.h), on the
+CPU: every launch that does passes the engine's and the launch table's
+checks, reaches every live row once, and no other shape is moved."""
+
+import dataclasses
+
+import numpy as np
+import pytest
+
+from furykernel_amd import kernels as K, runtime
+from furykernel_amd.engine import check_launch, params_struct
+from furykernel_amd.prefill import (QBLOCK, LiveRows, decode_placement, lower_prefill, prefill_placement, skinny_form)
+from furykernel_amd.program.check import check_program
+from furykernel_amd.program.decoder import ONE_B, SMALL_PREFILL, decoder_step
+from furykernel_amd.program.plan import PlanOptions, plan
+
+
+def lowered(dims, seqs, seq_rows, decode=False, bound=None, **kw):
+    """(the lowering, the step's real rows, its rows) as the sessions make it."""
+    dims = dataclasses.replace(dims, slots=max(seqs, 1))
+    if decode:
+        rows, _, _, real = decode_placement([0] * seqs, range(seqs), dims.slots)
+        run, chunks, at = QBLOCK, -(-seqs // 16), 1
+        live = LiveRows(chunks, chunks, rows, QBLOCK)
+    else:
+        rows, run, _, _, real = prefill_placement(seqs, seq_rows, dims.slots)
+        chunks, at = -(-seq_rows // 16), seq_rows
+        live = LiveRows(seqs * chunks, chunks, run)
+    c = check_program(decoder_step(dims, layers=1, position_bound=bound or (dims.context if decode else seq_rows), **kw))
+    return lower_prefill(c, plan(PlanOptions(sequence_rows=at), c), rows, run, True, live), real, rows
+
+
+CASES = {"1 x 100": (1, 100), "3 x 9": (3, 9), "2 x 700": (2, 700), "1 x 256": (1, 256), "4 x 1500": (4, 1500)}
+
+
+@pytest.mark.parametrize("case", [*CASES, "staged", "paged", "batch 1", "batch 8", "batch 41"])
+def test_every_launch_passes_the_checks_and_makes_the_live_rows(case):
+    if case.startswith("batch"):
+        low, real, rows = lowered(ONE_B, int(case[6:]), 1, decode=True)
+    elif case == "staged":
+        low, real, rows = lowered(ONE_B, 2, 64, bound=4096)
+    elif case == "paged":
+        low, real, rows = lowered(ONE_B, 2, 64, paging=(64, 128))
+    else:
+        low, real, rows = lowered(ONE_B, *CASES[case])
+    at, addr = 1 << 40, {}
+    for name, spec in low.buffers.items():
+        addr[name] = at
+        at += (spec.nbytes + 4095) // 4096 * 4096
+    skinny = 0
+    for L in low.launches:
+        check_launch(L, low.buffers)
+        spans = [(0, 0) if L.bind.get(b) is None else (addr[L.bind[b]], low.buffers[L.bind[b]].nbytes)
+                 for b in K.ABIS[L.entry].buffers]
+        runtime.launch_check(L.entry, L.groups, L.threads, L.lds_bytes, spans, params_struct(L))
+        if L.entry.startswith("fk_skinny_"):
+            skinny += 1
+            p = L.params
+            c = np.arange(p["live"])
+            first = (c // p["run_chunks"]) * p["run"] + (c % p["run_chunks"]) * 16 * p["apart"]
+            made = (first[:, None] + np.arange(16) * p["apart"]).reshape(-1)
+            made = made[made < rows]
+            assert np.unique(made).size == made.size and np.isin(real, made).all()
+            # a grid that misses a tile, a buffer short of its last byte
+            with pytest.raises(runtime.FkError):
+                runtime.launch_check(L.entry, L.groups - 8, L.threads, L.lds_bytes, spans, params_struct(L))
+            for b in ("a", "b0", "c0", "r0", "keys", "position", "rope", "c2"):
+                i = K.ABIS[L.entry].buffers.index(b)
+                if b in K.launch_reads(L.entry, p):
+                    short = list(spans)
+                    short[i] = (short[i][0], short[i][1] - 1)
+                    with pytest.raises(runtime.FkError):
+                        runtime.launch_check(L.entry, L.groups, L.threads, L.lds_bytes, short, params_struct(L))
+    assert skinny == {"4 x 1500": 0, "2 x 700": 2, "1 x 256": 4}.get(case, 5)
+
+
+def test_the_keys_of_the_head_follow_its_tile():
+    low, _, rows = lowered(ONE_B, 1, 100)
+    head, token = low.launches[-2:]
+    mode, (_, nb, _) = K.skinny_entry(head.entry)
+    assert mode == "store_keys" and token.entry == "fk_prefill_argmax_keys"
+    assert token.params["parts"] == 32000 // (16 * nb)
+    assert low.buffers[head.bind["keys"]].count == rows * token.params["parts"]
+
+
+def test_forms_by_size():
+    # the largest tile that fills half the chip; none where fk_gemm's rounds are as few
+    assert [skinny_form(c, 256, 2048, 8192, False) for c in (1, 3, 4, 7, 13, 16)] == \
+        ["m1n1", "m2n1", "m2n1", "m2n2", "m4n2", "m4n2"]
+    assert skinny_form(88, 1536, 2048, 8192, False) == "m8n8"
+    assert skinny_form(1, 256, 3072, 2048, True) == "m1n2"      # pairs of columns
+    assert skinny_form(22, 512, 16384, 2048, True) is None
+    assert skinny_form(512, 8192, 2048, 8192, False) is None
+    assert skinny_form(1, 256, 2048, 960, False) is None        # a short k
+    assert all(L.entry.startswith("fk_skinny") is False
+               for L in lowered(SMALL_PREFILL, 2, 100)[0].launches)
