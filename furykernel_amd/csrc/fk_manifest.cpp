@@ -334,6 +334,19 @@ std::vector<Entry> build() {
           p, sizeof(S));
     }
   {
+    using S = fk_rows_attend_params;
+    const std::vector<fk_abi_param> p = {FK_P(S, rows, "u32"),   FK_P(S, apart, "u32"),  FK_P(S, heads, "u32"),
+                                         FK_P(S, kv_heads, "u32"), FK_P(S, length, "u32"), FK_P(S, slots, "u32"),
+                                         FK_P(S, window, "u32"), FK_P(S, parts, "u32"),  FK_P(S, scale, "f32")};
+    for (const char *t : {"f16", "bf16"})
+      add(std::string("fk_rows_attend_") + t, 256,
+          {buf("qr", "read", "f16"), buf("kc", "read", t), buf("vc", "read", t), buf("position", "read", "u32"),
+           buf("slot", "read", "u32"), buf("out", "write", "f16"), buf("partials", "write", "f32")},
+          p, sizeof(S));
+    add("fk_rows_combine", 0, {buf("partials", "read", "f32"), buf("position", "read", "u32"), buf("out", "write", "f16")},
+        p, sizeof(S));
+  }
+  {
     using S = fk_prefill_gather_params;
     add("fk_prefill_gather", 256, {buf("table", "read", "f16"), buf("tokens", "read", "u32"), buf("x", "write", "f32")},
         {FK_P(S, rows, "u32"), FK_P(S, width, "u32"), FK_P(S, table_rows, "u32"), FK_P(S, table_f16, "u32"),
@@ -821,6 +834,27 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
       for (Need &n : need)
         if (std::strcmp(n.name, "c1") == 0 || std::strcmp(n.name, "c2") == 0) n.bytes = pool;
     }
+  } else if (std::strncmp(entry, "fk_rows_attend", 14) == 0 || std::strcmp(entry, "fk_rows_combine") == 0) {
+    fk_rows_attend_params p;
+    std::memcpy(&p, params, sizeof p);
+    const bool combine = entry[8] == 'c';
+    const uint32_t g = p.kv_heads && p.heads % p.kv_heads == 0 ? p.heads / p.kv_heads : 0;
+    // a tile is 256 keys; past a ring's last one a part would have none
+    if (p.rows == 0 || p.apart == 0 || g == 0 || g > 16 || p.length == 0 || p.slots == 0 || p.parts == 0 ||
+        p.parts > (p.length + 255) / 256 || (uint64_t)p.length * 128 >= 0xffffffffu ||
+        (uint64_t)groups != (uint64_t)p.rows * p.kv_heads * (combine ? 1 : p.parts) || (combine && threads != 64 * g))
+      return bad(err, cap, FK_ERR_ARG, "%s: %u rows, %u heads over %u, %u parts of a ring of %u in %u x %u threads",
+                 entry, p.rows, p.heads, p.kv_heads, p.parts, p.length, groups, threads);
+    const uint64_t last = (uint64_t)(p.rows - 1) * p.apart, wide = (uint64_t)p.heads * 64 * 2;
+    const uint64_t cache = (uint64_t)p.slots * p.kv_heads * p.length * 128;
+    need = {{"position", (last + 1) * 4}, {"out", (last / 256 + 1) * 256 * wide}};
+    if (!combine) {
+      need.push_back({"qr", (last + 1) * wide});
+      need.push_back({"kc", cache});
+      need.push_back({"vc", cache});
+      need.push_back({"slot", (last + 1) * 4});
+    }
+    if (combine || p.parts > 1) need.push_back({"partials", (uint64_t)p.rows * p.heads * p.parts * 66 * 4});
   } else if (std::strncmp(entry, "fk_skinny_", 10) == 0) {
     fk_skinny_params p;
     std::memcpy(&p, params, sizeof p);

@@ -7,4 +7,5 @@
 #include "fk_step.h"
 #include "fk_gemm.h"
 #include "fk_prefill.h"
+#include "fk_rows_attend.h"
 #include "fk_skinny.h"

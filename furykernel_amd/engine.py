@@ -56,6 +56,7 @@ _STRUCTS = {
     **{f"{form}{g}": K.PrefillAttendPagedParams for form in ("fk_prefill_attend_paged_g", "fk_prefill_attend_paged_f16_g")
        for g in (1, 2, 4)},
     **{e: K.SkinnyParams for e in K.ABIS if e.startswith("fk_skinny_")},
+    **{e: K.RowsAttendParams for e in ("fk_rows_attend_f16", "fk_rows_attend_bf16", "fk_rows_combine")},
     "fk_prefill_gather": K.PrefillGatherParams,
     "fk_prefill_norm_pack": K.PrefillNormParams,
     **{f"fk_prefill_norm_pack_w{w}": K.PrefillNormParams for w in K.NORM_PACK_HELD},

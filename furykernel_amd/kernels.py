@@ -114,6 +114,13 @@ class SkinnyParams(ctypes.Structure):
         [("block_size", ctypes.c_uint32), ("table_len", ctypes.c_uint32), ("blocks", ctypes.c_uint32)]
 
 
+class RowsAttendParams(ctypes.Structure):
+    """fk_rows_attend_params: the attention of rows each a sequence's one."""
+    _fields_ = [("rows", ctypes.c_uint32), ("apart", ctypes.c_uint32), ("heads", ctypes.c_uint32),
+                ("kv_heads", ctypes.c_uint32), ("length", ctypes.c_uint32), ("slots", ctypes.c_uint32),
+                ("window", ctypes.c_uint32), ("parts", ctypes.c_uint32), ("scale", ctypes.c_float)]
+
+
 class PrefillGatherParams(ctypes.Structure):
     _fields_ = [("rows", ctypes.c_uint32), ("width", ctypes.c_uint32), ("table_rows", ctypes.c_uint32),
                 ("table_f16", ctypes.c_uint32), ("factor", ctypes.c_float)]
@@ -349,6 +356,10 @@ def skinny_entry(entry: str) -> tuple[str, tuple]:
     return m.group(1), SKINNY_FORMS[m.group(2)]
 
 
+# Keys a threadgroup of the attention of a batch of rows takes at a time
+# (fk_rows_attend.h).
+ROWS_TILE = 256
+
 # Keys a block of the prefill attention stages (fk_attend.h): ring lengths are
 # multiples of it.
 ATTEND_KEYS = 64
@@ -375,6 +386,9 @@ ABIS: dict[str, KernelAbi] = {
     **{f"fk_skinny_{mode}_{form}": KernelAbi(f"fk_skinny_{mode}_{form}", SKINNY_BUFFERS, SkinnyParams, 64 * w)
        for form, (_, nb, w) in SKINNY_FORMS.items() for mode in SKINNY_MODES
        if nb > 1 or mode not in SKINNY_PAIR_MODES},
+    **{e: KernelAbi(e, ("qr", "kc", "vc", "position", "slot", "out", "partials"), RowsAttendParams, 256)
+       for e in ("fk_rows_attend_f16", "fk_rows_attend_bf16")},
+    "fk_rows_combine": KernelAbi("fk_rows_combine", ("partials", "position", "out"), RowsAttendParams),
     "fk_prefill_gather": KernelAbi("fk_prefill_gather", ("table", "tokens", "x"), PrefillGatherParams, 256),
     "fk_prefill_norm_pack": KernelAbi("fk_prefill_norm_pack", ("x", "gamma", "y"), PrefillNormParams, 256),
     **{f"fk_prefill_norm_pack_w{w}": KernelAbi(f"fk_prefill_norm_pack_w{w}", ("x", "gamma", "y"), PrefillNormParams,
@@ -780,6 +794,8 @@ def launch_reads(entry: str, params: dict) -> set[str]:
         if entry == "fk_gemm_f16_store_keys":
             need.add("keys")
         return need
+    if entry.startswith("fk_rows_attend"):
+        return set(abi.buffers) - (set() if params.get("parts", 1) > 1 else {"partials"})
     if entry.startswith("fk_skinny_"):
         mode, _ = skinny_entry(entry)
         n = params.get("n_anchors", 1)

@@ -46,7 +46,7 @@ from typing import Optional
 
 import numpy as np
 
-from .kernels import ATTEND_KEYS, NORM_PACK_HELD, SKINNY_FORMS, SKINNY_PAIR_MODES
+from .kernels import ATTEND_KEYS, NORM_PACK_HELD, ROWS_TILE, SKINNY_FORMS, SKINNY_PAIR_MODES
 from .layout import SLAB, pack, pair
 from .lower import ACT, BufferSpec, Launch, Lowered, LoweringError, rope_table
 from .program.check import CheckedProgram
@@ -71,6 +71,7 @@ class LiveRows:
     run_chunks: int
     run: int
     apart: int = 1
+    count: Optional[int] = None  # the rows themselves, where the last chunk is not whole
 
 
 def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Optional[int] = None,
@@ -93,8 +94,53 @@ def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Opti
     _Prefill(out, run_rows, scratch_slot).run()
     _fuse_qkv_rope(out)
     _fuse_argmax(out)
-    _skinny_gemms(out, live or LiveRows(rows // 16, rows // 16, rows))
+    live = live or LiveRows(rows // 16, rows // 16, rows)
+    _skinny_gemms(out, live)
+    _row_attention(out, live)
     return out
+
+
+def attend_parts(pairs: int, length: int) -> int:
+    """The threadgroups that share a (row, kv head)'s keys (fk_rows_attend.h)
+    among `pairs` of them over rings of `length`: enough for 1024 in all
+    (4 a CU, so that rows of different lengths even out), at least 4 (a long
+    row among many short ones would end the launch alone), and no more than
+    the ring's tiles.  Measured with their combine, 8 kv heads, µs in 1, 4
+    and 16 parts: 8 rows of up to 4095 positions 26.6, 14.2, 12.9; 64 such
+    rows 41.2, 38.9, 41.5; 41 rows of up to 700 10.3, 11.0, 11.8."""
+    parts = 4
+    while parts * pairs < 1024:
+        parts *= 2
+    return min(parts, -(-length // ROWS_TILE))
+
+
+def _row_attention(out: Lowered, live: LiveRows) -> None:
+    """The attention of a step whose query blocks hold one live row each (a
+    decode step's rows), its keys split over the chip: ``fk_rows_attend_*``
+    on those rows alone, and ``fk_rows_combine`` where a row's keys may take
+    more than one part.  Rings without staged rows."""
+    if live.apart != QBLOCK or live.count is None:
+        return
+    launches = []
+    for at in out.launches:
+        p = at.params
+        if not at.entry.startswith(("fk_prefill_attend_g", "fk_prefill_attend_f16_g")) or p["staged"]:
+            launches.append(at)
+            continue
+        pairs = live.count * p["kv_heads"]
+        parts = attend_parts(pairs, p["length"])
+        params = {f: p[f] for f in ("heads", "kv_heads", "length", "slots", "window", "scale")}
+        params.update(rows=live.count, apart=QBLOCK, parts=parts)
+        bind = {b: at.bind[b] for b in ("qr", "kc", "vc", "position", "slot", "out")}
+        bind["partials"] = None
+        if parts > 1:
+            bind["partials"] = out.buffer("attend:partials", "f32", live.count * p["heads"] * parts * (HEAD_DIM + 2))
+        launches.append(Launch(at.step, f"fk_rows_attend_{'bf16' if p['cache_bf16'] else 'f16'}", pairs * parts, 256,
+                               bind, params))
+        if parts > 1:
+            launches.append(Launch(at.step, "fk_rows_combine", pairs, 64 * (p["heads"] // p["kv_heads"]),
+                                   {b: bind[b] for b in ("partials", "position", "out")}, dict(params)))
+    out.launches[:] = launches
 
 
 def skinny_form(chunks: int, m: int, n: int, k: int, pairs: bool) -> Optional[str]:
@@ -867,7 +913,7 @@ class DecodeRows(_RowsSession):
         program = decoder_step(dims, "decode", embed, layers, position_bound=dims.context)
         chunks = -(-len(real) // 16)
         self._setup(device, kernels, dims, program, 1, rows, QBLOCK, pos, sl, real, True,
-                    LiveRows(chunks, chunks, rows, QBLOCK))
+                    LiveRows(chunks, chunks, rows, QBLOCK, len(real)))
 
 
 def decode_placement(positions, slots, n_slots: int) -> tuple:

@@ -401,6 +401,22 @@ typedef struct fk_prefill_attend_params {
                        staged runs read their own rows from ks and vs */
 } fk_prefill_attend_params;
 
+/* fk_rows_attend_{f16,bf16}, fk_rows_combine: the attention of `rows` rows,
+ * `apart` rows of the step from one to the next, each a sequence's one, over
+ * rings; the keys of a row go to `parts` threadgroups a kv head in tiles of
+ * 256, and partials hold [rows][kv_heads][parts][heads / kv_heads][66] f32. */
+typedef struct fk_rows_attend_params {
+  uint32_t rows;
+  uint32_t apart;
+  uint32_t heads;
+  uint32_t kv_heads; /* heads / kv_heads at most 16 */
+  uint32_t length;   /* ring length; positions are below it */
+  uint32_t slots;
+  uint32_t window;   /* 0: none; else a row sees positions > position - window */
+  uint32_t parts;
+  float scale;
+} fk_rows_attend_params;
+
 /* fk_prefill_attend_paged_g*: the attention over paged pools; `a.slots`,
  * `a.staged` and `a.run_rows` unused, `a.length` the positions a table covers
  * (table_len block_size). */

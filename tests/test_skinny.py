@@ -21,7 +21,7 @@ def lowered(dims, seqs, seq_rows, decode=False, bound=None, **kw):
     if decode:
         rows, _, _, real = decode_placement([0] * seqs, range(seqs), dims.slots)
         run, chunks, at = QBLOCK, -(-seqs // 16), 1
-        live = LiveRows(chunks, chunks, rows, QBLOCK)
+        live = LiveRows(chunks, chunks, rows, QBLOCK, seqs)
     else:
         rows, run, _, _, real = prefill_placement(seqs, seq_rows, dims.slots)
         chunks, at = -(-seq_rows // 16), seq_rows
@@ -81,6 +81,21 @@ def test_the_keys_of_the_head_follow_its_tile():
     assert mode == "store_keys" and token.entry == "fk_prefill_argmax_keys"
     assert token.params["parts"] == 32000 // (16 * nb)
     assert low.buffers[head.bind["keys"]].count == rows * token.params["parts"]
+
+
+@pytest.mark.parametrize("rows,context,parts", [(8, 4096, 16), (41, 4096, 4), (64, 4096, 4), (3, 256, 1), (1, 512, 2)])
+def test_a_batchs_attention_splits_its_keys(rows, context, parts):
+    low, _, _ = lowered(dataclasses.replace(ONE_B, context=context), rows, 1, decode=True)
+    entries = [L.entry for L in low.launches]
+    at = low.launches[entries.index("fk_rows_attend_f16")]
+    assert (at.groups, at.params["rows"], at.params["parts"]) == (rows * 8 * parts, rows, parts)
+    assert ("fk_rows_combine" in entries) == (parts > 1)
+    assert not any(e.startswith("fk_prefill_attend") for e in entries)
+
+
+def test_a_prefills_attention_stays():
+    low, _, _ = lowered(ONE_B, 3, 9)
+    assert [L.entry for L in low.launches].count("fk_prefill_attend_f16_g4") == 1
 
 
 def test_forms_by_size():
