@@ -29,12 +29,12 @@
 // matrix operations), which is why tiles grow with the rows.  Measured on
 // MI355X, f16, µs (fk_gemm's tiles in brackets):
 //
-//   live rows            16          64         112         208         704
-//   QKV  3072 x 2048    6.6 [47]    8.2 [47]  10.2 [47]   11.8 [47]   24.5 [47]
-//   O    2048 x 2048    5.2 [46]    6.2 [46]   7.4 [46]    9.0 [46]   16.7 [46]
-//   gate/up 2 x 8192   13.9 [45]   17.7 [45]  21.5 [44]   28.4 [44]    -  [51]
-//   down 2048 x 8192   12.2 [151]  15.4 [151] 18.3 [151]  22.9 [151]  43.8 [152]
-//   head 32000 x 2048  25.9 [58]   29.1 [56]  36.6 [55]     -  [55]
+//   live rows            16          64         112         208         704        1408
+//   QKV  3072 x 2048    7.1 [49]    8.7 [49]  10.9 [49]   12.9 [49]   26.0 [51]   42.7 [57]
+//   O    2048 x 2048    5.4 [50]    6.4 [50]   7.4 [50]    9.1 [50]   18.2 [55]   26.4 [55]
+//   gate/up 2 x 8192   13.6 [45]   17.9 [45]  20.8 [44]   28.0 [44]    -  [51]     -  [98]
+//   down 2048 x 8192   12.5 [160] 15.6 [160]  18.2 [161]  23.3 [161]  45.9 [160]  65.2 [160]
+//   head 32000 x 2048  26.7 [62]   31.0 [56]  38.5 [57]     -  [57]    -  [125]    -  [200]
 //
 // The forms (MB, NB, W, D) and where each is taken: prefill.py's skinny_form.
 //
@@ -148,6 +148,29 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
   const uint32_t fu = wave * D * CH * FK_WAVE + (lane % 16) * 4 + ((lane / 16) ^ fk::tile_swizzle(lane % 16));
   FK_LDS char *const ring = (FK_LDS char *)lds + wave * (D * CH * 1024);
 
+  // The epilogue's units: a row of blocks has NU, a round of MR rows of blocks
+  // UNITS, of which this wavefront takes wave, wave + W, ...: IT a round.
+  constexpr int UNITS = MR * NU, IT = (UNITS + W - 1) / W, ROUNDS = MB / MR;
+  auto unit_row = [&](int round, int it, uint32_t l) -> uint32_t {  // past the rows for a unit past the last
+    const uint32_t u = wave + it * W;
+    return u < (uint32_t)UNITS ? row_of(round * MR + u / NU, l % 16) : 0xffffffffu;
+  };
+  // What the units' rows are stored by is loaded here, and what they are
+  // combined with after the loop, all at once: loaded at its unit's turn,
+  // each would cost the unit a round trip (O of 1408 rows, 16 units a
+  // wavefront: 41 µs a launch in the step, now 26).
+  uint32_t upos[QKV ? ROUNDS : 1][QKV ? IT : 1], uslot[QKV ? ROUNDS : 1][QKV ? IT : 1];
+  if constexpr (QKV) {
+#pragma unroll
+    for (int round = 0; round < ROUNDS; round++)
+#pragma unroll
+      for (int it = 0; it < IT; it++) {
+        const uint32_t row = min(unit_row(round, it, lane), p.g.m - 1);
+        upos[round][it] = position[row];
+        uslot[round][it] = MODE == FK_GEMM_QKV_ROPE && !p.r.staged && anchor != 0 ? slot[row] : 0u;
+      }
+  }
+
   fk_float4v acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; i++)
@@ -184,6 +207,10 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
     _Pragma("unroll") for (int i_ = 0; i_ < MB; i_++)                                                           \
     _Pragma("unroll") for (int j_ = 0; j_ < NB; j_++)                                                           \
       acc[i_][j_] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb[j_].h, fa[i_].h, acc[i_][j_], 0, 0, 0);           \
+    if constexpr (MB * NB >= 64) { /* the accumulators stay in AGPRs from step to step */                       \
+      _Pragma("unroll") for (int i_ = 0; i_ < MB; i_++)                                                         \
+      _Pragma("unroll") for (int j_ = 0; j_ < NB; j_++) asm volatile("" : "+a"(acc[i_][j_]));                   \
+    }                                                                                                           \
   } while (0)
   auto loop = [&](auto streamed) {
     constexpr int HINT = decltype(streamed)::value ? 2 : 0;  // non-temporal
@@ -202,75 +229,105 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
   // (the down projection of 16 rows 12.2 µs against 13.0, gate and up 13.9
   // against 15.7); read by more, they are kept (the down projection of 112
   // rows, four tiles: 18.3 against 19.5).
-  if (tiles_m <= 2) loop(fk_bool_tag<true>{});
+  if constexpr (MB * NB >= 64) loop(fk_bool_tag<false>{});
+  else if (tiles_m <= 2) loop(fk_bool_tag<true>{});
   else loop(fk_bool_tag<false>{});
 #undef FK_SKINNY_LOAD
 #undef FK_SKINNY_STEP
 #undef FK_SKINNY_VMCNT
+  // (The lane index is taken anew through an asm statement, so that nothing of
+  // the epilogue is computed before the loop and held in registers across it.)
+  uint32_t lane_e;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(lane_e) : "v"(lane));
+  const uint32_t nq = 4 * (lane_e / 16);
+  // A unit's first column among its anchor's (QKV: in its head, d).
+  auto unit_col = [&](uint32_t un) -> uint32_t {
+    if constexpr (MODE == FK_GEMM_SILU_MUL) return n0 + 16 * un + nq;
+    else if constexpr (QKV) return (NB == 2 ? n0 % 64 : un % 2 * 16) + nq;
+    else return n0 + 16 * un * U + nq;
+  };
+  const uint32_t ld = anchor == 0 ? p.g.ldc[0] : (anchor == 1 ? p.g.ldc[1] : p.g.ldc[2]);
+  fk_float4v with[ROUNDS][IT][QKV ? 2 : 1];  // the residual's columns; QKV: two pairs' (cos, sin) twice
+  if constexpr (MODE == FK_GEMM_ADD || QKV) {
+#pragma unroll
+    for (int round = 0; round < ROUNDS; round++)
+#pragma unroll
+      for (int it = 0; it < IT; it++) {
+        const uint32_t col = unit_col((wave + it * W) % NU);
+        if constexpr (QKV) {
+          const float *const cs = rope + (size_t)min(upos[round][it], p.r.rope_rows - 1) * 64 + 2 * col;
+          with[round][it][0] = *reinterpret_cast<const fk_float4v *>(cs);
+          with[round][it][1] = *reinterpret_cast<const fk_float4v *>(cs + 4);
+        } else {
+          const uint32_t row = min(unit_row(round, it, lane_e), p.g.m - 1);
+          with[round][it][0] = *reinterpret_cast<const fk_float4v *>(r0 + (size_t)row * ld + col);
+        }
+      }
+  }
   // Nothing may still be landing in LDS when the sums take the rings' place.
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
 
 #pragma unroll
-  for (int i0 = 0; i0 < MB; i0 += MR) {
-    if (i0) __syncthreads();
+  for (int round = 0; round < ROUNDS; round++) {
+    if (round) __syncthreads();
 #pragma unroll
     for (int i = 0; i < MR; i++)
 #pragma unroll
-      for (int j = 0; j < NB; j++) sums[wave][i * NB + j][lane] = acc[i0 + i][j];
+      for (int j = 0; j < NB; j++) sums[wave][i * NB + j][lane_e] = acc[round * MR + i][j];
     __syncthreads();
-    // Unit u of the round: row block u / NU's unit u % NU.
-    for (uint32_t u = wave; u < (uint32_t)(MR * NU); u += W) {
-      const uint32_t i = u / NU, un = u % NU;
-      // Its block q (0 .. U - 1) among the row's.
-      auto block = [&](int q) -> uint32_t {
-        if constexpr (MODE == FK_GEMM_SILU_MUL) return un + q * (NB / 2);
-        else if constexpr (QKV && NB == 2) return q;
-        else if constexpr (QKV) return un / 2 * 4 + un % 2 + 2 * q;
-        else return un * U + q;
-      };
+    // (Unrolled where a unit's operands are in registers; elsewhere a loop,
+    // since straight-line code that runs once is fetched at its own cost:
+    // gate and up of 208 rows unrolled, 31 µs against 28.)
+    constexpr int UNROLL = MODE == FK_GEMM_ADD || QKV ? IT : 1;
+#pragma unroll UNROLL
+    for (int it = 0; it < IT; it++) {
+      const uint32_t u = wave + it * W;
+      if (u >= (uint32_t)UNITS) break;
+      const uint32_t un = u % NU;
+      const uint32_t row = unit_row(round, it, lane_e);
+      const uint32_t col = unit_col(un);
+      // The sum of the unit's block q.
       auto total = [&](int q) {
-        const uint32_t at = i * NB + block(q);
-        fk_float4v v = sums[0][at][lane];
+        uint32_t j;
+        if constexpr (MODE == FK_GEMM_SILU_MUL) j = un + q * (NB / 2);
+        else if constexpr (QKV && NB == 2) j = q;
+        else if constexpr (QKV) j = un / 2 * 4 + un % 2 + 2 * q;
+        else j = un * U + q;
+        const uint32_t at = u / NU * NB + j;
+        fk_float4v v = sums[0][at][lane_e];
 #pragma unroll
-        for (int w = 1; w < W; w++) v += sums[w][at][lane];
+        for (int w = 1; w < W; w++) v += sums[w][at][lane_e];
         return v;
       };
-      const uint32_t row = row_of(i0 + i, lane % 16);
-      const uint32_t nq = 4 * (lane / 16);
       if constexpr (MODE == FK_GEMM_SILU_MUL) {
         const fk_float4v g = total(0), up = total(1);
         if (row >= p.g.m) continue;
         uint16_t h[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) h[r] = fk::to_f16((p.g.act == FK_ACT_GELU_TANH ? fk::act_hw<true>(g[r]) : fk::act_hw<false>(g[r])) * up[r]);
-        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(c0) +
-                                   fk::tile_offset(row, n0 + 16 * un + nq, p.g.ldc[0])) =
+        for (int r = 0; r < 4; r++)
+          h[r] = fk::to_f16((p.g.act == FK_ACT_GELU_TANH ? fk::act_hw<true>(g[r]) : fk::act_hw<false>(g[r])) * up[r]);
+        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(c0) + fk::tile_offset(row, col, ld)) =
             make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
       } else if constexpr (QKV) {
+        // The unit's columns d .. d + 3 of its head, and their partners d + 32 ..
         const fk_float4v lo = total(0), hi = total(1);
         if (row >= p.g.m) continue;
-        // The unit's columns d .. d + 3 of its head, and their partners d + 32 ..
         const uint32_t head = n0 / 64 + (NB == 2 ? 0 : un / 2);
-        const uint32_t d = (NB == 2 ? n0 % 64 : un % 2 * 16) + nq;
-        const uint32_t pos = position[row];
-        const float4 t01 = *reinterpret_cast<const float4 *>(rope + (size_t)min(pos, p.r.rope_rows - 1) * 64 + 2 * d);
-        const float4 t23 =
-            *reinterpret_cast<const float4 *>(rope + (size_t)min(pos, p.r.rope_rows - 1) * 64 + 2 * d + 4);
-        const float cs[4] = {t01.x, t01.z, t23.x, t23.z};
-        const float sn[4] = {t01.y, t01.w, t23.y, t23.w};
+        const uint32_t pos = upos[round][it];
         const bool bf16 = p.r.cache_bf16 != 0 && anchor != 0;
         uint16_t l4[4], h4[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          const float xr = anchor != 2 ? lo[r] * cs[r] - hi[r] * sn[r] : lo[r];
-          const float yr = anchor != 2 ? hi[r] * cs[r] + lo[r] * sn[r] : hi[r];
+          const float cs = with[round][it][r / 2][r % 2 * 2], sn = with[round][it][r / 2][r % 2 * 2 + 1];
+          const float xr = anchor != 2 ? lo[r] * cs - hi[r] * sn : lo[r];
+          const float yr = anchor != 2 ? hi[r] * cs + lo[r] * sn : hi[r];
           l4[r] = bf16 ? fk::narrow_bf16(xr) : fk::to_f16(xr);
           h4[r] = bf16 ? fk::narrow_bf16(yr) : fk::to_f16(yr);
         }
         uint16_t *dst = reinterpret_cast<uint16_t *>(anchor == 0 ? c0 : (anchor == 1 ? c1 : c2));
         if (anchor == 0) {
-          dst += (size_t)row * p.g.ldc[0] + head * 64;
+          dst += (size_t)row * ld + head * 64;
         } else if constexpr (MODE == FK_GEMM_QKV_ROPE_PAGED) {
           // a position past its table stores nothing
           if (pos / p.pg.block_size >= p.pg.table_len) continue;
@@ -279,29 +336,26 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
         } else if (p.r.staged) {
           dst += ((size_t)row * p.r.kv_heads + head) * 64;
         } else {
-          dst += (((size_t)min(slot[row], p.r.slots - 1) * p.r.kv_heads + head) * p.r.length + pos % p.r.length) * 64;
+          dst += (((size_t)min(uslot[round][it], p.r.slots - 1) * p.r.kv_heads + head) * p.r.length + pos % p.r.length) * 64;
         }
-        *reinterpret_cast<uint2 *>(dst + d) =
+        *reinterpret_cast<uint2 *>(dst + col) =
             make_uint2(l4[0] | ((uint32_t)l4[1] << 16), l4[2] | ((uint32_t)l4[3] << 16));
-        *reinterpret_cast<uint2 *>(dst + d + 32) =
+        *reinterpret_cast<uint2 *>(dst + col + 32) =
             make_uint2(h4[0] | ((uint32_t)h4[1] << 16), h4[2] | ((uint32_t)h4[3] << 16));
       } else {
         float *const out = reinterpret_cast<float *>(anchor == 0 ? c0 : (anchor == 1 ? c1 : c2));
-        const uint32_t ld = anchor == 0 ? p.g.ldc[0] : (anchor == 1 ? p.g.ldc[1] : p.g.ldc[2]);
         uint64_t best = 0;
 #pragma unroll
         for (int q = 0; q < U; q++) {
           fk_float4v v = total(q);
-          const uint32_t col = n0 + 16 * (un * U + q) + nq;
-          const size_t o = (size_t)row * ld + col;
           if (row < p.g.m) {
-            if (MODE == FK_GEMM_ADD) v = *reinterpret_cast<const fk_float4v *>(r0 + o) + v;
-            *reinterpret_cast<fk_float4v *>(out + o) = v;
+            if (MODE == FK_GEMM_ADD) v = with[round][it][0] + v;
+            *reinterpret_cast<fk_float4v *>(out + (size_t)row * ld + col + 16 * q) = v;
           }
           if constexpr (MODE == FK_GEMM_STORE_KEYS) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-              const uint64_t key = fk::argmax_key(v[r], col + r);
+              const uint64_t key = fk::argmax_key(v[r], col + 16 * q + r);
               best = key > best ? key : best;
             }
           }
@@ -315,7 +369,7 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
                                    (uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)best, s);
             best = other > best ? other : best;
           }
-          if (lane < 16 && row < p.g.m) keys[(size_t)row * (ld / (16 * NB)) + n0 / (16 * NB)] = best;
+          if (lane_e < 16 && row < p.g.m) keys[(size_t)row * (ld / (16 * NB)) + n0 / (16 * NB)] = best;
         }
       }
     }
@@ -334,26 +388,28 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
     skinny_tile<MODE, MB, NB, W, D>(a, b0, b1, b2, c0, c1, c2, r0, position, slot, rope, keys, p);                \
   }
 
-#define FK_SKINNY_FORM(FORM, MB, NB, W, D)                                      \
-  FK_SKINNY_ENTRY(fk_skinny_store_##FORM, FK_GEMM_STORE, MB, NB, W, 2)          \
-  FK_SKINNY_ENTRY(fk_skinny_add_##FORM, FK_GEMM_ADD, MB, NB, W, 2)              \
-  FK_SKINNY_ENTRY(fk_skinny_store_keys_##FORM, FK_GEMM_STORE_KEYS, MB, NB, W, D)
-#define FK_SKINNY_PAIR_FORM(FORM, MB, NB, W, D)                                 \
-  FK_SKINNY_FORM(FORM, MB, NB, W, D)                                            \
-  FK_SKINNY_ENTRY(fk_skinny_silu_mul_##FORM, FK_GEMM_SILU_MUL, MB, NB, W, D)    \
-  FK_SKINNY_ENTRY(fk_skinny_qkv_rope_##FORM, FK_GEMM_QKV_ROPE, MB, NB, W, 2)    \
-  FK_SKINNY_ENTRY(fk_skinny_qkv_rope_paged_##FORM, FK_GEMM_QKV_ROPE_PAGED, MB, NB, W, 2)
+// S: the ring's steps in the modes that stream many tiles (gate and up, the
+// logits), D in the rest.
+#define FK_SKINNY_FORM(FORM, MB, NB, W, D, S)                                   \
+  FK_SKINNY_ENTRY(fk_skinny_store_##FORM, FK_GEMM_STORE, MB, NB, W, D)          \
+  FK_SKINNY_ENTRY(fk_skinny_add_##FORM, FK_GEMM_ADD, MB, NB, W, D)              \
+  FK_SKINNY_ENTRY(fk_skinny_store_keys_##FORM, FK_GEMM_STORE_KEYS, MB, NB, W, S)
+#define FK_SKINNY_PAIR_FORM(FORM, MB, NB, W, D, S)                              \
+  FK_SKINNY_FORM(FORM, MB, NB, W, D, S)                                         \
+  FK_SKINNY_ENTRY(fk_skinny_silu_mul_##FORM, FK_GEMM_SILU_MUL, MB, NB, W, S)    \
+  FK_SKINNY_ENTRY(fk_skinny_qkv_rope_##FORM, FK_GEMM_QKV_ROPE, MB, NB, W, D)    \
+  FK_SKINNY_ENTRY(fk_skinny_qkv_rope_paged_##FORM, FK_GEMM_QKV_ROPE_PAGED, MB, NB, W, D)
 
 #ifndef FK_SKINNY_FORMS
 #define FK_SKINNY_FORMS
-FK_SKINNY_FORM(m1n1, 1, 1, 8, 2)
-FK_SKINNY_PAIR_FORM(m1n2, 1, 2, 8, 1)
-FK_SKINNY_FORM(m2n1, 2, 1, 8, 2)
-FK_SKINNY_PAIR_FORM(m2n2, 2, 2, 8, 2)
-FK_SKINNY_PAIR_FORM(m2n4, 2, 4, 4, 2)
-FK_SKINNY_PAIR_FORM(m4n2, 4, 2, 8, 2)
-FK_SKINNY_PAIR_FORM(m4n4, 4, 4, 4, 2)
-FK_SKINNY_PAIR_FORM(m4n8, 4, 8, 4, 2)
-FK_SKINNY_PAIR_FORM(m8n4, 8, 4, 4, 2)
-FK_SKINNY_PAIR_FORM(m8n8, 8, 8, 4, 2)
+FK_SKINNY_FORM(m1n1, 1, 1, 8, 2, 2)
+FK_SKINNY_PAIR_FORM(m1n2, 1, 2, 8, 2, 1)
+FK_SKINNY_FORM(m2n1, 2, 1, 8, 2, 2)
+FK_SKINNY_PAIR_FORM(m2n2, 2, 2, 8, 2, 2)
+FK_SKINNY_PAIR_FORM(m2n4, 2, 4, 4, 2, 2)
+FK_SKINNY_PAIR_FORM(m4n2, 4, 2, 8, 2, 2)
+FK_SKINNY_PAIR_FORM(m4n4, 4, 4, 4, 2, 2)
+FK_SKINNY_PAIR_FORM(m4n8, 4, 8, 4, 2, 2)
+FK_SKINNY_PAIR_FORM(m8n4, 8, 4, 4, 2, 2)
+FK_SKINNY_PAIR_FORM(m8n8, 8, 8, 4, 2, 1)
 #endif

@@ -143,37 +143,50 @@ def _row_attention(out: Lowered, live: LiveRows) -> None:
     out.launches[:] = launches
 
 
-def skinny_form(chunks: int, m: int, n: int, k: int, pairs: bool) -> Optional[str]:
-    """The form of fk_skinny that a GEMM of `chunks` live chunks of 16 rows
-    (of a step of m) by n weight rows of k columns takes, or None where the
-    256 × 256 tiles of fk_gemm are faster (MI355X, 256 CUs; µs, f16):
+# What a tile of each form of fk_skinny costs a CU: µs a tile and a step of 32
+# columns (fitted on MI355X to launches at n 2048 and k 2048 and 8192), and
+# whether a CU holds one tile at a time (its LDS is half a CU's or more) or
+# several.
+SKINNY_COST = {"m1n1": (1.1, 0.037, False), "m1n2": (1.4, 0.054, False), "m2n1": (1.4, 0.047, False),
+               "m2n2": (1.9, 0.056, False), "m2n4": (2.3, 0.089, False), "m4n2": (2.4, 0.074, True),
+               "m4n4": (3.3, 0.110, False), "m4n8": (7.0, 0.150, True), "m8n4": (7.0, 0.150, True),
+               "m8n8": (11.5, 0.202, True)}
 
-    - A launch of 256 × 256 tiles costs its rounds of 256 tiles, whatever
-      its rows: 46 a round at k 2048, 151 at 8192.  A round of skinny's
-      largest tiles (128 × 128, k split in 4) costs about half of that (25
-      and 66), so skinny takes over at half as many rounds more: at n 2048,
-      1408 rows take 25 against 46 (k 2048) and 66 against 152 (k 8192); at
-      n 16384, 208 rows 28 against 44, but 352 rows (two rounds) 49 against
-      47 and 704 (three) 74 against 51.
-    - Of its forms, the largest tile of which there are 140 or more (half
-      the chip busy): a larger one reads its operands fewer times, a smaller
-      one fills more CUs.  At k 8192 and n 2048: 16 rows 12.2 (m1n1), 112
-      rows 18.3 (m2n2; m4n2's 128 tiles 25.6), 208 rows 22.9 (m4n2), 352
-      rows 32 (m4n4), 704 rows 44 (m8n4; m8n8's 96 tiles 61).
-    - A k shorter than 1024 leaves a wavefront under four steps to
-      overlap."""
+
+def skinny_form(chunks: int, m: int, n: int, k: int, mode: str) -> Optional[str]:
+    """The form of fk_skinny that a GEMM of `chunks` live chunks of 16 rows
+    (of a step of m) by n weight rows of k columns takes for the epilogue
+    `mode`, or None where the 256 × 256 tiles of fk_gemm are faster: the
+    least of
+
+    - fk_gemm: its tiles in rounds of 256 (one a CU), 0.55 µs a step of 32
+      columns and 11 a round, 17 with the residual's or QKV's epilogue (46
+      and 52 at k 2048, 158 for down, whatever the rows);
+    - a form: 2 µs, and SKINNY_COST's for as many tiles as a CU takes.
+
+    So, measured: O and down (n 2048) of 1408 rows take m8n8's 176 tiles (26
+    against 55, 65 against 160 at k 8192); gate and up (n 16384) of 208 rows
+    its 256 (28 against 44), but of 352 rows, two rounds, fk_gemm (49 against
+    47).  Among forms, down: 16 rows m1n1 (12.5), 112 rows m2n2 (18.2; m4n2,
+    half as many tiles, 25.6), 352 rows m4n4 (33.7; m4n2 43), 704 rows m8n4
+    (45.9; m4n4 60).  A k shorter than 1024 leaves a wavefront under four
+    steps to overlap and stays."""
     if k < 1024 or m * k * 2 >= 0xfffffff0:
         return None
-    tiles = (m // SLAB) * (n // SLAB)
-    largest = -(-chunks // 8) * (n // 128)
-    if 2 * -(-largest // 256) > 3 * -(-tiles // 256):
-        return None
+    steps = k / 32
+    pairs = mode in SKINNY_PAIR_MODES
+    ends = 11 if mode in ("store", "silu_mul", "store_keys") else 17
+    least = -(-(m // SLAB) * (n // SLAB) // 256) * (ends + 0.55 * steps)
     best = None
     for form, (mb, nb, _) in SKINNY_FORMS.items():
         if mb >= 2 * chunks or (pairs and nb == 1):
             continue
-        if best is None or -(-chunks // mb) * (n // (16 * nb)) >= 140:
-            best = form
+        tile, step, one = SKINNY_COST[form]
+        share = -(-chunks // mb) * (n // (16 * nb)) / 256
+        share = max(1.0, float(np.ceil(share))) if one else (share + 0.25 if share > 1 else 1.0)
+        cost = 2 + share * (tile + steps * step)
+        if cost < least:
+            best, least = form, cost
     return best
 
 
@@ -187,7 +200,7 @@ def _skinny_gemms(out: Lowered, live: LiveRows) -> None:
         p = gm.params
         mode = gm.entry[len("fk_gemm_f16_"):]
         n = 2 * p["ldc"][0] if mode == "silu_mul" else p["first_col"][p["n_anchors"]]
-        form = skinny_form(live.chunks, p["m"], n, p["k"], mode in SKINNY_PAIR_MODES)
+        form = skinny_form(live.chunks, p["m"], n, p["k"], mode)
         if form is None:
             continue
         mb, nb, waves = SKINNY_FORMS[form]

@@ -71,7 +71,7 @@ def test_every_launch_passes_the_checks_and_makes_the_live_rows(case):
                     short[i] = (short[i][0], short[i][1] - 1)
                     with pytest.raises(runtime.FkError):
                         runtime.launch_check(L.entry, L.groups, L.threads, L.lds_bytes, short, params_struct(L))
-    assert skinny == {"4 x 1500": 0, "2 x 700": 2, "1 x 256": 4}.get(case, 5)
+    assert skinny == {"4 x 1500": 0, "2 x 700": 3, "1 x 256": 4}.get(case, 5)
 
 
 def test_the_keys_of_the_head_follow_its_tile():
@@ -99,13 +99,21 @@ def test_a_prefills_attention_stays():
 
 
 def test_forms_by_size():
-    # the largest tile that fills half the chip; none where fk_gemm's rounds are as few
-    assert [skinny_form(c, 256, 2048, 8192, False) for c in (1, 3, 4, 7, 13, 16)] == \
-        ["m1n1", "m2n1", "m2n1", "m2n2", "m4n2", "m4n2"]
-    assert skinny_form(88, 1536, 2048, 8192, False) == "m8n8"
-    assert skinny_form(1, 256, 3072, 2048, True) == "m1n2"      # pairs of columns
-    assert skinny_form(22, 512, 16384, 2048, True) is None
-    assert skinny_form(512, 8192, 2048, 8192, False) is None
-    assert skinny_form(1, 256, 2048, 960, False) is None        # a short k
+    def down(c):
+        return skinny_form(c, -(-c // 16) * 256, 2048, 8192, "add")
+    # larger tiles as the rows grow; fk_gemm where its rounds are full
+    assert [down(c) for c in (1, 3, 4, 7, 13, 22, 88, 128, 512)] == \
+        ["m1n1", "m2n1", "m2n1", "m2n2", "m4n2", "m4n4", "m8n8", "m8n8", None]
+    assert skinny_form(1, 256, 3072, 2048, "qkv_rope") == "m1n2"      # pairs of columns
+    assert skinny_form(22, 512, 16384, 2048, "silu_mul") is None
+    assert skinny_form(1, 256, 2048, 960, "add") is None              # a short k
+    for c in range(1, 400):
+        m = -(-c // 16) * 256
+        for n, k, mode in ((3072, 2048, "qkv_rope_paged"), (16384, 2048, "silu_mul"), (32000, 2048, "store_keys"),
+                           (256, 1024, "store"), (512, 16384, "add")):
+            form = skinny_form(c, m, n, k, mode)
+            if form is not None:
+                mb, nb, _ = K.SKINNY_FORMS[form]
+                assert mb < 2 * c and n % (16 * nb) == 0 and (nb > 1 or mode not in K.SKINNY_PAIR_MODES)
     assert all(L.entry.startswith("fk_skinny") is False
                for L in lowered(SMALL_PREFILL, 2, 100)[0].launches)
