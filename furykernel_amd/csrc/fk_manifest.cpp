@@ -105,6 +105,34 @@ struct SkinnyForm {
 const SkinnyForm skinny_forms[] = {{"m1n1", 1, 1, 8}, {"m1n2", 1, 2, 8}, {"m2n1", 2, 1, 8}, {"m2n2", 2, 2, 8},
                                    {"m2n4", 2, 4, 4}, {"m4n2", 4, 2, 8}, {"m4n4", 4, 4, 4}, {"m4n8", 4, 8, 4},
                                    {"m8n4", 8, 4, 4}, {"m8n8", 8, 8, 4}};
+// The forms of the prefill attention whose keys are split among groups of
+// wavefronts: heads (wavefronts) a group, groups.
+struct SplitForm {
+  uint32_t heads, groups;
+};
+const SplitForm split_forms[] = {{4, 2}, {2, 2}, {1, 2}, {2, 4}, {1, 4}};
+
+// What an entry of the prefill attention is, by its name
+// (fk_prefill_attend_[paged_][f16_]g<heads>, fk_split_attend_[paged_][f16_]h<heads>k<groups>).
+struct AttendEntry {
+  bool is = false, paged = false, f16 = false;
+  uint32_t heads = 0, groups = 1;  // wavefronts a group of keys, groups
+  // threadgroups a (query block, kv head) of `g` query heads, 0 if they don't divide
+  uint32_t parts(uint32_t g) const { return groups == 1 ? g == heads : (g && g % heads == 0 ? g / heads : 0); }
+};
+AttendEntry attend_entry(const char *entry) {
+  AttendEntry a;
+  const bool split = std::strncmp(entry, "fk_split_attend_", 16) == 0;
+  if (!split && std::strncmp(entry, "fk_prefill_attend_", 18) != 0) return a;
+  const char *at = entry + (split ? 16 : 18);
+  if (std::strncmp(at, "paged_", 6) == 0) a.paged = true, at += 6;
+  if (std::strncmp(at, "f16_", 4) == 0) a.f16 = true, at += 4;
+  a.heads = (uint32_t)(at[1] - '0');
+  if (split) a.groups = (uint32_t)(at[3] - '0');
+  a.is = true;
+  return a;
+}
+
 const char *const skinny_modes[] = {"store", "add", "store_keys", "silu_mul", "qkv_rope", "qkv_rope_paged"};
 
 bool skinny_pairs(const char *mode) {
@@ -395,29 +423,36 @@ std::vector<Entry> build() {
   }
   {
     using S = fk_prefill_attend_params;
-    for (const char *form : {"fk_prefill_attend_g", "fk_prefill_attend_f16_g"})
-    for (int g : {1, 2, 4})
-      add(form + std::to_string(g), 64 * g,
-          {buf("qr", "read", "f16"), buf("kc", "read", "f16"), buf("vc", "read", "f16"),
-           buf("position", "read", "u32"), buf("slot", "read", "u32"), buf("out", "write", "f16"),
-           buf("ks", "read", "f16"), buf("vs", "read", "f16")},
-          {FK_P(S, rows, "u32"), FK_P(S, heads, "u32"), FK_P(S, kv_heads, "u32"), FK_P(S, length, "u32"),
-           FK_P(S, slots, "u32"), FK_P(S, window, "u32"), FK_P(S, cache_bf16, "u32"), FK_P(S, scale, "f32"),
-           FK_P(S, staged, "u32"), FK_P(S, run_rows, "u32")},
-          sizeof(S));
+    const std::vector<fk_abi_buffer> b = {buf("qr", "read", "f16"), buf("kc", "read", "f16"), buf("vc", "read", "f16"),
+                                          buf("position", "read", "u32"), buf("slot", "read", "u32"),
+                                          buf("out", "write", "f16"), buf("ks", "read", "f16"), buf("vs", "read", "f16")};
+    const std::vector<fk_abi_param> p = {FK_P(S, rows, "u32"), FK_P(S, heads, "u32"), FK_P(S, kv_heads, "u32"),
+                                         FK_P(S, length, "u32"), FK_P(S, slots, "u32"), FK_P(S, window, "u32"),
+                                         FK_P(S, cache_bf16, "u32"), FK_P(S, scale, "f32"), FK_P(S, staged, "u32"),
+                                         FK_P(S, run_rows, "u32")};
+    for (const char *form : {"", "f16_"}) {
+      for (int g : {1, 2, 4}) add("fk_prefill_attend_" + (form + ("g" + std::to_string(g))), 64 * g, b, p, sizeof(S));
+      for (const SplitForm &f : split_forms)
+        add("fk_split_attend_" + (form + ("h" + std::to_string(f.heads))) + "k" + std::to_string(f.groups),
+            64 * f.heads * f.groups, b, p, sizeof(S));
+    }
   }
   {
     using S = fk_prefill_attend_paged_params;
-    for (const char *form : {"fk_prefill_attend_paged_g", "fk_prefill_attend_paged_f16_g"})
-    for (int g : {1, 2, 4})
-      add(form + std::to_string(g), 64 * g,
-          {buf("qr", "read", "f16"), buf("kc", "read", "f16"), buf("vc", "read", "f16"),
-           buf("position", "read", "u32"), buf("table", "read", "u32"), buf("out", "write", "f16")},
-          {FK_P(S, a.rows, "u32"), FK_P(S, a.heads, "u32"), FK_P(S, a.kv_heads, "u32"), FK_P(S, a.length, "u32"),
-           FK_P(S, a.slots, "u32"), FK_P(S, a.window, "u32"), FK_P(S, a.cache_bf16, "u32"), FK_P(S, a.scale, "f32"),
-           FK_P(S, a.staged, "u32"), FK_P(S, a.run_rows, "u32"), FK_P(S, g.block_size, "u32"),
-           FK_P(S, g.table_len, "u32"), FK_P(S, g.blocks, "u32")},
-          sizeof(S));
+    const std::vector<fk_abi_buffer> b = {buf("qr", "read", "f16"), buf("kc", "read", "f16"), buf("vc", "read", "f16"),
+                                          buf("position", "read", "u32"), buf("table", "read", "u32"),
+                                          buf("out", "write", "f16")};
+    const std::vector<fk_abi_param> p = {
+        FK_P(S, a.rows, "u32"),       FK_P(S, a.heads, "u32"),     FK_P(S, a.kv_heads, "u32"), FK_P(S, a.length, "u32"),
+        FK_P(S, a.slots, "u32"),      FK_P(S, a.window, "u32"),    FK_P(S, a.cache_bf16, "u32"), FK_P(S, a.scale, "f32"),
+        FK_P(S, a.staged, "u32"),     FK_P(S, a.run_rows, "u32"),  FK_P(S, g.block_size, "u32"),
+        FK_P(S, g.table_len, "u32"),  FK_P(S, g.blocks, "u32")};
+    for (const char *form : {"paged_", "paged_f16_"}) {
+      for (int g : {1, 2, 4}) add("fk_prefill_attend_" + (form + ("g" + std::to_string(g))), 64 * g, b, p, sizeof(S));
+      for (const SplitForm &f : split_forms)
+        add("fk_split_attend_" + (form + ("h" + std::to_string(f.heads))) + "k" + std::to_string(f.groups),
+            64 * f.heads * f.groups, b, p, sizeof(S));
+    }
   }
   add("fk_prefill_softcap", 256, {buf("x", "read", "f32"), buf("y", "write", "f32")},
       {FK_P(fk_prefill_softcap_params, count, "u32"), FK_P(fk_prefill_softcap_params, cap, "f32")},
@@ -910,13 +945,13 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
       need.push_back({"slot", m * 4 * (paged ? p.pg.table_len : 1)});
       need.push_back({"rope", (uint64_t)p.r.rope_rows * 256});
     }
-  } else if (std::strncmp(entry, "fk_prefill_attend_g", 19) == 0 ||
-             std::strncmp(entry, "fk_prefill_attend_f16_g", 23) == 0) {
+  } else if (attend_entry(entry).is && !attend_entry(entry).paged) {
+    const AttendEntry form = attend_entry(entry);
     fk_prefill_attend_params p;
     std::memcpy(&p, params, sizeof p);
     // The f16 form loads f16 ring rows straight into LDS: no bf16 rows to
     // convert, no staged rows.
-    if (entry[18] == 'f' && (p.cache_bf16 || p.staged))
+    if (form.f16 && (p.cache_bf16 || p.staged))
       return bad(err, cap, FK_ERR_ARG, "%s: bf16 caches %u or staged rows %u", entry, p.cache_bf16, p.staged);
     const uint64_t kw = (uint64_t)p.kv_heads * 64 * 2;
     need = {{"qr", (uint64_t)p.rows * p.heads * 64 * 2},
@@ -925,16 +960,17 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
             {"position", (uint64_t)p.rows * 4},
             {"slot", (uint64_t)p.rows * 4},
             {"out", (uint64_t)p.rows * p.heads * 64 * 2}};
-    const uint32_t g = (uint32_t)(entry[std::strlen(entry) - 1] - '0');
+    const uint32_t parts = p.kv_heads && p.heads % p.kv_heads == 0 ? form.parts(p.heads / p.kv_heads) : 0;
     if ((p.staged && p.run_rows == 0) || (p.run_rows && (p.run_rows % 32 || p.rows % p.run_rows)) || p.rows % 32 ||
         p.rows == 0 || p.kv_heads == 0)
       return bad(err, cap, FK_ERR_ARG, "%s: runs of %u rows in a step of %u (multiples of 32 that divide it)", entry,
                  p.run_rows, p.rows);
     // The grid is every (query block, kv head), heaviest first: a larger
     // grid would index blocks past their run; the heads are the group's
-    // wavefronts; keys go by blocks of 64 positions.
-    if (p.heads != g * p.kv_heads || p.length == 0 || p.length % 64 || p.slots == 0 ||
-        (uint64_t)groups != (uint64_t)(p.rows / 32) * p.kv_heads || threads != g * 64)
+    // wavefronts (a split form's: its parts of them, its groups of keys
+    // times); keys go by blocks of 64 positions.
+    if (parts == 0 || p.length == 0 || p.length % 64 || p.slots == 0 ||
+        (uint64_t)groups != (uint64_t)(p.rows / 32) * p.kv_heads * parts || threads != form.heads * form.groups * 64)
       return bad(err, cap, FK_ERR_ARG, "%s: %u heads over %u, a ring of %u, %u threadgroups of %u threads", entry,
                  p.heads, p.kv_heads, p.length, groups, threads);
     if (p.staged) {
@@ -962,22 +998,22 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
             {"v", (uint64_t)p.rows * kw * 4}, {"position", (uint64_t)p.rows * 4},
             {"table", (uint64_t)p.rows * pp.g.table_len * 4}, {"rope", (uint64_t)p.rope_rows * p.rotated * 8},
             {"qr", (uint64_t)p.rows * p.heads * p.head_dim * 2}, {"kc", pool}, {"vc", pool}};
-  } else if (std::strncmp(entry, "fk_prefill_attend_paged_g", 25) == 0 ||
-             std::strncmp(entry, "fk_prefill_attend_paged_f16_g", 29) == 0) {
+  } else if (attend_entry(entry).is) {
+    const AttendEntry form = attend_entry(entry);
     fk_prefill_attend_paged_params pp;
     std::memcpy(&pp, params, sizeof pp);
     const fk_prefill_attend_params &p = pp.a;
-    const uint32_t g = (uint32_t)(entry[std::strlen(entry) - 1] - '0');
+    const uint32_t parts = p.kv_heads && p.heads % p.kv_heads == 0 ? form.parts(p.heads / p.kv_heads) : 0;
     // The f16 form loads f16 pool rows straight into LDS, at 32-bit offsets
     // into the pool, through a block table it holds in LDS (256 entries).
-    if (entry[24] == 'f' &&
+    if (form.f16 &&
         (p.cache_bf16 || pp.g.table_len > 256 ||
          (uint64_t)pp.g.blocks * p.kv_heads * pp.g.block_size * 128 > 0xFFFFFFFFull))
       return bad(err, cap, FK_ERR_ARG, "%s: bf16 caches %u, tables of %u, a pool of %u blocks", entry, p.cache_bf16,
                  pp.g.table_len, pp.g.blocks);
-    if (p.rows == 0 || p.rows % 32 || p.kv_heads == 0 || p.heads != g * p.kv_heads || p.staged ||
+    if (p.rows == 0 || p.rows % 32 || parts == 0 || p.staged ||
         (p.run_rows && (p.run_rows % 32 || p.rows % p.run_rows)) || pp.g.block_size == 0 || pp.g.table_len == 0 ||
-        pp.g.blocks == 0 || groups != (p.rows / 32) * p.kv_heads)
+        pp.g.blocks == 0 || groups != (p.rows / 32) * p.kv_heads * parts)
       return bad(err, cap, FK_ERR_ARG, "%s: %u rows, %u heads over %u, blocks of %u, tables of %u, %u threadgroups",
                  entry, p.rows, p.heads, p.kv_heads, pp.g.block_size, pp.g.table_len, groups);
     const uint64_t pool = (uint64_t)pp.g.blocks * p.kv_heads * pp.g.block_size * 64 * 2;

@@ -1,7 +1,8 @@
 // fk_attend.h — the prefill's causal attention on the matrix cores
-// (src/FuryKernel/Program/Eval.hs:351-380 per row).  Built into a code object
-// of its own (fk_attend.hip) with the compiler's VGPR form of the matrix
-// operations: the online softmax rescales its output accumulators with
+// (src/FuryKernel/Program/Eval.hs:351-380 per row).  Its entries are
+// fk_attend.hip's, a code object of their own built with the compiler's VGPR
+// form of the matrix operations, and fk_split_attend.h's, whose launch bounds
+// select that form: the online softmax rescales its output accumulators with
 // plain arithmetic, which on accumulators held in AGPRs would copy them out
 // and back every block of keys.
 #pragma once
@@ -71,7 +72,12 @@ typedef float fk_float2v __attribute__((ext_vector_type(2)));
 // would place them; keys past the block's last query read that query's own
 // row (its score is masked and its probability 0, so a finite row is all
 // it needs).
-template <uint32_t G, bool PG = false, bool DIRECT = false>
+// KS: the block's keys split among KS groups of G wavefronts, group i taking
+// the key blocks i, i + KS, ... through buffers of its own; their outputs meet
+// in LDS at the end (fk_split_attend_*).  G is then the query heads of a
+// group, which may be fewer than a kv head's: a threadgroup takes one of the
+// kv head's heads / kv_heads / G parts.
+template <uint32_t G, bool PG = false, bool DIRECT = false, uint32_t KS = 1>
 __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc,
                                                const uint16_t *__restrict__ vc, const uint32_t *__restrict__ position,
                                                const uint32_t *__restrict__ slot, uint16_t *__restrict__ out,
@@ -79,13 +85,16 @@ __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, 
                                                const fk_prefill_attend_params &p,
                                                const fk_paging &pg = fk_paging{}) {
   // The two buffers of K and of V: four objects (see the direct loop for why).
-  __shared__ __attribute__((aligned(16))) uint16_t ks0[FK_ATT_KB * 64], ks1[FK_ATT_KB * 64];
-  __shared__ __attribute__((aligned(16))) uint16_t vs0[FK_ATT_KB * 64], vs1[FK_ATT_KB * 64];
-  constexpr uint32_t nthreads = G * FK_WAVE;
+  __shared__ __attribute__((aligned(16))) uint16_t ks0s[KS * FK_ATT_KB * 64], ks1s[KS * FK_ATT_KB * 64];
+  __shared__ __attribute__((aligned(16))) uint16_t vs0s[KS * FK_ATT_KB * 64], vs1s[KS * FK_ATT_KB * 64];
+  constexpr uint32_t nthreads = G * FK_WAVE;           // threads of a group
   constexpr uint32_t per = FK_ATT_KB * 8 / nthreads;   // 16-byte units of K (and of V) a thread stages
-  const uint32_t tid = threadIdx.x;
+  const uint32_t ksi = KS == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x / nthreads);  // the group
+  const uint32_t tid = threadIdx.x - ksi * nthreads;
   const uint32_t lane = tid & (FK_WAVE - 1);
   const uint32_t wave = tid / FK_WAVE;
+  uint16_t *const ks0 = ks0s + ksi * FK_ATT_KB * 64, *const ks1 = ks1s + ksi * FK_ATT_KB * 64;
+  uint16_t *const vs0 = vs0s + ksi * FK_ATT_KB * 64, *const vs1 = vs1s + ksi * FK_ATT_KB * 64;
   // Heaviest first: a block's keys grow with its place in its run (a
   // sequence's consecutive positions), so threadgroup j takes, of every run
   // and kv head, the run's last block first, then the one before: the
@@ -93,11 +102,12 @@ __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, 
   const uint32_t qblocks = p.rows / 32;
   const uint32_t per_run = (p.run_rows ? p.run_rows : p.rows) / 32;  // blocks a run
   const uint32_t runs = qblocks / per_run;
-  const uint32_t t_rank = blockIdx.x / (runs * p.kv_heads);
-  const uint32_t rest = blockIdx.x % (runs * p.kv_heads);
-  const uint32_t r0 = ((rest / p.kv_heads) * per_run + (per_run - 1 - t_rank)) * 32;  // the block's first row
-  const uint32_t g = rest % p.kv_heads;                                               // kv head
-  const uint32_t h = g * G + wave;                   // this wavefront's query head
+  const uint32_t parts = KS == 1 ? 1u : p.heads / p.kv_heads / G;  // threadgroups a kv head
+  const uint32_t t_rank = blockIdx.x / (runs * p.kv_heads * parts);
+  const uint32_t rest = blockIdx.x % (runs * p.kv_heads * parts);
+  const uint32_t r0 = ((rest / (p.kv_heads * parts)) * per_run + (per_run - 1 - t_rank)) * 32;  // the block's first row
+  const uint32_t g = rest / parts % p.kv_heads;                                                 // kv head
+  const uint32_t h = (g * parts + rest % parts) * G + wave;  // this wavefront's query head
   const uint32_t p0 = position[r0];
   const uint32_t sl = PG ? 0u : min(slot[r0], p.slots - 1);
   const uint32_t *const tab = slot + (size_t)r0 * pg.table_len;  // PG: the block's table
@@ -310,6 +320,8 @@ __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, 
   // block kb + 1's K and V rows are on their way from the caches into
   // registers, and go into the other pair after (every wavefront left it at
   // the last barrier); one barrier a block.
+  // (KS groups: group i's blocks are kb0 + i, kb0 + i + KS, ...; the groups
+  // meet the same barriers, those whose blocks have ended without work.)
   const uint32_t kb0 = first_pos / FK_ATT_KB, kb_last = last_pos / FK_ATT_KB;
   if constexpr (DIRECT) {
     // Block kb's rows into buffer buf: wavefront w's q-th load fills keys
@@ -326,7 +338,7 @@ __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, 
     __shared__ uint32_t ltab[PG ? FK_ATT_TABLE : 1];
     if constexpr (PG) {
       const uint32_t used = min(last_pos / pg.block_size + 1, pg.table_len);
-      for (uint32_t i = tid; i < used; i += nthreads) ltab[i] = min(tab[i], pg.blocks - 1);
+      for (uint32_t i = threadIdx.x; i < used; i += KS * nthreads) ltab[i] = min(tab[i], pg.blocks - 1);
       __syncthreads();
     }
     // A ring block whose keys all come before the block's last query reads
@@ -380,39 +392,99 @@ __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, 
     // block; with them the loads fly during the block.
     auto blk = [&](uint32_t kb, const uint16_t *__restrict__ kbuf, const uint16_t *__restrict__ vbuf,
                    uint16_t *__restrict__ kdst, uint16_t *__restrict__ vdst) {
-      if (kb < kb_last) fetch_direct(kb + 1, kdst, vdst);
-      step(kb, kbuf, vbuf);
+      if (kb + KS <= kb_last) fetch_direct(kb + KS, kdst, vdst);
+      if (KS == 1 || kb <= kb_last) step(kb, kbuf, vbuf);
     };
-    fetch_direct(kb0, ks0, vs0);
+    if (KS == 1 || kb0 + ksi <= kb_last) fetch_direct(kb0 + ksi, ks0, vs0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    for (uint32_t kb = kb0; kb <= kb_last; kb++) {
-      const bool odd = (kb - kb0) & 1;
+    bool odd = false;
+    for (uint32_t kbg = kb0; kbg <= kb_last; kbg += KS, odd = !odd) {
+      const uint32_t kb = kbg + ksi;
       blk(kb, odd ? ks1 : ks0, odd ? vs1 : vs0, odd ? ks0 : ks1, odd ? vs0 : vs1);
       __builtin_amdgcn_s_waitcnt(0);  // this wavefront's loads of block kb + 1 landed
       __syncthreads();
     }
   } else {
-  if constexpr (PG) locate(kb0);
-  fetch(kreg, kc, kst, kb0);
-  fetch(vreg, vc, vst, kb0);
-  stash_k(0);
-  stash_v(0);
+  if (KS == 1 || kb0 + ksi <= kb_last) {
+    if constexpr (PG) locate(kb0 + ksi);
+    fetch(kreg, kc, kst, kb0 + ksi);
+    fetch(vreg, vc, vst, kb0 + ksi);
+    stash_k(0);
+    stash_v(0);
+  }
   __syncthreads();
-  for (uint32_t kb = kb0; kb <= kb_last; kb++) {
-    const uint32_t buf = (kb - kb0) & 1;
-    if (kb < kb_last) {
-      if constexpr (PG) locate(kb + 1);
-      fetch(kreg, kc, kst, kb + 1);
-      fetch(vreg, vc, vst, kb + 1);
+  uint32_t buf = 0;
+  for (uint32_t kbg = kb0; kbg <= kb_last; kbg += KS, buf ^= 1) {
+    const uint32_t kb = kbg + ksi;
+    if (kb + KS <= kb_last) {
+      if constexpr (PG) locate(kb + KS);
+      fetch(kreg, kc, kst, kb + KS);
+      fetch(vreg, vc, vst, kb + KS);
     }
-    step(kb, buf ? ks1 : ks0, buf ? vs1 : vs0);
-    if (kb < kb_last) {
+    if (KS == 1 || kb <= kb_last) step(kb, buf ? ks1 : ks0, buf ? vs1 : vs0);
+    if (kb + KS <= kb_last) {
       stash_k(buf ^ 1);
       stash_v(buf ^ 1);
     }
     __syncthreads();
   }
+  }
+
+  if constexpr (KS > 1) {
+    // The groups' outputs, added by the first in the order of the groups:
+    // each query's reference maximum, sum and Oᵀ through LDS (the K and V
+    // buffers, free after the last barrier; a wavefront's state 8.5 KB),
+    // brought to the largest of the references.
+    constexpr uint32_t HALF = KS * FK_ATT_KB * 64 / 2;  // floats an array of buffers holds
+    static_assert((KS - 1) * G * FK_WAVE * 16 <= HALF, "the outputs must fit the buffers");
+    float *const of0 = reinterpret_cast<float *>(ks0s), *const of1 = reinterpret_cast<float *>(ks1s);
+    float *const mf = reinterpret_cast<float *>(vs0s);
+    const uint32_t at = (((ksi - 1) * G + wave) * FK_WAVE + lane) * 4;
+    constexpr uint32_t APART = (KS - 1) * G * FK_WAVE * 4;  // from a quarter of Oᵀ's registers to the next
+    if (ksi) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        *reinterpret_cast<fk_float4v *>(of0 + q * APART + at) =
+            fk_float4v{o[0][4 * q], o[0][4 * q + 1], o[0][4 * q + 2], o[0][4 * q + 3]};
+        *reinterpret_cast<fk_float4v *>(of1 + q * APART + at) =
+            fk_float4v{o[1][4 * q], o[1][4 * q + 1], o[1][4 * q + 2], o[1][4 * q + 3]};
+      }
+      mf[at / 4] = mrun;
+      mf[APART / 4 + at / 4] = lrun;
+    }
+    __syncthreads();
+    if (ksi) return;
+    float mg[KS], all = mrun;
+#pragma unroll
+    for (uint32_t i = 1; i < KS; i++) {
+      mg[i] = mf[((i - 1) * G + wave) * FK_WAVE + lane];
+      all = __builtin_fmaxf(all, mg[i]);
+    }
+    const float mc = all == -__builtin_inff() ? 0.0f : all;
+    const float f0 = __builtin_amdgcn_exp2f(mrun - mc);
+    lrun *= f0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      o[0][r] *= f0;
+      o[1][r] *= f0;
+    }
+#pragma unroll
+    for (uint32_t i = 1; i < KS; i++) {
+      const uint32_t from = (((i - 1) * G + wave) * FK_WAVE + lane) * 4;
+      const float f = __builtin_amdgcn_exp2f(mg[i] - mc);
+      lrun += mf[APART / 4 + from / 4] * f;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const fk_float4v a = *reinterpret_cast<const fk_float4v *>(of0 + q * APART + from);
+        const fk_float4v b = *reinterpret_cast<const fk_float4v *>(of1 + q * APART + from);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          o[0][4 * q + r] += a[r] * f;
+          o[1][4 * q + r] += b[r] * f;
+        }
+      }
+    }
   }
 
   // O = Oᵀ / sum into the tile layout: lane l's query row, d = 32 db + 8 gg +
@@ -428,55 +500,3 @@ __device__ __forceinline__ void prefill_attend(const uint16_t *__restrict__ qr, 
       *reinterpret_cast<uint2 *>(out + fk::tile_offset(qrow, col, qw)) = make_uint2(lo, hi);
     }
 }
-
-// One entry a group size G = heads / kv_heads (threads 64 G).
-#define FK_PREFILL_ATTEND(G)                                                                                    \
-  extern "C" __global__ void __launch_bounds__(64 * G) fk_prefill_attend_g##G(                         \
-      const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,       \
-      const uint32_t *__restrict__ position, const uint32_t *__restrict__ slot, uint16_t *__restrict__ out,   \
-      const uint16_t *__restrict__ ks, const uint16_t *__restrict__ vs, fk_prefill_attend_params p) {          \
-    prefill_attend<G>(qr, kc, vc, position, slot, out, ks, vs, p);                                              \
-  }
-FK_PREFILL_ATTEND(1)
-FK_PREFILL_ATTEND(2)
-FK_PREFILL_ATTEND(4)
-
-// The same over f16 rings with no staged rows, each block's rows loaded
-// straight into LDS (the same bindings; ks and vs unused).
-#define FK_PREFILL_ATTEND_F16(G)                                                                                \
-  extern "C" __global__ void __launch_bounds__(64 * G) fk_prefill_attend_f16_g##G(                     \
-      const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,       \
-      const uint32_t *__restrict__ position, const uint32_t *__restrict__ slot, uint16_t *__restrict__ out,   \
-      const uint16_t *__restrict__ ks, const uint16_t *__restrict__ vs, fk_prefill_attend_params p) {          \
-    prefill_attend<G, false, true>(qr, kc, vc, position, slot, out, nullptr, nullptr, p);                      \
-  }
-FK_PREFILL_ATTEND_F16(1)
-FK_PREFILL_ATTEND_F16(2)
-FK_PREFILL_ATTEND_F16(4)
-
-// The same over paged pools: kc and vc the pools, `table` the rows' block
-// tables; no staged rows.
-#define FK_PREFILL_ATTEND_PAGED(G)                                                                                \
-  extern "C" __global__ void __launch_bounds__(64 * G) fk_prefill_attend_paged_g##G(                             \
-      const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,         \
-      const uint32_t *__restrict__ position, const uint32_t *__restrict__ table, uint16_t *__restrict__ out,     \
-      fk_prefill_attend_paged_params p) {                                                                        \
-    prefill_attend<G, true>(qr, kc, vc, position, table, out, nullptr, nullptr, p.a, p.g);                       \
-  }
-FK_PREFILL_ATTEND_PAGED(1)
-FK_PREFILL_ATTEND_PAGED(2)
-FK_PREFILL_ATTEND_PAGED(4)
-
-// The same over f16 pools (under 4 GiB, tables of at most FK_ATT_TABLE
-// blocks), each block's rows loaded straight into LDS.
-#define FK_PREFILL_ATTEND_PAGED_F16(G)                                                                            \
-  extern "C" __global__ void __launch_bounds__(64 * G) fk_prefill_attend_paged_f16_g##G(                         \
-      const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc, const uint16_t *__restrict__ vc,         \
-      const uint32_t *__restrict__ position, const uint32_t *__restrict__ table, uint16_t *__restrict__ out,     \
-      fk_prefill_attend_paged_params p) {                                                                        \
-    prefill_attend<G, true, true>(qr, kc, vc, position, table, out, nullptr, nullptr, p.a, p.g);                 \
-  }
-FK_PREFILL_ATTEND_PAGED_F16(1)
-FK_PREFILL_ATTEND_PAGED_F16(2)
-FK_PREFILL_ATTEND_PAGED_F16(4)
-

@@ -9,3 +9,4 @@
 #include "fk_prefill.h"
 #include "fk_rows_attend.h"
 #include "fk_skinny.h"
+#include "fk_split_attend.h"

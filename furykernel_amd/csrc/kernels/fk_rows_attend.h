@@ -258,7 +258,7 @@ __device__ __forceinline__ void rows_attend(const uint16_t *__restrict__ qr, con
   }
 }
 
-extern "C" __global__ void __launch_bounds__(64 * FK_ROWS_WAVES)
+extern "C" __global__ void __launch_bounds__(64 * FK_ROWS_WAVES, 2)
     fk_rows_attend_f16(const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc,
                        const uint16_t *__restrict__ vc, const uint32_t *__restrict__ position,
                        const uint32_t *__restrict__ slot, uint16_t *__restrict__ out, float *__restrict__ partials,
@@ -266,7 +266,7 @@ extern "C" __global__ void __launch_bounds__(64 * FK_ROWS_WAVES)
   rows_attend<false>(qr, kc, vc, position, slot, out, partials, p);
 }
 
-extern "C" __global__ void __launch_bounds__(64 * FK_ROWS_WAVES)
+extern "C" __global__ void __launch_bounds__(64 * FK_ROWS_WAVES, 2)
     fk_rows_attend_bf16(const uint16_t *__restrict__ qr, const uint16_t *__restrict__ kc,
                         const uint16_t *__restrict__ vc, const uint32_t *__restrict__ position,
                         const uint32_t *__restrict__ slot, uint16_t *__restrict__ out, float *__restrict__ partials,

@@ -53,8 +53,7 @@ _STRUCTS = {
     "fk_gemm_f16_silu_mul": K.GemmParams,
     "fk_gemm_f16_qkv_rope": K.GemmQkvParams,
     "fk_gemm_f16_qkv_rope_paged": K.GemmQkvPagedParams,
-    **{f"{form}{g}": K.PrefillAttendPagedParams for form in ("fk_prefill_attend_paged_g", "fk_prefill_attend_paged_f16_g")
-       for g in (1, 2, 4)},
+    **{e: K.PrefillAttendPagedParams if "_paged_" in e else K.PrefillAttendParams for e in K.ATTEND_FORMS},
     **{e: K.SkinnyParams for e in K.ABIS if e.startswith("fk_skinny_")},
     **{e: K.RowsAttendParams for e in ("fk_rows_attend_f16", "fk_rows_attend_bf16", "fk_rows_combine")},
     "fk_prefill_gather": K.PrefillGatherParams,
@@ -62,8 +61,6 @@ _STRUCTS = {
     **{f"fk_prefill_norm_pack_w{w}": K.PrefillNormParams for w in K.NORM_PACK_HELD},
     "fk_prefill_rope_store": K.PrefillRopeParams,
     "fk_prefill_rope_store_paged": K.PrefillRopePagedParams,
-    **{f"{form}{g}": K.PrefillAttendParams for form in ("fk_prefill_attend_g", "fk_prefill_attend_f16_g")
-       for g in (1, 2, 4)},
     "fk_prefill_argmax": K.PrefillArgmaxParams,
     "fk_prefill_argmax_keys": K.PrefillArgmaxKeysParams,
     "fk_prefill_land": K.PrefillLandParams,

@@ -364,6 +364,49 @@ ROWS_TILE = 256
 # multiples of it.
 ATTEND_KEYS = 64
 
+# The prefill attention's forms with a block's keys split among groups of
+# wavefronts (fk_attend.h): heads (wavefronts) a group, groups.
+ATTEND_SPLITS = ((4, 2), (2, 2), (1, 2), (2, 4), (1, 4))
+# Entry -> threads: rings and paged pools, staged through registers or (f16)
+# loaded straight into LDS, by the heads a kv head or split.
+ATTEND_FORMS = {f"fk_prefill_attend_{form}g{g}": 64 * g for form in ("", "f16_", "paged_", "paged_f16_")
+                for g in (1, 2, 4)}
+ATTEND_FORMS.update({f"fk_split_attend_{form}h{h}k{k}": 64 * h * k for form in ("", "f16_", "paged_", "paged_f16_")
+                     for h, k in ATTEND_SPLITS})
+
+
+def attend_launch(form: str, rows: int, heads: int, kv_heads: int, keys: int) -> tuple[str, int, int]:
+    """The entry, threadgroups and threads of the prefill attention of `rows`
+    rows ("", "f16_", "paged_", "paged_f16_": where its keys come from), the
+    rows' positions below `keys`.
+
+    A wavefront takes a block of 32 rows and a query head and walks the
+    block's keys, 64 at a time; few such pairs leave SIMDs idle (1024 on the
+    chip, and up to four wavefronts a SIMD to hide a block's latency), so
+    below 2560 their keys are split among groups of wavefronts
+    (fk_split_attend_*): in two, below 768 in four (all the LDS of a CU); and
+    below 1280 the heads of a kv head go to threadgroups of their own, for
+    256 or more.  MI355X, f16, 8 kv heads of 4, µs unsplit and split:
+
+    - 256 rows from position 3000 (256 pairs): 48.0, h1k4 22.9, h4k2 36.4;
+    - 512 from 3072: 52.1, h2k4 25.9, h1k4 43.2; from 0: 11.0, h2k4 8.7;
+    - 1024 from 0: 18.5, h2k2 13.6, h4k2 15.8; from 3072: 59.5, 46.9, 46.7;
+    - 2048 from 0 (2048 pairs): 36.6, h4k2 31.3, h2k2 34.7;
+    - 2 x 1536 (3072 pairs): 32.0, h4k2 33.5.
+
+    Fewer than eight blocks of keys stay: their merge would cost what the
+    split saves (256 rows from 0: 7.8, at best 6.7).  The rule is the same
+    for every place that the keys come from, so that staged, paged and ring
+    steps of one shape agree bit for bit."""
+    g = heads // kv_heads
+    pairs = rows // 32 * heads
+    if pairs >= 2560 or keys < 8 * ATTEND_KEYS:
+        return f"fk_prefill_attend_{form}g{g}", rows // 32 * kv_heads, 64 * g
+    h = g if pairs >= 1280 else min(g, 2) if pairs >= 512 else 1
+    k = 2 if pairs >= 768 else 4
+    return f"fk_split_attend_{form}h{h}k{k}", pairs // h, 64 * h * k
+
+
 # Row widths the one-pass RMSNorm-to-tiles holds in registers (fk_prefill.h).
 NORM_PACK_HELD = (512, 1024, 2048, 4096)
 
@@ -398,12 +441,10 @@ ABIS: dict[str, KernelAbi] = {
                                              PrefillRopePagedParams),
     "fk_prefill_rope_store": KernelAbi("fk_prefill_rope_store", ("q", "k", "v", "position", "slot", "rope", "qr",
                                                                  "kc", "vc"), PrefillRopeParams),
-    **{f"{form}{g}": KernelAbi(f"{form}{g}", ("qr", "kc", "vc", "position", "slot", "out", "ks", "vs"),
-                               PrefillAttendParams, 64 * g)
-       for form in ("fk_prefill_attend_g", "fk_prefill_attend_f16_g") for g in (1, 2, 4)},
-    **{f"{form}{g}": KernelAbi(f"{form}{g}", ("qr", "kc", "vc", "position", "table", "out"),
-                               PrefillAttendPagedParams, 64 * g)
-       for form in ("fk_prefill_attend_paged_g", "fk_prefill_attend_paged_f16_g") for g in (1, 2, 4)},
+    **{e: KernelAbi(e, ("qr", "kc", "vc", "position", "slot", "out", "ks", "vs"), PrefillAttendParams, threads)
+       for e, threads in ATTEND_FORMS.items() if "_paged_" not in e},
+    **{e: KernelAbi(e, ("qr", "kc", "vc", "position", "table", "out"), PrefillAttendPagedParams, threads)
+       for e, threads in ATTEND_FORMS.items() if "_paged_" in e},
     "fk_prefill_land": KernelAbi("fk_prefill_land", ("ks", "vs", "position", "slot", "kc", "vc"),
                                  PrefillLandParams, 256),
     "fk_prefill_argmax": KernelAbi("fk_prefill_argmax", ("x", "out"), PrefillArgmaxParams, 256),
@@ -620,7 +661,8 @@ class Kernels:
         one below 2^-24 flushes to zero, so bf16 caches are for values inside
         f16's range, as the prefill's own stores of f16-range rows are."""
         g = heads // kv_heads if kv_heads and heads % kv_heads == 0 else 0
-        entry = f"fk_prefill_attend_{'g' if cache_bf16 else 'f16_g'}{g}"
+        form = "" if cache_bf16 else "f16_"
+        entry = f"fk_prefill_attend_{form}g{g}"
         if rows <= 0 or rows % 256 or kv_heads <= 0 or heads % kv_heads or heads // kv_heads not in (1, 2, 4):
             raise LaunchError(f"{entry}: {rows} rows, {heads} heads over {kv_heads}")
         if length <= 0 or length % ATTEND_KEYS:
@@ -638,7 +680,8 @@ class Kernels:
         _need(out, rows * heads * 64 * 2, "out", entry)
         bound = {"qr": qr.ptr, "kc": kc.ptr, "vc": vc.ptr, "position": position.ptr, "slot": slot.ptr, "out": out.ptr,
                  "ks": 0, "vs": 0}
-        self.launch(entry, (rows // 32) * kv_heads, 64 * (heads // kv_heads), bound,
+        entry, groups, threads = attend_launch(form, rows, heads, kv_heads, length)
+        self.launch(entry, groups, threads, bound,
                     PrefillAttendParams(rows, heads, kv_heads, length, slots, window, int(cache_bf16), scale), stream)
 
     def rmsnorm(self, x: runtime.Buffer, gamma: runtime.Buffer | None, y: runtime.Buffer, rows: int, width: int,
@@ -805,6 +848,6 @@ def launch_reads(entry: str, params: dict) -> set[str]:
         return need | {"add": {"r0"}, "store_keys": {"keys"}}.get(mode, set())
     if entry == "fk_rmsnorm_f32" or entry.startswith("fk_prefill_norm_pack"):
         return set(abi.buffers) - ({"gamma"} if not params.get("has_gamma") else set())
-    if entry.startswith(("fk_prefill_attend_g", "fk_prefill_attend_f16_g")):
+    if entry in ATTEND_FORMS and "_paged_" not in entry:
         return set(abi.buffers) - (set() if params.get("staged") else {"ks", "vs"})
     return set(abi.buffers)

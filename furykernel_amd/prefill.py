@@ -46,7 +46,8 @@ from typing import Optional
 
 import numpy as np
 
-from .kernels import ATTEND_KEYS, NORM_PACK_HELD, ROWS_TILE, SKINNY_FORMS, SKINNY_PAIR_MODES
+from .kernels import (ATTEND_FORMS, ATTEND_KEYS, NORM_PACK_HELD, ROWS_TILE, SKINNY_FORMS, SKINNY_PAIR_MODES,
+                      attend_launch)
 from .layout import SLAB, pack, pair
 from .lower import ACT, BufferSpec, Launch, Lowered, LoweringError, rope_table
 from .program.check import CheckedProgram
@@ -72,6 +73,7 @@ class LiveRows:
     run: int
     apart: int = 1
     count: Optional[int] = None  # the rows themselves, where the last chunk is not whole
+    keys: Optional[int] = None   # their positions are below it, where that is known
 
 
 def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Optional[int] = None,
@@ -97,6 +99,7 @@ def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Opti
     live = live or LiveRows(rows // 16, rows // 16, rows)
     _skinny_gemms(out, live)
     _row_attention(out, live)
+    _split_attention(out, live)
     return out
 
 
@@ -124,7 +127,7 @@ def _row_attention(out: Lowered, live: LiveRows) -> None:
     launches = []
     for at in out.launches:
         p = at.params
-        if not at.entry.startswith(("fk_prefill_attend_g", "fk_prefill_attend_f16_g")) or p["staged"]:
+        if at.entry not in ATTEND_FORMS or "_paged_" in at.entry or p["staged"]:
             launches.append(at)
             continue
         pairs = live.count * p["kv_heads"]
@@ -141,6 +144,17 @@ def _row_attention(out: Lowered, live: LiveRows) -> None:
             launches.append(Launch(at.step, "fk_rows_combine", pairs, 64 * (p["heads"] // p["kv_heads"]),
                                    {b: bind[b] for b in ("partials", "position", "out")}, dict(params)))
     out.launches[:] = launches
+
+
+def _split_attention(out: Lowered, live: LiveRows) -> None:
+    """Each prefill attention as the form that fills the chip
+    (kernels.attend_launch)."""
+    for at in out.launches:
+        if at.entry in ATTEND_FORMS:
+            p = at.params
+            form = at.entry[len("fk_prefill_attend_"):at.entry.rindex("g")]
+            at.entry, at.groups, at.threads = attend_launch(form, p["rows"], p["heads"], p["kv_heads"],
+                                                            min(live.keys or p["length"], p["length"]))
 
 
 # What a tile of each form of fk_skinny costs a CU: µs a tile and a step of 32
@@ -904,7 +918,7 @@ class PrefillSession(_RowsSession):
                                rope_rotated=rope_rotated, paging=paging)
         chunks = -(-seq_rows // 16)
         self._setup(device, kernels, dims, program, seq_rows, rows, run, positions, slots, real, pad,
-                    LiveRows(seqs * chunks, chunks, run), paging, rows_tables)
+                    LiveRows(seqs * chunks, chunks, run, keys=run), paging, rows_tables)
         if paging is not None:
             self.tables = tables
 

@@ -25,7 +25,7 @@ def lowered(dims, seqs, seq_rows, decode=False, bound=None, **kw):
     else:
         rows, run, _, _, real = prefill_placement(seqs, seq_rows, dims.slots)
         chunks, at = -(-seq_rows // 16), seq_rows
-        live = LiveRows(seqs * chunks, chunks, run)
+        live = LiveRows(seqs * chunks, chunks, run, keys=run)
     c = check_program(decoder_step(dims, layers=1, position_bound=bound or (dims.context if decode else seq_rows), **kw))
     return lower_prefill(c, plan(PlanOptions(sequence_rows=at), c), rows, run, True, live), real, rows
 
@@ -93,9 +93,16 @@ def test_a_batchs_attention_splits_its_keys(rows, context, parts):
     assert not any(e.startswith("fk_prefill_attend") for e in entries)
 
 
-def test_a_prefills_attention_stays():
-    low, _, _ = lowered(ONE_B, 3, 9)
-    assert [L.entry for L in low.launches].count("fk_prefill_attend_f16_g4") == 1
+@pytest.mark.parametrize("seqs,seq_rows,kw,entry", [
+    (3, 9, {}, "fk_prefill_attend_f16_g4"), (1, 500, {}, "fk_split_attend_f16_h2k4"),
+    (2, 700, {}, "fk_split_attend_f16_h4k2"), (2, 700, {"paging": (64, 128)}, "fk_split_attend_paged_f16_h4k2"),
+    (1, 512, {"bound": 4096}, "fk_split_attend_h2k4"), (4, 2048, {}, "fk_prefill_attend_f16_g4")])
+def test_a_prefills_attention_splits_its_keys_where_its_blocks_are_few(seqs, seq_rows, kw, entry):
+    low, _, rows = lowered(ONE_B, seqs, seq_rows, **kw)
+    at = [L for L in low.launches if L.entry in K.ATTEND_FORMS]
+    assert [L.entry for L in at] == [entry]
+    h = int(entry[entry.rindex("h") + 1]) if "split" in entry else 4
+    assert at[0].groups == rows // 32 * 32 // h and at[0].threads == K.ATTEND_FORMS[entry]
 
 
 def test_forms_by_size():
