@@ -15,6 +15,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <deque>
 #include <string>
@@ -133,7 +134,10 @@ AttendEntry attend_entry(const char *entry) {
   return a;
 }
 
-const char *const skinny_modes[] = {"store", "add", "store_keys", "silu_mul", "qkv_rope", "qkv_rope_paged"};
+// Threads of fk_rows_norm_w<width>.
+uint32_t rows_norm_threads(uint32_t width) { return width / 8 < 256 ? width / 8 : 256; }
+
+const char *const skinny_modes[] = {"store", "add", "part", "store_keys", "silu_mul", "qkv_rope", "qkv_rope_paged"};
 
 bool skinny_pairs(const char *mode) {
   return std::strcmp(mode, "silu_mul") == 0 || std::strncmp(mode, "qkv_rope", 8) == 0;
@@ -348,6 +352,7 @@ std::vector<Entry> build() {
       using S = fk_skinny_params;
       std::vector<fk_abi_param> p = gemm_params();
       p.insert(p.end(), {FK_P(S, live, "u32"), FK_P(S, run_chunks, "u32"), FK_P(S, run, "u32"), FK_P(S, apart, "u32"),
+                         FK_P(S, compact, "u32"), FK_P(S, parts, "u32"),
                          FK_PX(S, r.kv_heads, "kv_heads", "u32"), FK_PX(S, r.rope_rows, "rope_rows", "u32"),
                          FK_PX(S, r.length, "length", "u32"), FK_PX(S, r.slots, "slots", "u32"),
                          FK_PX(S, r.cache_bf16, "cache_bf16", "u32"), FK_PX(S, r.staged, "staged", "u32"),
@@ -365,7 +370,8 @@ std::vector<Entry> build() {
     using S = fk_rows_attend_params;
     const std::vector<fk_abi_param> p = {FK_P(S, rows, "u32"),   FK_P(S, apart, "u32"),  FK_P(S, heads, "u32"),
                                          FK_P(S, kv_heads, "u32"), FK_P(S, length, "u32"), FK_P(S, slots, "u32"),
-                                         FK_P(S, window, "u32"), FK_P(S, parts, "u32"),  FK_P(S, scale, "f32")};
+                                         FK_P(S, window, "u32"), FK_P(S, parts, "u32"),  FK_P(S, compact, "u32"),
+                                         FK_P(S, scale, "f32")};
     for (const char *t : {"f16", "bf16"})
       add(std::string("fk_rows_attend_") + t, 256,
           {buf("qr", "read", "f16"), buf("kc", "read", t), buf("vc", "read", t), buf("position", "read", "u32"),
@@ -373,6 +379,27 @@ std::vector<Entry> build() {
           p, sizeof(S));
     add("fk_rows_combine", 0, {buf("partials", "read", "f32"), buf("position", "read", "u32"), buf("out", "write", "f16")},
         p, sizeof(S));
+  }
+  {
+    using S = fk_rows_norm_params;
+    const std::vector<fk_abi_param> p = {
+        FK_P(S, m, "u32"),       FK_P(S, width, "u32"),     FK_P(S, live, "u32"),   FK_P(S, run_chunks, "u32"),
+        FK_P(S, run, "u32"),     FK_P(S, apart, "u32"),     FK_P(S, compact, "u32"), FK_P(S, eps, "f32"),
+        FK_P(S, factor, "f32"),  FK_P(S, has_gamma, "u32"), FK_P(S, source, "u32"), FK_P(S, table_rows, "u32"),
+        FK_P(S, gfactor, "f32"), FK_P(S, parts, "u32")};
+    for (uint32_t w : {512u, 1024u, 2048u, 4096u})
+      add("fk_rows_norm_w" + std::to_string(w), rows_norm_threads(w),
+          {buf("x", "read", "f32"), buf("table", "read", "f16"), buf("tokens", "read", "u32"),
+           buf("partials", "read", "f32"), buf("gamma", "read", "f32"), buf("xout", "write", "f32"),
+           buf("y", "write", "f16")},
+          p, sizeof(S));
+  }
+  {
+    using S = fk_rows_token_params;
+    add("fk_rows_token", 256, {buf("keys", "read", "u64"), buf("out", "write", "u32")},
+        {FK_P(S, m, "u32"), FK_P(S, live, "u32"), FK_P(S, run_chunks, "u32"), FK_P(S, run, "u32"),
+         FK_P(S, apart, "u32"), FK_P(S, parts, "u32")},
+        sizeof(S));
   }
   {
     using S = fk_prefill_gather_params;
@@ -869,6 +896,33 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
       for (Need &n : need)
         if (std::strcmp(n.name, "c1") == 0 || std::strcmp(n.name, "c2") == 0) n.bytes = pool;
     }
+  } else if (std::strncmp(entry, "fk_rows_norm", 12) == 0) {
+    fk_rows_norm_params p;
+    std::memcpy(&p, params, sizeof p);
+    const bool gather = p.source == FK_ROWS_GATHER_F16 || p.source == FK_ROWS_GATHER_F32;
+    if (p.m == 0 || p.m % 256 || p.width != (uint32_t)std::strtoul(entry + 14, nullptr, 10) || p.live == 0 ||
+        p.run_chunks == 0 || p.apart == 0 || (p.compact && (uint64_t)p.live * 16 > p.m) || p.source > FK_ROWS_PARTS ||
+        (gather && p.table_rows == 0) || (p.source == FK_ROWS_PARTS && p.parts == 0) || groups != p.live * 16)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u chunks of rows of %u in a step of %u, source %u, %u threadgroups", entry,
+                 p.live, p.width, p.m, p.source, groups);
+    const uint64_t row = (uint64_t)p.m * p.width;
+    need = {{"y", row * 2}};
+    if (p.has_gamma) need.push_back({"gamma", (uint64_t)p.width * 4});
+    if (p.source != FK_ROWS_STORED) need.push_back({"xout", row * 4});
+    if (gather) {
+      need.push_back({"table", (uint64_t)p.table_rows * p.width * (p.source == FK_ROWS_GATHER_F16 ? 2 : 4)});
+      need.push_back({"tokens", (uint64_t)p.m * 4});
+    } else {
+      need.push_back({"x", row * 4});
+    }
+    if (p.source == FK_ROWS_PARTS) need.push_back({"partials", (uint64_t)p.parts * p.live * 16 * p.width * 4});
+  } else if (std::strcmp(entry, "fk_rows_token") == 0) {
+    fk_rows_token_params p;
+    std::memcpy(&p, params, sizeof p);
+    if (p.m == 0 || p.live == 0 || p.run_chunks == 0 || p.apart == 0 || p.parts == 0 || groups != p.live * 16)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u chunks of rows of %u keys, %u threadgroups", entry, p.live, p.parts,
+                 groups);
+    need = {{"keys", (uint64_t)p.m * p.parts * 8}, {"out", (uint64_t)p.m * 4}};
   } else if (std::strncmp(entry, "fk_rows_attend", 14) == 0 || std::strcmp(entry, "fk_rows_combine") == 0) {
     fk_rows_attend_params p;
     std::memcpy(&p, params, sizeof p);
@@ -902,7 +956,7 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
     const fk_gemm_params &g = p.g;
     const uint32_t cols = g.n_anchors >= 1 && g.n_anchors <= 3 ? g.first_col[g.n_anchors] : 0;
     bool shape = f && g.m && g.m % 256 == 0 && g.k && g.k % 64 == 0 && cols && p.live && p.run_chunks && p.apart &&
-                 (uint64_t)g.m * g.k * 2 < 0xfffffff0u && (silu ? g.n_anchors == 1 && g.ldc[0] == cols && cols % 128 == 0
+                 (!p.compact || (uint64_t)p.live * 16 <= g.m) && (uint64_t)g.m * g.k * 2 < 0xfffffff0u && (silu ? g.n_anchors == 1 && g.ldc[0] == cols && cols % 128 == 0
                                                                 : g.first_col[0] == 0);
     for (uint32_t j = 0; shape && !silu && j < g.n_anchors; j++)
       shape = g.first_col[j + 1] > g.first_col[j] && (g.first_col[j + 1] - g.first_col[j]) % 256 == 0 &&
@@ -910,7 +964,9 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
     // SiLU·mul: the pair's 2 cols weight rows.
     const uint64_t tiles_n = shape ? (uint64_t)(silu ? 2 * cols : cols) / (16 * f->nb) : 0;
     const uint64_t tiles_m = shape ? ((uint64_t)p.live + f->mb - 1) / f->mb : 0;
-    if (!shape || (uint64_t)groups != (tiles_n + 7) / 8 * 8 * tiles_m)
+    const uint64_t split = mode == "part" ? p.parts : 1;
+    if (mode == "part" && (p.parts == 0 || g.n_anchors != 1)) shape = false;
+    if (!shape || (uint64_t)groups != (tiles_n + 7) / 8 * 8 * tiles_m * split)
       return bad(err, cap, FK_ERR_ARG, "%s: %u rows, k %u, %u anchors over %u columns, %u chunks of rows in %u threadgroups",
                  entry, g.m, g.k, g.n_anchors, cols, p.live, groups);
     const uint64_t m = g.m;
@@ -919,7 +975,9 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
     for (uint32_t j = 0; j < g.n_anchors; j++) {
       const uint64_t wide = silu ? 2ull * cols : g.first_col[j + 1] - g.first_col[j];
       need.push_back({bn[j], wide * g.k * 2});
-      if (!qkv || j == 0) need.push_back({cn[j], m * g.ldc[j] * (silu || qkv ? 2 : 4)});
+      // (live chunks one after another: never past the step's rows, checked above)
+      const uint64_t rows = mode == "part" ? split * p.live * 16 : m;
+      if (!qkv || j == 0) need.push_back({cn[j], rows * g.ldc[j] * (silu || qkv ? 2 : 4)});
     }
     if (mode == "add") {
       if (g.n_anchors != 1) return bad(err, cap, FK_ERR_ARG, "%s: %u anchors", entry, g.n_anchors);

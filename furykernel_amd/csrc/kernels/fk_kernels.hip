@@ -8,5 +8,6 @@
 #include "fk_gemm.h"
 #include "fk_prefill.h"
 #include "fk_rows_attend.h"
+#include "fk_rows_norm.h"
 #include "fk_skinny.h"
 #include "fk_split_attend.h"

@@ -246,7 +246,7 @@ __device__ __forceinline__ void rows_attend(const uint16_t *__restrict__ qr, con
       oo += so[w][q][d] * f;
     }
     if (whole) {
-      out[fk::tile_offset(row, (g * G + q) * 64 + d, qw)] = fk::to_f16(oo / ll);
+      out[fk::tile_offset(p.compact ? i : row, (g * G + q) * 64 + d, qw)] = fk::to_f16(oo / ll);
     } else {
       float *const to = partials + (((size_t)(i * p.kv_heads + g) * p.parts + part) * G + q) * 66;
       to[d] = oo;
@@ -312,5 +312,5 @@ extern "C" __global__ void __launch_bounds__(1024)
     }
     mm = mn;
   }
-  out[fk::tile_offset(row, (g * G + q) * 64 + d, p.heads * 64)] = fk::to_f16(oo / ll);
+  out[fk::tile_offset(p.compact ? i : row, (g * G + q) * 64 + d, p.heads * 64)] = fk::to_f16(oo / ll);
 }

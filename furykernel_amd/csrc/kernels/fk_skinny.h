@@ -38,12 +38,18 @@
 //
 // The forms (MB, NB, W, D) and where each is taken: prefill.py's skinny_form.
 //
+// FK_GEMM_PART splits k among threadgroups too, for the residual projections
+// of up to 200 rows, whose tiles are too few to fill the chip: partial sums
+// that the norm after them adds (fk_rows_norm.h).
+//
 // Live rows: the rows that fill a step out to whole tiles (prefill.py) are
 // skipped.  Chunk c of the live rows is rows first + i · apart (i = 0 .. 15),
 // first = (c / run_chunks) · run + (c mod run_chunks) · 16 · apart: the
 // leading rows of each run of a prefill (apart 1), or a decode step's rows,
-// one a query block (apart 32, one run).  A chunk's rows past g.m read zeros
-// and store nothing.
+// one a query block (apart 32, one run; the tiled matrices between its
+// kernels then hold the live chunks alone, `compact`: read at their spaced
+// rows, 64 bytes each, the down projection of 41 rows took 20 µs against
+// 15.5).  A chunk's rows past g.m read zeros and store nothing.
 #pragma once
 
 #include "fk_common.h"
@@ -91,8 +97,11 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
   const uint32_t cols = MODE == FK_GEMM_SILU_MUL ? 2 * p.g.ldc[0] : p.g.first_col[p.g.n_anchors];
   const uint32_t tiles_n = cols / (16 * NB);
   const uint32_t at = blockIdx.x / 8;
-  const uint32_t tn = (at / tiles_m) * 8 + blockIdx.x % 8;
   const uint32_t tm = at % tiles_m;
+  // (FK_GEMM_PART: the parts of a tile follow its tiles of rows)
+  const uint32_t parts = MODE == FK_GEMM_PART ? p.parts : 1u;
+  const uint32_t part = MODE == FK_GEMM_PART ? at / tiles_m % parts : 0u;
+  const uint32_t tn = (at / (tiles_m * parts)) * 8 + blockIdx.x % 8;
   if (tn >= tiles_n) return;
 
   // The weights' chunks (16 rows) of the tile's column blocks, one 256-row
@@ -137,9 +146,10 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
   uint32_t av[MB];
 #pragma unroll
   for (int i = 0; i < MB; i++) {
-    const uint32_t row = row_of(i, lane / 4);
-    const uint32_t rr = row % 16;
     // past the rows: past the buffer, where loads read zeros
+    const uint32_t c = tm * MB + i;
+    const uint32_t row = p.compact ? (c < p.live ? c * 16 + lane / 4 : 0xffffffffu) : row_of(i, lane / 4);
+    const uint32_t rr = row % 16;
     av[i] = row < p.g.m ? (row / 256) * (256 * k * 2) + (row % 256 / 16) * 1024 +
                               (rr * 4 + ((lane % 4) ^ fk::tile_swizzle(lane / 4) ^ fk::tile_swizzle(rr))) * 16
                         : 0xfffffff0u;
@@ -177,12 +187,14 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
 #pragma unroll
     for (int j = 0; j < NB; j++) acc[i][j] = fk_float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
-  const uint32_t count = wave < steps ? (steps - wave + W - 1) / W : 0;  // this wavefront's steps
+  // This wavefront's steps: first, first + stride, ...
+  const uint32_t first = part * W + wave, stride = parts * W;
+  const uint32_t count = first < steps ? (steps - first + stride - 1) / stride : 0;
   // Slot S: step X of this wavefront's.  Steps past the last repeat it, so
   // that every wait counts the same loads; they are never multiplied.
 #define FK_SKINNY_LOAD(S, X)                                                                                    \
   do {                                                                                                          \
-    const uint32_t at_ = min(wave + (uint32_t)(X) * W, steps - 1) * 16384;                                      \
+    const uint32_t at_ = min(first + (uint32_t)(X) * stride, steps - 1) * 16384;                                   \
     FK_LDS char *d_ = ring + (S) * (CH * 1024);                                                                 \
     _Pragma("unroll") for (int j_ = 0; j_ < NB; j_++)                                                           \
       __builtin_amdgcn_raw_ptr_buffer_load_lds(bsrc, d_ + j_ * 1024, 16, bv + chunk_of(j_) * 1024, at_, 0, HINT); \
@@ -307,7 +319,8 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
 #pragma unroll
         for (int r = 0; r < 4; r++)
           h[r] = fk::to_f16((p.g.act == FK_ACT_GELU_TANH ? fk::act_hw<true>(g[r]) : fk::act_hw<false>(g[r])) * up[r]);
-        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(c0) + fk::tile_offset(row, col, ld)) =
+        *reinterpret_cast<uint2 *>(reinterpret_cast<uint16_t *>(c0) +
+                                   fk::tile_offset(p.compact ? (tm * MB + round * MR + u / NU) * 16 + lane_e % 16 : row, col, ld)) =
             make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
       } else if constexpr (QKV) {
         // The unit's columns d .. d + 3 of its head, and their partners d + 32 ..
@@ -348,7 +361,13 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
 #pragma unroll
         for (int q = 0; q < U; q++) {
           fk_float4v v = total(q);
-          if (row < p.g.m) {
+          if (MODE == FK_GEMM_PART) {
+            // [parts][live 16][ld]: every row of a live chunk, the rows past
+            // the step's zeros
+            const uint32_t c = tm * MB + round * MR + u / NU;
+            if (c < p.live)
+              *reinterpret_cast<fk_float4v *>(out + ((size_t)part * p.live * 16 + c * 16 + lane_e % 16) * ld + col) = v;
+          } else if (row < p.g.m) {
             if (MODE == FK_GEMM_ADD) v = with[round][it][0] + v;
             *reinterpret_cast<fk_float4v *>(out + (size_t)row * ld + col + 16 * q) = v;
           }
@@ -391,6 +410,7 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
 // S: the ring's steps in the modes that stream many tiles (gate and up, the
 // logits), D in the rest.
 #define FK_SKINNY_FORM(FORM, MB, NB, W, D, S)                                   \
+  FK_SKINNY_ENTRY(fk_skinny_part_##FORM, FK_GEMM_PART, MB, NB, W, D)            \
   FK_SKINNY_ENTRY(fk_skinny_store_##FORM, FK_GEMM_STORE, MB, NB, W, D)          \
   FK_SKINNY_ENTRY(fk_skinny_add_##FORM, FK_GEMM_ADD, MB, NB, W, D)              \
   FK_SKINNY_ENTRY(fk_skinny_store_keys_##FORM, FK_GEMM_STORE_KEYS, MB, NB, W, S)

@@ -56,6 +56,8 @@ _STRUCTS = {
     **{e: K.PrefillAttendPagedParams if "_paged_" in e else K.PrefillAttendParams for e in K.ATTEND_FORMS},
     **{e: K.SkinnyParams for e in K.ABIS if e.startswith("fk_skinny_")},
     **{e: K.RowsAttendParams for e in ("fk_rows_attend_f16", "fk_rows_attend_bf16", "fk_rows_combine")},
+    **{f"fk_rows_norm_w{w}": K.RowsNormParams for w in K.ROWS_NORM_THREADS},
+    "fk_rows_token": K.RowsTokenParams,
     "fk_prefill_gather": K.PrefillGatherParams,
     "fk_prefill_norm_pack": K.PrefillNormParams,
     **{f"fk_prefill_norm_pack_w{w}": K.PrefillNormParams for w in K.NORM_PACK_HELD},

@@ -109,7 +109,8 @@ class SkinnyParams(ctypes.Structure):
     """fk_skinny_params: the GEMM's, the rows it makes, then the QKV
     epilogue's RoPE, caches and paging."""
     _fields_ = GemmParams._fields_ + [("live", ctypes.c_uint32), ("run_chunks", ctypes.c_uint32),
-                                      ("run", ctypes.c_uint32), ("apart", ctypes.c_uint32)] + \
+                                      ("run", ctypes.c_uint32), ("apart", ctypes.c_uint32),
+                                      ("compact", ctypes.c_uint32), ("parts", ctypes.c_uint32)] + \
         GemmQkvParams._fields_[len(GemmParams._fields_):] + \
         [("block_size", ctypes.c_uint32), ("table_len", ctypes.c_uint32), ("blocks", ctypes.c_uint32)]
 
@@ -118,7 +119,20 @@ class RowsAttendParams(ctypes.Structure):
     """fk_rows_attend_params: the attention of rows each a sequence's one."""
     _fields_ = [("rows", ctypes.c_uint32), ("apart", ctypes.c_uint32), ("heads", ctypes.c_uint32),
                 ("kv_heads", ctypes.c_uint32), ("length", ctypes.c_uint32), ("slots", ctypes.c_uint32),
-                ("window", ctypes.c_uint32), ("parts", ctypes.c_uint32), ("scale", ctypes.c_float)]
+                ("window", ctypes.c_uint32), ("parts", ctypes.c_uint32), ("compact", ctypes.c_uint32),
+                ("scale", ctypes.c_float)]
+
+
+class RowsNormParams(ctypes.Structure):
+    """fk_rows_norm_params: the live rows made (`source`), stored and normed."""
+    _fields_ = [(f, ctypes.c_uint32) for f in ("m", "width", "live", "run_chunks", "run", "apart", "compact")] + \
+        [("eps", ctypes.c_float), ("factor", ctypes.c_float), ("has_gamma", ctypes.c_uint32),
+         ("source", ctypes.c_uint32), ("table_rows", ctypes.c_uint32), ("gfactor", ctypes.c_float),
+         ("parts", ctypes.c_uint32)]
+
+
+class RowsTokenParams(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_uint32) for f in ("m", "live", "run_chunks", "run", "apart", "parts")]
 
 
 class PrefillGatherParams(ctypes.Structure):
@@ -345,7 +359,7 @@ STEP_GEMV_BUFFERS = ("w0", "w1", "w2", "y0", "y1", "y2", "src", "src2", "gamma",
 SKINNY_FORMS = {"m1n1": (1, 1, 8), "m1n2": (1, 2, 8), "m2n1": (2, 1, 8), "m2n2": (2, 2, 8), "m2n4": (2, 4, 4),
                 "m4n2": (4, 2, 8), "m4n4": (4, 4, 4), "m4n8": (4, 8, 4), "m8n4": (8, 4, 4), "m8n8": (8, 8, 4)}
 SKINNY_PAIR_MODES = ("silu_mul", "qkv_rope", "qkv_rope_paged")
-SKINNY_MODES = ("store", "add", "store_keys") + SKINNY_PAIR_MODES
+SKINNY_MODES = ("store", "add", "part", "store_keys") + SKINNY_PAIR_MODES
 SKINNY_BUFFERS = ("a", "b0", "b1", "b2", "c0", "c1", "c2", "r0", "position", "slot", "rope", "keys")
 _SKINNY = re.compile(r"^fk_skinny_(\w+)_(m\dn\d)$")
 
@@ -355,6 +369,11 @@ def skinny_entry(entry: str) -> tuple[str, tuple]:
     m = _SKINNY.match(entry)
     return m.group(1), SKINNY_FORMS[m.group(2)]
 
+
+# What makes a row that fk_rows_norm norms (fk_rows_norm.h); its threads by the
+# row's width.
+ROWS_STORED, ROWS_GATHER_F16, ROWS_GATHER_F32, ROWS_PARTS = range(4)
+ROWS_NORM_THREADS = {512: 64, 1024: 128, 2048: 256, 4096: 256}
 
 # Keys a threadgroup of the attention of a batch of rows takes at a time
 # (fk_rows_attend.h).
@@ -431,6 +450,9 @@ ABIS: dict[str, KernelAbi] = {
        if nb > 1 or mode not in SKINNY_PAIR_MODES},
     **{e: KernelAbi(e, ("qr", "kc", "vc", "position", "slot", "out", "partials"), RowsAttendParams, 256)
        for e in ("fk_rows_attend_f16", "fk_rows_attend_bf16")},
+    **{f"fk_rows_norm_w{w}": KernelAbi(f"fk_rows_norm_w{w}", ("x", "table", "tokens", "partials", "gamma", "xout", "y"),
+                                       RowsNormParams, t) for w, t in ROWS_NORM_THREADS.items()},
+    "fk_rows_token": KernelAbi("fk_rows_token", ("keys", "out"), RowsTokenParams, 256),
     "fk_rows_combine": KernelAbi("fk_rows_combine", ("partials", "position", "out"), RowsAttendParams),
     "fk_prefill_gather": KernelAbi("fk_prefill_gather", ("table", "tokens", "x"), PrefillGatherParams, 256),
     "fk_prefill_norm_pack": KernelAbi("fk_prefill_norm_pack", ("x", "gamma", "y"), PrefillNormParams, 256),
@@ -837,6 +859,14 @@ def launch_reads(entry: str, params: dict) -> set[str]:
         if entry == "fk_gemm_f16_store_keys":
             need.add("keys")
         return need
+    if entry.startswith("fk_rows_norm"):
+        source = params.get("source", ROWS_STORED)
+        need = {"y"} | ({"gamma"} if params.get("has_gamma") else set())
+        if source != ROWS_STORED:
+            need.add("xout")
+        if source in (ROWS_GATHER_F16, ROWS_GATHER_F32):
+            return need | {"table", "tokens"}
+        return need | {"x"} | ({"partials"} if source == ROWS_PARTS else set())
     if entry.startswith("fk_rows_attend"):
         return set(abi.buffers) - (set() if params.get("parts", 1) > 1 else {"partials"})
     if entry.startswith("fk_skinny_"):

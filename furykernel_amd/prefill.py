@@ -46,8 +46,8 @@ from typing import Optional
 
 import numpy as np
 
-from .kernels import (ATTEND_FORMS, ATTEND_KEYS, NORM_PACK_HELD, ROWS_TILE, SKINNY_FORMS, SKINNY_PAIR_MODES,
-                      attend_launch)
+from .kernels import (ATTEND_FORMS, ATTEND_KEYS, NORM_PACK_HELD, ROWS_GATHER_F16, ROWS_GATHER_F32, ROWS_NORM_THREADS,
+                      ROWS_PARTS, ROWS_STORED, ROWS_TILE, SKINNY_FORMS, SKINNY_PAIR_MODES, attend_launch)
 from .layout import SLAB, pack, pair
 from .lower import ACT, BufferSpec, Launch, Lowered, LoweringError, rope_table
 from .program.check import CheckedProgram
@@ -98,8 +98,10 @@ def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Opti
     _fuse_argmax(out)
     live = live or LiveRows(rows // 16, rows // 16, rows)
     _skinny_gemms(out, live)
+    _rows_norms(out, live)
     _row_attention(out, live)
     _split_attention(out, live)
+    _compact(out, live)
     return out
 
 
@@ -167,16 +169,19 @@ SKINNY_COST = {"m1n1": (1.1, 0.037, False), "m1n2": (1.4, 0.054, False), "m2n1":
                "m8n8": (11.5, 0.202, True)}
 
 
-def skinny_form(chunks: int, m: int, n: int, k: int, mode: str) -> Optional[str]:
+def skinny_form(chunks: int, m: int, n: int, k: int, mode: str, splits: tuple = (1,)) -> Optional[tuple]:
     """The form of fk_skinny that a GEMM of `chunks` live chunks of 16 rows
     (of a step of m) by n weight rows of k columns takes for the epilogue
-    `mode`, or None where the 256 × 256 tiles of fk_gemm are faster: the
-    least of
+    `mode` and the threadgroups its k is split among (one of `splits`; more
+    than one leaves partial sums), or None where the 256 × 256 tiles of
+    fk_gemm are faster: the least of
 
     - fk_gemm: its tiles in rounds of 256 (one a CU), 0.55 µs a step of 32
       columns and 11 a round, 17 with the residual's or QKV's epilogue (46
       and 52 at k 2048, 158 for down, whatever the rows);
-    - a form: 2 µs, and SKINNY_COST's for as many tiles as a CU takes.
+    - a form: 2 µs, and SKINNY_COST's for as many tiles as a CU takes, of a
+      split's share of the steps; and its partial sums' way to HBM and back
+      at 4 TB/s.
 
     So, measured: O and down (n 2048) of 1408 rows take m8n8's 176 tiles (26
     against 55, 65 against 160 at k 8192); gate and up (n 16384) of 208 rows
@@ -196,27 +201,40 @@ def skinny_form(chunks: int, m: int, n: int, k: int, mode: str) -> Optional[str]
         if mb >= 2 * chunks or (pairs and nb == 1):
             continue
         tile, step, one = SKINNY_COST[form]
-        share = -(-chunks // mb) * (n // (16 * nb)) / 256
-        share = max(1.0, float(np.ceil(share))) if one else (share + 0.25 if share > 1 else 1.0)
-        cost = 2 + share * (tile + steps * step)
-        if cost < least:
-            best, least = form, cost
+        for parts in splits:
+            share = -(-chunks // mb) * (n // (16 * nb)) * parts / 256
+            share = max(1.0, float(np.ceil(share))) if one else (share + 0.25 if share > 1 else 1.0)
+            cost = 2 + share * (tile + steps / parts * step)
+            if parts > 1:
+                cost += parts * chunks * 16 * n * 8 / 4e6
+            if cost < least:
+                best, least = (form, parts), cost
     return best
+
+
+def _reads(out: Lowered, i: int, name: str) -> Optional[int]:
+    """The first launch after i that binds buffer `name`."""
+    return next((j for j in range(i + 1, len(out.launches)) if name in out.launches[j].bind.values()), None)
 
 
 def _skinny_gemms(out: Lowered, live: LiveRows) -> None:
     """Each GEMM of too few live rows for fk_gemm's tiles, as the form of
     fk_skinny that ``skinny_form`` picks: the same epilogue on the live rows
-    alone."""
+    alone.  A residual's GEMM whose rows the next launch norms may leave partial
+    sums, which that norm (then ``fk_rows_norm``) adds to the residual."""
     for i, gm in enumerate(out.launches):
         if not gm.entry.startswith("fk_gemm_f16_"):
             continue
         p = gm.params
         mode = gm.entry[len("fk_gemm_f16_"):]
         n = 2 * p["ldc"][0] if mode == "silu_mul" else p["first_col"][p["n_anchors"]]
-        form = skinny_form(live.chunks, p["m"], n, p["k"], mode)
-        if form is None:
+        norm = out.launches[i + 1] if mode == "add" and i + 1 < len(out.launches) else None
+        if norm is not None and not (_rows_norm_of(norm, live) and norm.bind["x"] == gm.bind["c0"]):
+            norm = None
+        picked = skinny_form(live.chunks, p["m"], n, p["k"], mode, (1, 2, 4, 8) if norm else (1,))
+        if picked is None:
             continue
+        form, split = picked
         mb, nb, waves = SKINNY_FORMS[form]
         bind = dict(gm.bind)
         if "table" in bind:
@@ -228,10 +246,95 @@ def _skinny_gemms(out: Lowered, live: LiveRows) -> None:
             for am in out.launches:
                 if am.entry == "fk_prefill_argmax_keys" and am.bind["keys"] == bind["keys"]:
                     am.params["parts"] = parts
-        groups = -(-(n // (16 * nb)) // 8) * 8 * -(-live.chunks // mb)
+        if split > 1:
+            mode = "part"
+            # one buffer for every launch: the next one has read it
+            name = "skinny:partials"
+            count = max(split * live.chunks * 16 * n, out.buffers[name].count if name in out.buffers else 0)
+            out.buffers[name] = BufferSpec(name, "f32", count)
+            _to_rows_norm(norm, live, p["m"],
+                          {"x": bind["r0"], "xout": bind["c0"], "partials": name}, source=ROWS_PARTS, parts=split)
+            bind["r0"], bind["c0"] = None, name
+        groups = -(-(n // (16 * nb)) // 8) * 8 * -(-live.chunks // mb) * split
         out.launches[i] = Launch(gm.step, f"fk_skinny_{mode}_{form}", groups, 64 * waves, bind,
                                  dict(p, live=live.chunks, run_chunks=live.run_chunks, run=live.run,
-                                      apart=live.apart))
+                                      apart=live.apart, parts=split))
+
+
+# Live chunks up to which the kernels between the GEMMs take the live rows
+# alone (fk_rows_norm.h), a threadgroup a row: past 2,000 rows they are bound
+# by HBM, not by their latency, and the plain ones take four rows a
+# threadgroup.
+ROWS_NORM_CHUNKS = 128
+
+
+def _rows_norm_of(launch: Launch, live: LiveRows) -> bool:
+    """Whether fk_rows_norm can take the place of `launch`."""
+    return live.chunks <= ROWS_NORM_CHUNKS and launch.entry.startswith("fk_prefill_norm_pack_w") and \
+        launch.params["width"] in ROWS_NORM_THREADS
+
+
+def _to_rows_norm(norm: Launch, live: LiveRows, rows: int, bind: dict, **params) -> None:
+    """`norm` as fk_rows_norm on the live rows, which `bind` and `params`
+    say how to make."""
+    p = norm.params
+    norm.bind = {"x": None, "table": None, "tokens": None, "partials": None, "xout": None,
+                 "gamma": norm.bind["gamma"], "y": norm.bind["y"], **bind}
+    norm.entry = f"fk_rows_norm_w{p['width']}"
+    norm.groups, norm.threads = live.chunks * 16, ROWS_NORM_THREADS[p["width"]]
+    norm.params = dict({f: p[f] for f in ("width", "eps", "factor", "has_gamma")}, m=rows, live=live.chunks,
+                       run_chunks=live.run_chunks, run=live.run, apart=live.apart, **params)
+
+
+def _rows_norms(out: Lowered, live: LiveRows) -> None:
+    """The norms whose rows a fk_skinny GEMM reads, on the live rows alone
+    (``fk_rows_norm``), a gather right before one folded into it; and the
+    greedy token of those rows' keys (``fk_rows_token``)."""
+    gone = []
+    for i, norm in enumerate(out.launches):
+        if _rows_norm_of(norm, live):
+            reader = _reads(out, i, norm.bind["y"])
+            if reader is None or not out.launches[reader].entry.startswith("fk_skinny_"):
+                continue
+            x = norm.bind["x"]
+            before = next((j for j in range(i - 1, -1, -1) if x in out.launches[j].bind.values()), None)
+            made = out.launches[before] if before is not None else None
+            if before == i - 1 and made.entry == "fk_prefill_gather" and made.params["width"] == norm.params["width"]:
+                g = made.params
+                _to_rows_norm(norm, live, g["rows"], {"table": made.bind["table"], "tokens": made.bind["tokens"],
+                                                      "xout": x},
+                              source=ROWS_GATHER_F16 if g["table_f16"] else ROWS_GATHER_F32,
+                              table_rows=g["table_rows"], gfactor=g["factor"])
+                gone.append(before)
+            else:
+                _to_rows_norm(norm, live, norm.params["rows"], {"x": x}, source=ROWS_STORED)
+        elif norm.entry == "fk_prefill_argmax_keys" and live.chunks <= ROWS_NORM_CHUNKS:
+            made = next(L for L in reversed(out.launches[:i]) if L.bind.get("keys") == norm.bind["keys"])
+            if made.entry.startswith("fk_skinny_"):
+                norm.entry, norm.groups, norm.threads = "fk_rows_token", live.chunks * 16, 256
+                norm.params = dict(m=norm.params["rows"], parts=norm.params["parts"], live=live.chunks,
+                                   run_chunks=live.run_chunks, run=live.run, apart=live.apart)
+    out.launches[:] = [L for i, L in enumerate(out.launches) if i not in gone]
+
+
+def _compact(out: Lowered, live: LiveRows) -> None:
+    """Where the live rows lie apart (a decode step's, one a query block), the
+    tiled values between their kernels hold them one after another, if every
+    launch that touches those values can."""
+    if live.apart == 1:
+        return
+    tiled, takes = set(), []
+    for L in out.launches:
+        if L.entry.startswith("fk_skinny_"):
+            takes.append(L)
+            tiled |= {L.bind["a"]} | ({L.bind["c0"]} if "_silu_mul_" in L.entry else set())
+        elif L.entry.startswith(("fk_rows_norm", "fk_rows_attend", "fk_rows_combine")):
+            takes.append(L)
+            tiled.add(L.bind["y" if "norm" in L.entry else "out"])
+    if any(tiled & set(L.bind.values()) for L in out.launches if not any(L is t for t in takes)):
+        return
+    for L in takes:
+        L.params["compact"] = 1
 
 
 def _fuse_argmax(out: Lowered) -> None:

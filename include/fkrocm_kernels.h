@@ -305,7 +305,8 @@ enum {
                            the V cache (C2), at each row's slot and position */
   FK_GEMM_STORE_KEYS = 4, /* one anchor's C = A B^T (f32 rows), and for each row and 128 columns the greedy
                              token's 64-bit key of their largest element: keys [M][N / 128] */
-  FK_GEMM_QKV_ROPE_PAGED = 5 /* FK_GEMM_QKV_ROPE with the caches paged pools, through each row's block table */
+  FK_GEMM_QKV_ROPE_PAGED = 5, /* FK_GEMM_QKV_ROPE with the caches paged pools, through each row's block table */
+  FK_GEMM_PART = 6      /* fk_skinny alone: partial sums of C = A B^T, k split among `parts` threadgroups */
 };
 
 typedef struct fk_gemm_params {
@@ -348,6 +349,8 @@ typedef struct fk_skinny_params {
   uint32_t run_chunks; /* chunks of a run that are live */
   uint32_t run;        /* rows from run to run */
   uint32_t apart;      /* rows from row to row of a chunk */
+  uint32_t compact;    /* the tiled matrices (A, the SiLU·mul product) hold the live chunks one after another */
+  uint32_t parts;      /* fk_skinny_part_*: k split among this many threadgroups, their sums into C0 [parts][live 16][ldc] */
   fk_gemm_rope_params r; /* the QKV epilogue's; paged: `length`, `slots`, `staged` unused */
   fk_paging pg;          /* paged */
 } fk_skinny_params;
@@ -401,6 +404,42 @@ typedef struct fk_prefill_attend_params {
                        staged runs read their own rows from ks and vs */
 } fk_prefill_attend_params;
 
+/* fk_rows_norm_w*: RMSNorm of the live rows (chunks as fk_skinny_params) into
+ * f16 tiles, the row first made as `source` says and stored in xout. */
+enum {
+  FK_ROWS_STORED = 0,     /* rows x, as they are (xout unused) */
+  FK_ROWS_GATHER_F16 = 1, /* the token's row of the f16 table times gfactor */
+  FK_ROWS_GATHER_F32 = 2, /* the same of an f32 table */
+  FK_ROWS_PARTS = 3       /* x plus the sum of `parts` partials [parts][live 16][width] */
+};
+
+typedef struct fk_rows_norm_params {
+  uint32_t m;
+  uint32_t width;
+  uint32_t live;
+  uint32_t run_chunks;
+  uint32_t run;
+  uint32_t apart;
+  uint32_t compact; /* y holds the live chunks one after another */
+  float eps;
+  float factor;
+  uint32_t has_gamma;
+  uint32_t source;
+  uint32_t table_rows;
+  float gfactor;
+  uint32_t parts;
+} fk_rows_norm_params;
+
+/* fk_rows_token: the greedy token of the live rows from `parts` keys each. */
+typedef struct fk_rows_token_params {
+  uint32_t m;
+  uint32_t live;
+  uint32_t run_chunks;
+  uint32_t run;
+  uint32_t apart;
+  uint32_t parts;
+} fk_rows_token_params;
+
 /* fk_rows_attend_{f16,bf16}, fk_rows_combine: the attention of `rows` rows,
  * `apart` rows of the step from one to the next, each a sequence's one, over
  * rings; the keys of a row go to `parts` threadgroups a kv head in tiles of
@@ -414,6 +453,7 @@ typedef struct fk_rows_attend_params {
   uint32_t slots;
   uint32_t window;   /* 0: none; else a row sees positions > position - window */
   uint32_t parts;
+  uint32_t compact;  /* out holds row i at row i, not i apart */
   float scale;
 } fk_rows_attend_params;
 

@@ -34,7 +34,7 @@ def attend(device, kernels, heads, kvh, length, positions, parts, window=0, bf16
     pos[:rows * APART:APART], sl[:rows * APART:APART] = positions, slot
     bufs = [device.upload(x) for x in (q, *bits, pos, sl, np.full(m * heads * 64, 3.0, np.float16))]
     part = device.alloc(rows * heads * parts * 66 * 4)
-    p = K.RowsAttendParams(rows, APART, heads, kvh, length, slots, window, parts, scale)
+    p = K.RowsAttendParams(rows, APART, heads, kvh, length, slots, window, parts, 0, scale)
     names = ("qr", "kc", "vc", "position", "slot", "out")
     bind = dict({n: b.ptr for n, b in zip(names, bufs)}, partials=part.ptr)
     print(f"rows attend {heads}/{kvh} length {length} rows {rows} parts {parts} window {window}", flush=True)

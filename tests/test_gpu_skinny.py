@@ -39,6 +39,7 @@ def live_rows(m, live, run_chunks, run, apart):
 def launch(device, kernels, mode, form, shape, bs, cs, n, bind=None, **params):
     m, live, run_chunks, run, apart, k = shape
     mb, nb, waves = K.SKINNY_FORMS[form]
+    params.setdefault("parts", 1)
     p = K.SkinnyParams(m=m, k=k, n_anchors=len(n), live=live, run_chunks=run_chunks, run=run, apart=apart, **params)
     first = np.concatenate([[0], np.cumsum(n)]).tolist()
     for i in range(4):
@@ -51,7 +52,8 @@ def launch(device, kernels, mode, form, shape, bs, cs, n, bind=None, **params):
     bound_to.update({f"c{i}": c.ptr for i, c in enumerate(cs)})
     bound_to.update({name: b.ptr for name, b in (bind or {}).items()})
     print(f"skinny {mode} {form} {shape} {n}", flush=True)
-    kernels.launch(f"fk_skinny_{mode}_{form}", -(-tiles_n // 8) * 8 * -(-live // mb), 64 * waves, bound_to, p)
+    kernels.launch(f"fk_skinny_{mode}_{form}", -(-tiles_n // 8) * 8 * -(-live // mb) * params["parts"],
+                   64 * waves, bound_to, p)
     device.sync()
 
 
@@ -186,4 +188,92 @@ def test_qkv_turns_and_stores_the_heads(device, kernels, form, where):
 
 
 def test_the_params_are_the_kernels():
-    assert ctypes.sizeof(K.SkinnyParams) == ctypes.sizeof(K.GemmParams) + 13 * 4
+    assert ctypes.sizeof(K.SkinnyParams) == ctypes.sizeof(K.GemmParams) + 15 * 4
+
+
+@pytest.mark.parametrize("parts", [1, 2, 5])
+@pytest.mark.parametrize("form", FORMS)
+def test_parts_sum_to_the_product(device, kernels, form, parts):
+    """Partial sums over parts of k (more than it has steps for, at 5), every
+    row of a live chunk, the live chunks one after another in A and C."""
+    for shape in (ROWS[2], ROWS[5], (256, 3, 3, 256, 1, 64)):
+        m, live, k = shape[0], shape[1], shape[-1]
+        a, w = f16((live * 16, k)), f16((256, k))
+        full = np.zeros((m, k), np.float16)
+        full[:live * 16] = a
+        ba, bw = device.upload(pack(full)), device.upload(pack(w))
+        bc = device.upload(np.full((parts * live * 16 + 1, 256), MARK, np.float32))
+        try:
+            launch(device, kernels, "part", form, shape, [bw], [bc], [256], {"a": ba}, parts=parts, compact=1)
+            got = bc.read(np.float32).reshape(-1, 256)
+            assert np.all(got[-1] == MARK)
+            got = got[:-1].reshape(parts, live * 16, 256).astype(np.float64).sum(axis=0)
+            exact = a.astype(np.float64) @ w.astype(np.float64).T
+            assert np.all(np.abs(got - exact) <= bound(a, w))
+        finally:
+            for b in (ba, bw, bc):
+                b.free()
+
+
+@pytest.mark.parametrize("shape", [ROWS[3], ROWS[5]], ids=["runs", "apart"])
+@pytest.mark.parametrize("source", [K.ROWS_STORED, K.ROWS_GATHER_F16, K.ROWS_GATHER_F32, K.ROWS_PARTS])
+@pytest.mark.parametrize("width", list(K.ROWS_NORM_THREADS))
+def test_rows_norm(device, kernels, width, source, shape):
+    """fk_rows_norm: each way a row is made, then its RMSNorm within one f16
+    rounding of binary64's, tiled in place or live rows alone."""
+    m, live, run_chunks, run, apart, _ = shape
+    rows = live_rows(*shape[:-1])
+    index = np.arange(live * 16)[:rows.size] if apart > 1 else None
+    rng = np.random.default_rng(width + source)
+    x = rng.standard_normal((m, width)).astype(np.float32)
+    gain = (1 + 0.1 * rng.standard_normal(width)).astype(np.float32)
+    table = rng.standard_normal((50, width)).astype(np.float16 if source == K.ROWS_GATHER_F16 else np.float32)
+    tokens = rng.integers(0, 60, m).astype(np.uint32)      # past the table: its last row
+    parts = rng.standard_normal((3, live * 16, width)).astype(np.float32)
+    where = np.concatenate([np.arange(c * 16, c * 16 + 16) for c in range(live)])[:rows.size]
+    if source == K.ROWS_STORED:
+        want = x[rows].astype(np.float64)
+    elif source == K.ROWS_PARTS:
+        want = x[rows].astype(np.float64) + parts[:, where].astype(np.float64).sum(axis=0)
+    else:
+        want = table[np.minimum(tokens[rows], 49)].astype(np.float64) * 1.25
+    bufs = {"x": device.upload(x), "table": device.upload(table), "tokens": device.upload(tokens),
+            "partials": device.upload(parts), "gamma": device.upload(gain),
+            "xout": device.upload(np.full((m, width), MARK, np.float32)),
+            "y": device.upload(np.full(m * width, MARK, np.float16))}
+    p = K.RowsNormParams(m, width, live, run_chunks, run, apart, int(apart > 1), 1e-5, 1.0, 1, source, 50, 1.25, 3)
+    try:
+        kernels.launch(f"fk_rows_norm_w{width}", live * 16, K.ROWS_NORM_THREADS[width],
+                       {n: b.ptr for n, b in bufs.items()}, p)
+        device.sync()
+        y = unpack(bufs["y"].read(np.float16), m, width).astype(np.float64)
+        xout = bufs["xout"].read(np.float32).reshape(m, width)
+        if source == K.ROWS_STORED:
+            assert np.all(xout == MARK)
+        else:
+            # three additions of binary32 rounding, or a product
+            assert np.all(np.abs(xout[rows] - want) <= 4 * 2.0**-24 * (np.abs(want) + 8))
+            assert np.all(np.delete(xout, rows, axis=0) == MARK)
+        tiles = rows if apart == 1 else index
+        normed = want * (np.mean(want * want, axis=1, keepdims=True) + 1e-5) ** -0.5 * gain
+        assert np.all(np.abs(y[tiles] - normed) <= np.abs(normed) * (2.0**-11 + 2.0**-18) + 2.0**-20)
+        assert np.all(np.delete(y, tiles, axis=0) == MARK)
+    finally:
+        for b in bufs.values():
+            b.free()
+
+
+@pytest.mark.parametrize("parts", [1, 250, 2000])
+def test_rows_token(device, kernels, parts):
+    m, live, run_chunks, run, apart, _ = shape = ROWS[5]
+    rows = live_rows(*shape[:-1])
+    keys = np.random.default_rng(parts).integers(0, 1 << 63, (m, parts), dtype=np.uint64)
+    bk, out = device.upload(keys), device.upload(np.full(m, 9, np.uint32))
+    kernels.launch("fk_rows_token", live * 16, 256, {"keys": bk.ptr, "out": out.ptr},
+                   K.RowsTokenParams(m, live, run_chunks, run, apart, parts))
+    device.sync()
+    got = out.read(np.uint32)
+    want = 0xFFFFFFFF - (keys.max(axis=1) & 0xFFFFFFFF)
+    assert np.array_equal(got[rows], want[rows].astype(np.uint32)) and np.all(np.delete(got, rows) == 9)
+    bk.free()
+    out.free()

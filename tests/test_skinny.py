@@ -66,7 +66,7 @@ def test_every_launch_passes_the_checks_and_makes_the_live_rows(case):
                 runtime.launch_check(L.entry, L.groups - 8, L.threads, L.lds_bytes, spans, params_struct(L))
             for b in ("a", "b0", "c0", "r0", "keys", "position", "rope", "c2"):
                 i = K.ABIS[L.entry].buffers.index(b)
-                if b in K.launch_reads(L.entry, p):
+                if b in K.launch_reads(L.entry, p) and not (b == "c0" and "_part_" in L.entry):
                     short = list(spans)
                     short[i] = (short[i][0], short[i][1] - 1)
                     with pytest.raises(runtime.FkError):
@@ -78,7 +78,7 @@ def test_the_keys_of_the_head_follow_its_tile():
     low, _, rows = lowered(ONE_B, 1, 100)
     head, token = low.launches[-2:]
     mode, (_, nb, _) = K.skinny_entry(head.entry)
-    assert mode == "store_keys" and token.entry == "fk_prefill_argmax_keys"
+    assert mode == "store_keys" and token.entry == "fk_rows_token"
     assert token.params["parts"] == 32000 // (16 * nb)
     assert low.buffers[head.bind["keys"]].count == rows * token.params["parts"]
 
@@ -106,21 +106,56 @@ def test_a_prefills_attention_splits_its_keys_where_its_blocks_are_few(seqs, seq
 
 
 def test_forms_by_size():
-    def down(c):
-        return skinny_form(c, -(-c // 16) * 256, 2048, 8192, "add")
+    def down(c, splits=(1,)):
+        return skinny_form(c, -(-c // 16) * 256, 2048, 8192, "add", splits)
     # larger tiles as the rows grow; fk_gemm where its rounds are full
-    assert [down(c) for c in (1, 3, 4, 7, 13, 22, 88, 128, 512)] == \
+    assert [down(c) and down(c)[0] for c in (1, 3, 4, 7, 13, 22, 88, 128, 512)] == \
         ["m1n1", "m2n1", "m2n1", "m2n2", "m4n2", "m4n4", "m8n8", "m8n8", None]
-    assert skinny_form(1, 256, 3072, 2048, "qkv_rope") == "m1n2"      # pairs of columns
+    # k split further where a norm adds the parts, until they cost what they save
+    assert [down(c, (1, 2, 4, 8)) for c in (1, 4, 7, 13, 64)] == \
+        [("m1n2", 4), ("m4n2", 4), ("m4n4", 4), ("m4n4", 2), ("m4n8", 1)]
+    assert skinny_form(1, 256, 3072, 2048, "qkv_rope") == ("m1n2", 1)      # pairs of columns
     assert skinny_form(22, 512, 16384, 2048, "silu_mul") is None
-    assert skinny_form(1, 256, 2048, 960, "add") is None              # a short k
+    assert skinny_form(1, 256, 2048, 960, "add") is None                   # a short k
     for c in range(1, 400):
         m = -(-c // 16) * 256
         for n, k, mode in ((3072, 2048, "qkv_rope_paged"), (16384, 2048, "silu_mul"), (32000, 2048, "store_keys"),
                            (256, 1024, "store"), (512, 16384, "add")):
-            form = skinny_form(c, m, n, k, mode)
-            if form is not None:
-                mb, nb, _ = K.SKINNY_FORMS[form]
+            picked = skinny_form(c, m, n, k, mode)
+            if picked is not None:
+                mb, nb, _ = K.SKINNY_FORMS[picked[0]]
                 assert mb < 2 * c and n % (16 * nb) == 0 and (nb > 1 or mode not in K.SKINNY_PAIR_MODES)
     assert all(L.entry.startswith("fk_skinny") is False
                for L in lowered(SMALL_PREFILL, 2, 100)[0].launches)
+
+
+def test_the_kernels_between_the_gemms_take_the_live_rows():
+    low, real, rows = lowered(ONE_B, 41, 1, decode=True)
+    norms = [L for L in low.launches if L.entry == "fk_rows_norm_w2048"]
+    assert [L.params["source"] for L in norms] == [K.ROWS_GATHER_F16, K.ROWS_PARTS, K.ROWS_PARTS]
+    assert all(L.groups == 48 for L in norms)     # 41 rows in chunks of 16
+    assert not any(L.entry.startswith(("fk_prefill_norm", "fk_prefill_gather", "fk_prefill_argmax"))
+                   for L in low.launches)
+    # each part's sums are read, and only by the norm after it
+    for i, L in enumerate(low.launches):
+        if "_part_" in L.entry:
+            norm = low.launches[i + 1]
+            assert norm.bind["partials"] == L.bind["c0"] and norm.params["parts"] == L.params["parts"] > 1
+            assert low.buffers[L.bind["c0"]].count >= L.params["parts"] * 48 * 2048
+    # the tiled values hold the live rows one after another, everywhere
+    assert all(L.params["compact"] == 1 for L in low.launches if L.entry != "fk_rows_token")
+
+
+def test_a_prefills_tiled_values_stay_in_place():
+    low, _, _ = lowered(ONE_B, 1, 100)
+    assert not any(L.params.get("compact") for L in low.launches)
+    # past ROWS_NORM_CHUNKS the plain kernels stay
+    low, _, _ = lowered(ONE_B, 4, 700)
+    assert not any(L.entry.startswith(("fk_rows", "fk_skinny_part")) for L in low.launches)
+
+
+def test_a_batch_through_fk_gemm_is_not_compact():
+    # k 512: fk_gemm's, which reads the step's rows in place
+    low, _, _ = lowered(SMALL_PREFILL, 4, 1, decode=True)
+    assert any(L.entry.startswith("fk_gemm") for L in low.launches)
+    assert not any(L.params.get("compact") for L in low.launches)
