@@ -302,6 +302,32 @@ std::vector<Entry> build() {
          FK_P(S, groups_per_rank, "u32")},
         sizeof(S));
   }
+  for (const char *t : {"f16", "bf16"}) {
+    using S = fk_step_router_params;
+    add(std::string("fk_step_router_") + t, 1024,
+        {buf("x", "read", "f32"), buf("gamma", "read", "f32"), buf("y", "write", "f32"), buf("w", "read", t),
+         buf("logits", "write", "f32"), buf("scale", "read", "f32"), buf("ids", "write", "u32"),
+         buf("ws", "write", "f32")},
+        {FK_P(S, width, "u32"), FK_P(S, experts, "u32"), FK_P(S, k, "u32"), FK_P(S, has_gamma, "u32"),
+         FK_P(S, has_scale, "u32"), FK_P(S, eps, "f32"), FK_P(S, factor, "f32")},
+        sizeof(S));
+  }
+  for (const char *t : {"f16", "bf16", "f32"}) {
+    using S = fk_gemv_routed_act_params;
+    add(std::string("fk_gemv_routed_act_") + t, 256,
+        {buf("table", "read", "u64"), buf("ids", "read", "u32"), buf("x", "read", "f32"), buf("y", "write", "f32"),
+         buf("out", "write", "f32")},
+        {FK_P(S, n, "u32"), FK_P(S, k, "u32"), FK_P(S, ranks, "u32"), FK_P(S, shared, "u32"), FK_P(S, entries, "u32"),
+         FK_P(S, groups_per_rank, "u32"), FK_P(S, act, "u32")},
+        sizeof(S));
+    using C = fk_gemv_routed_combine_params;
+    add(std::string("fk_gemv_routed_combine_") + t, 256,
+        {buf("table", "read", "u64"), buf("ids", "read", "u32"), buf("x", "read", "f32"), buf("y", "write", "f32"),
+         buf("w", "read", "f32"), buf("res", "read", "f32"), buf("out", "write", "f32")},
+        {FK_P(C, n, "u32"), FK_P(C, k, "u32"), FK_P(C, ranks, "u32"), FK_P(C, shared, "u32"), FK_P(C, entries, "u32"),
+         FK_P(C, residual, "u32")},
+        sizeof(C));
+  }
   add("fk_step_advance", 0,
       {buf("next_token", "read", "u32"), buf("token", "write", "u32"), buf("position", "read_write", "u32")},
       {FK_P(fk_step_advance_params, context, "u32"), FK_P(fk_step_advance_params, step, "u32")},
@@ -818,6 +844,46 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
                  p.rows, p.width, p.count, p.table_rows, groups, threads);
     need = {{"table", (uint64_t)p.table_rows * p.width * eb}, {"tokens", (uint64_t)p.rows * p.count * 4},
             {"y", n * 4}};
+  } else if (std::strncmp(entry, "fk_step_router_", 15) == 0) {
+    fk_step_router_params p;
+    std::memcpy(&p, params, sizeof p);
+    if (p.width == 0 || p.width % 8 || p.width > 2048 || p.experts == 0 || p.experts > 32 || p.k < 1 || p.k > 8 ||
+        p.k > p.experts || groups != 1)
+      return bad(err, cap, FK_ERR_ARG, "%s: the %u largest of %u rows of %u, %u threadgroups", entry, p.k, p.experts,
+                 p.width, groups);
+    need = {{"x", (uint64_t)p.width * 4},       {"y", (uint64_t)p.width * 4}, {"w", (uint64_t)p.experts * p.width * 2},
+            {"logits", (uint64_t)p.experts * 4}, {"ids", (uint64_t)p.k * 4},   {"ws", (uint64_t)p.k * 4}};
+    if (p.has_gamma) need.push_back({"gamma", (uint64_t)p.width * 4});
+    if (p.has_scale) need.push_back({"scale", (uint64_t)p.experts * 4});
+  } else if (std::strncmp(entry, "fk_gemv_routed_act_", 19) == 0) {
+    fk_gemv_routed_act_params p;
+    std::memcpy(&p, params, sizeof p);
+    const uint32_t pack = std::strcmp(entry + 19, "f32") == 0 ? 4 : 8;
+    if (p.entries == 0 || p.ranks == 0 || p.n == 0 || p.n % 2 || p.k == 0 || p.k % pack || p.k / pack > 512 ||
+        p.groups_per_rank == 0 || groups != p.ranks * p.groups_per_rank || p.groups_per_rank * 4ull < p.n / 2 ||
+        p.act > FK_ACT_GELU_TANH)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u ranks of %u rows at k %u, activation %u, in %u groups", entry, p.ranks,
+                 p.n, p.k, p.act, groups);
+    need = {{"table", (uint64_t)p.entries * 8},
+            {"ids", (uint64_t)p.ranks * 4},
+            {"x", (uint64_t)(p.shared ? 1 : p.ranks) * p.k * 4},
+            {"y", (uint64_t)p.ranks * p.n * 4},
+            {"out", (uint64_t)p.ranks * (p.n / 2) * 4}};
+  } else if (std::strncmp(entry, "fk_gemv_routed_combine_", 23) == 0) {
+    fk_gemv_routed_combine_params p;
+    std::memcpy(&p, params, sizeof p);
+    const uint32_t pack = std::strcmp(entry + 23, "f32") == 0 ? 4 : 8;
+    if (p.entries == 0 || p.ranks == 0 || p.ranks > 4 || p.n == 0 || p.k == 0 || p.k % pack ||
+        p.k / pack > (p.ranks > 2 ? 128u : 256u) || groups * 4ull < p.n)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u ranks of %u rows at k %u in %u groups", entry, p.ranks, p.n, p.k,
+                 groups);
+    need = {{"table", (uint64_t)p.entries * 8},
+            {"ids", (uint64_t)p.ranks * 4},
+            {"x", (uint64_t)(p.shared ? 1 : p.ranks) * p.k * 4},
+            {"y", (uint64_t)p.ranks * p.n * 4},
+            {"w", (uint64_t)p.ranks * 4},
+            {"out", (uint64_t)p.n * 4}};
+    if (p.residual) need.push_back({"res", (uint64_t)p.n * 4});
   } else if (std::strncmp(entry, "fk_gemv_routed_", 15) == 0) {
     fk_gemv_routed_params p;
     std::memcpy(&p, params, sizeof p);

@@ -240,27 +240,38 @@ __device__ __forceinline__ void gemv_wave(const WT *__restrict__ w, const XT *__
   }
 }
 
-// The same rows and order with every load in flight at once, for rows of at
-// most 64 KPL packs: each lane issues all of its packs' 16-byte loads — W's
+// One pack's products into its chains: four to a chain, (p0 + p1) + (p2 + p3).
+template <int P>
+__device__ __forceinline__ void add_pack(float (&acc)[P / 4], const float (&xf)[P], const float (&wf)[P], bool live) {
+#pragma unroll
+  for (int c = 0; c < P / 4; c++) {
+    const float p0 = xf[4 * c] * wf[4 * c];
+    const float p1 = xf[4 * c + 1] * wf[4 * c + 1];
+    const float p2 = xf[4 * c + 2] * wf[4 * c + 2];
+    const float p3 = xf[4 * c + 3] * wf[4 * c + 3];
+    const float sum = acc[c] + ((p0 + p1) + (p2 + p3));
+    acc[c] = live ? sum : acc[c];
+  }
+}
+
+// The same order with every load in flight at once, for rows of at most
+// 64 KPL packs: the sums of R rows wr[q], every lane's, times one x (XR = 1)
+// or one each (XR = R).  Each lane issues all of its packs' 16-byte loads — W's
 // first, then x's, the indices clamped into the row so every load is
 // unconditional and the compiler keeps them all outstanding — and only then
 // computes, packs past the row skipped.  One round trip to memory a
 // wavefront, where the loop above waits for each unrolled group of packs in
 // turn.  FULL: the row fills every lane's KPL packs (k = 64 KPL P), so no
 // pack needs the check.
-template <typename WT, typename XT, int P, int R, int KPL, bool FULL>
-__device__ __forceinline__ void gemv_wave_inflight(const WT *__restrict__ w, const XT *__restrict__ x,
-                                                   const float *__restrict__ scale, float *__restrict__ y,
-                                                   uint32_t n, uint32_t k, uint32_t row0) {
+template <typename WT, typename XT, int P, int R, int XR, int KPL, bool FULL>
+__device__ __forceinline__ void gemv_sums_inflight(const WT *const (&wr)[R], const XT *const (&xr)[XR], uint32_t packs,
+                                                   float (&t)[R]) {
   constexpr int C = P / 4;
   constexpr int XW = P * (int)sizeof(XT) / 16;  // 16-byte words of an x pack
   static_assert(P * sizeof(WT) == 16, "a W pack is one 16-byte load");
+  static_assert(XR == 1 || XR == R, "one x, or one a row");
   const uint32_t lane = threadIdx.x & (FK_WAVE - 1);
-  const uint32_t packs = k / P;
-  const WT *wr[R];
-#pragma unroll
-  for (int q = 0; q < R; q++) wr[q] = w + (size_t)min(row0 + q, n - 1) * k;
-  uint4 wv[R][KPL], xv[KPL][XW];
+  uint4 wv[R][KPL], xv[XR][KPL][XW];
 #pragma unroll
   for (int it = 0; it < KPL; it++) {
     const uint32_t jc = min(lane + FK_WAVE * (uint32_t)it, packs - 1);
@@ -271,7 +282,9 @@ __device__ __forceinline__ void gemv_wave_inflight(const WT *__restrict__ w, con
   for (int it = 0; it < KPL; it++) {
     const uint32_t jc = min(lane + FK_WAVE * (uint32_t)it, packs - 1);
 #pragma unroll
-    for (int u = 0; u < XW; u++) xv[it][u] = reinterpret_cast<const uint4 *>(x + (size_t)jc * P)[u];
+    for (int q = 0; q < XR; q++)
+#pragma unroll
+      for (int u = 0; u < XW; u++) xv[q][it][u] = reinterpret_cast<const uint4 *>(xr[q] + (size_t)jc * P)[u];
   }
   float acc[R][C];
 #pragma unroll
@@ -282,32 +295,41 @@ __device__ __forceinline__ void gemv_wave_inflight(const WT *__restrict__ w, con
   for (int it = 0; it < KPL; it++) {
     // A pack past the row is computed from the clamped loads and not added:
     // a select, so that no load sits in a branch.
-    const bool live = lane + FK_WAVE * (uint32_t)it < packs;
+    const bool live = FULL || lane + FK_WAVE * (uint32_t)it < packs;
     float xf[P];
-    unpack<P>(xv[it], xf, XT{});
 #pragma unroll
     for (int q = 0; q < R; q++) {
+      if (q < XR) unpack<P>(xv[q < XR ? q : 0][it], xf, XT{});
       float wf[P];
       unpack_w<P>(wv[q][it], wf, WT{});
-#pragma unroll
-      for (int c = 0; c < C; c++) {
-        float p0 = xf[4 * c] * wf[4 * c];
-        float p1 = xf[4 * c + 1] * wf[4 * c + 1];
-        float p2 = xf[4 * c + 2] * wf[4 * c + 2];
-        float p3 = xf[4 * c + 3] * wf[4 * c + 3];
-        const float sum = acc[q][c] + ((p0 + p1) + (p2 + p3));
-        acc[q][c] = FULL || live ? sum : acc[q][c];
-      }
+      add_pack<P>(acc[q], xf, wf, live);
     }
   }
 #pragma unroll
   for (int q = 0; q < R; q++) {
-    float t = acc[q][0];
+    t[q] = acc[q][0];
 #pragma unroll
-    for (int c = 1; c < C; c++) t = t + acc[q][c];
-    t = wave_sum(t);
+    for (int c = 1; c < C; c++) t[q] = t[q] + acc[q][c];
+  }
+  wave_sums<R>(t);
+}
+
+// R rows of y = W x by one wavefront, in flight at once.
+template <typename WT, typename XT, int P, int R, int KPL, bool FULL>
+__device__ __forceinline__ void gemv_wave_inflight(const WT *__restrict__ w, const XT *__restrict__ x,
+                                                   const float *__restrict__ scale, float *__restrict__ y,
+                                                   uint32_t n, uint32_t k, uint32_t row0) {
+  const uint32_t lane = threadIdx.x & (FK_WAVE - 1);
+  const WT *wr[R];
+#pragma unroll
+  for (int q = 0; q < R; q++) wr[q] = w + (size_t)min(row0 + q, n - 1) * k;
+  const XT *const xr[1] = {x};
+  float t[R];
+  gemv_sums_inflight<WT, XT, P, R, 1, KPL, FULL>(wr, xr, k / P, t);
+#pragma unroll
+  for (int q = 0; q < R; q++) {
     const uint32_t row = row0 + q;
-    if (lane == 0 && row < n) y[row] = scale ? t * scale[row] : t;
+    if (lane == 0 && row < n) y[row] = scale ? t[q] * scale[row] : t[q];
   }
 }
 

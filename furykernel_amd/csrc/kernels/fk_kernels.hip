@@ -7,6 +7,7 @@
 #include "fk_step.h"
 #include "fk_gemm.h"
 #include "fk_prefill.h"
+#include "fk_routed.h"
 #include "fk_rows_attend.h"
 #include "fk_rows_norm.h"
 #include "fk_skinny.h"

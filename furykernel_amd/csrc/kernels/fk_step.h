@@ -177,57 +177,77 @@ extern "C" __global__ void __launch_bounds__(FK_STEP_THREADS)
   }
 }
 
-// Routing: one wavefront, k rounds of the wavefront's largest key among the
-// logits not yet taken (the argmax keys, a NaN's the lowest), then lane 0's
-// weights.
-extern "C" __global__ void __launch_bounds__(FK_WAVE)
-    fk_step_route(const float *__restrict__ x, const float *__restrict__ scale, uint32_t *__restrict__ ids,
-                  float *__restrict__ ws, fk_step_route_params p) {
-  const uint32_t lane = threadIdx.x;
-  uint32_t taken[8];
-  float tv[8];
+namespace fk {
+
+// The larger of a lane's key and that of the lane CTRL pairs it with.
+template <int CTRL>
+__device__ __forceinline__ uint64_t dpp_max_key(uint64_t v) {
+  const uint64_t o = ((uint64_t)(uint32_t)dpp_i<CTRL>((int)(v >> 32)) << 32) | (uint32_t)dpp_i<CTRL>((int)(uint32_t)v);
+  return o > v ? o : v;
+}
+
+// The wavefront's largest key, every lane: within rows of 16 lanes by DPP,
+// then across the four rows (wave_max's steps).
+__device__ __forceinline__ uint64_t wave_max_key(uint64_t v) {
+  v = dpp_max_key<0xB1>(v);   // quad_perm [1, 0, 3, 2]
+  v = dpp_max_key<0x4E>(v);   // quad_perm [2, 3, 0, 1]
+  v = dpp_max_key<0x141>(v);  // row_half_mirror
+  v = dpp_max_key<0x140>(v);  // row_mirror
+  uint64_t best = 0;
 #pragma unroll
-  for (int r = 0; r < 8; r++) taken[r] = 0xFFFFFFFFu, tv[r] = 0.0f;
+  for (int r = 0; r < 4; r++) {
+    const uint64_t o = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), 16 * r) << 32) |
+                       (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 16 * r);
+    best = o > best ? o : best;
+  }
+  return best;
+}
+
+// Routing by one wavefront: k rounds of the wavefront's largest key among the
+// logits x not yet taken (the argmax keys, a NaN's the lowest), then lane r
+// the weight of rank r, the exps' sum in rank order.
+__device__ __forceinline__ void route_row(const float *x, const float *__restrict__ scale, uint32_t *__restrict__ ids,
+                                          float *__restrict__ ws, uint32_t n, uint32_t k, bool has_scale) {
+  const uint32_t lane = threadIdx.x & (FK_WAVE - 1);
+  uint32_t taken[8], mine = 0;
+#pragma unroll
+  for (int r = 0; r < 8; r++) taken[r] = 0xFFFFFFFFu;
 #pragma unroll
   for (int r = 0; r < 8; r++) {
-    if ((uint32_t)r < p.k) {
+    if ((uint32_t)r < k) {
       uint64_t best = 0;
-      for (uint32_t i = lane; i < p.n; i += FK_WAVE) {
+      for (uint32_t i = lane; i < n; i += FK_WAVE) {
         bool seen = false;
 #pragma unroll
         for (int q = 0; q < 8; q++) seen |= q < r && taken[q] == i;
         const float v = x[i];
-        const uint64_t key = __builtin_isnan(v) ? (uint64_t)(0xFFFFFFFFu - i) : fk::argmax_key(v, i);
+        const uint64_t key = __builtin_isnan(v) ? (uint64_t)(0xFFFFFFFFu - i) : argmax_key(v, i);
         if (!seen && key > best) best = key;
       }
-#pragma unroll
-      for (int m = 1; m < FK_WAVE; m <<= 1) {
-        const uint64_t o = __shfl_xor(best, m);
-        best = o > best ? o : best;
-      }
-      taken[r] = 0xFFFFFFFFu - (uint32_t)(best & 0xFFFFFFFFu);
-      tv[r] = x[taken[r]];
+      taken[r] = 0xFFFFFFFFu - (uint32_t)(wave_max_key(best) & 0xFFFFFFFFu);
+      mine = lane == (uint32_t)r ? taken[r] : mine;
     }
   }
-  if (lane == 0) {
-    float e[8], total = 0.0f;
+  // (Lanes past k take index 0 and store nothing.)
+  const float e = exp_once(x[mine] - x[taken[0]]);
+  float total = 0.0f;
 #pragma unroll
-    for (int r = 0; r < 8; r++) {
-      if ((uint32_t)r < p.k) {
-        e[r] = fk::exp_once(tv[r] - tv[0]);
-        total = total + e[r];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 8; r++) {
-      if ((uint32_t)r < p.k) {
-        float w = e[r] / total;
-        if (p.has_scale) w = w * scale[taken[r]];
-        ids[r] = taken[r];
-        ws[r] = w;
-      }
-    }
+  for (int r = 0; r < 8; r++)
+    if ((uint32_t)r < k) total = total + readlane_f(e, r);
+  if (lane < k) {
+    float w = e / total;
+    if (has_scale) w = w * scale[mine];
+    ids[lane] = mine;
+    ws[lane] = w;
   }
+}
+
+}  // namespace fk
+
+extern "C" __global__ void __launch_bounds__(FK_WAVE)
+    fk_step_route(const float *__restrict__ x, const float *__restrict__ scale, uint32_t *__restrict__ ids,
+                  float *__restrict__ ws, fk_step_route_params p) {
+  fk::route_row(x, scale, ids, ws, p.n, p.k, p.has_scale != 0);
 }
 
 // CombineRanks, and the residual add after it.

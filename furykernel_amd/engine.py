@@ -17,7 +17,7 @@ import numpy as np
 
 from . import kernels as K
 from . import runtime
-from .lower import Launch, Lowered, rope_table
+from .lower import Launch, Lowered, rope_table, routed_fusions
 
 _NP = {"f32": np.float32, "f16": np.float16, "bf16": np.uint16, "u32": np.uint32, "u16": np.uint16,
        "u64": np.uint64}
@@ -38,6 +38,9 @@ _STRUCTS = {
     "fk_gemv_routed_f32_r1": K.GemvRoutedParams,
     "fk_gemv_routed_bf16_r1": K.GemvRoutedParams,
     "fk_gemv_routed_bf16_r2": K.GemvRoutedParams,
+    **{f"fk_step_router_{t}": K.RouterParams for t in ("f16", "bf16")},
+    **{f"fk_gemv_routed_act_{t}": K.GemvRoutedActParams for t in ("f16", "bf16", "f32")},
+    **{f"fk_gemv_routed_combine_{t}": K.GemvRoutedCombineParams for t in ("f16", "bf16", "f32")},
     "fk_step_elementwise": K.ElementwiseParams,
     "fk_gemv_p4_f32": K.GemvParams,
     "fk_gemv_p4_f16": K.GemvParams,
@@ -224,6 +227,8 @@ class Engine:
         self.table = runtime.Table(device)
         for launch in lowered.launches:
             self._add(launch)
+        # first launch -> (launches, the table's index of the one that does what they do)
+        self._fused = {first: (count, self._add(launch)) for first, count, launch in routed_fusions(lowered)}
         self._advance: dict = {}
 
     def _add(self, launch: Launch) -> int:
@@ -298,6 +303,8 @@ class Engine:
             (not picks or picks[-1] == last)
         if folded:
             picks[-1] = self._advance_index(**advance)
+        if self._fused:
+            picks = self._with_fused(picks)
         # runs of consecutive indices go to the table in one call each
         i = 0
         while i < len(picks):
@@ -308,6 +315,18 @@ class Engine:
             i = j + 1
         if advance is not None and not folded:
             self.enqueue_advance(stream=stream, **advance)
+
+    def _with_fused(self, picks: list) -> list:
+        """`picks` with each run of launches that one launch does in their
+        place as that one."""
+        out, i = [], 0
+        while i < len(picks):
+            count, index = self._fused.get(picks[i], (1, picks[i]))
+            if picks[i:i + count] != list(range(picks[i], picks[i] + count)):
+                count, index = 1, picks[i]
+            out.append(index)
+            i += count
+        return out
 
     def _advance_index(self, token_out: str, token_in: str, position: str, context: int, step: int = 1) -> int:
         """The token launch that also advances (the greedy token it makes is

@@ -288,6 +288,19 @@ class CombineRanksParams(ctypes.Structure):
     _fields_ = [("seg", ctypes.c_uint32), ("ranks", ctypes.c_uint32), ("residual", ctypes.c_uint32)]
 
 
+class RouterParams(ctypes.Structure):
+    _fields_ = [(f, ctypes.c_uint32) for f in ("width", "experts", "k", "has_gamma", "has_scale")] + \
+        [("eps", ctypes.c_float), ("factor", ctypes.c_float)]
+
+
+class GemvRoutedActParams(ctypes.Structure):
+    _fields_ = GemvRoutedParams._fields_ + [("act", ctypes.c_uint32)]
+
+
+class GemvRoutedCombineParams(ctypes.Structure):
+    _fields_ = GemvRoutedParams._fields_[:5] + [("residual", ctypes.c_uint32)]
+
+
 class StepCombineParams(ctypes.Structure):
     _fields_ = [("heads", ctypes.c_uint32), ("head_dim", ctypes.c_uint32), ("splits", ctypes.c_uint32)]
 
@@ -491,6 +504,13 @@ ABIS: dict[str, KernelAbi] = {
     **{e: KernelAbi(e, ("table", "ids", "x", "y"), GemvRoutedParams)
        for e in ("fk_gemv_routed_f16_r1", "fk_gemv_routed_f16_r2", "fk_gemv_routed_f32_r1",
                  "fk_gemv_routed_bf16_r1", "fk_gemv_routed_bf16_r2")},
+    **{f"fk_step_router_{t}": KernelAbi(f"fk_step_router_{t}", ("x", "gamma", "y", "w", "logits", "scale", "ids", "ws"),
+                                        RouterParams, 1024) for t in ("f16", "bf16")},
+    **{f"fk_gemv_routed_act_{t}": KernelAbi(f"fk_gemv_routed_act_{t}", ("table", "ids", "x", "y", "out"),
+                                            GemvRoutedActParams, 256) for t in ("f16", "bf16", "f32")},
+    **{f"fk_gemv_routed_combine_{t}": KernelAbi(f"fk_gemv_routed_combine_{t}",
+                                                ("table", "ids", "x", "y", "w", "res", "out"),
+                                                GemvRoutedCombineParams, 256) for t in ("f16", "bf16", "f32")},
     "fk_step_elementwise": KernelAbi("fk_step_elementwise", ("a", "b", "c", "y"), ElementwiseParams),
     **{f"fk_step_gather_{t}": KernelAbi(f"fk_step_gather_{t}", ("table", "tokens", "y"), GatherParams)
        for t in ("f32", "f16", "bf16")},
@@ -824,6 +844,11 @@ def launch_reads(entry: str, params: dict) -> set[str]:
         return need
     if entry == "fk_step_route":
         return {"x", "ids", "ws"} | ({"scale"} if params.get("has_scale") else set())
+    if entry.startswith("fk_step_router_"):
+        return set(abi.buffers) - (set() if params.get("has_gamma") else {"gamma"}) - \
+            (set() if params.get("has_scale") else {"scale"})
+    if entry.startswith("fk_gemv_routed_combine_"):
+        return set(abi.buffers) - (set() if params.get("residual") else {"res"})
     if entry == "fk_step_combine_ranks":
         return {"w", "x", "y"} | ({"res"} if params.get("residual") else set())
     if entry == "fk_step_act_mul":

@@ -258,6 +258,97 @@ def _fuse_light(out: Lowered, compute_units: int, choose: Optional[Callable] = N
     out.launches = fused
 
 
+# What the threadgroup of fk_routed.h's router holds.
+ROUTER_WIDTH, ROUTER_EXPERTS = 2048, 32
+
+
+def routed_fusions(out: Lowered) -> list:
+    """(first launch, launches, the launch that does what they do) of the
+    routed steps' launches that fk_routed.h's kernels take, every value that
+    those store stored as before:
+
+    - the norm of a row, the router's logits of it and their route, where one
+      threadgroup holds them (4.2 µs less a step at 2048 columns, of 16 and of
+      32 experts; 2 less at 512 of 8);
+    - a routed GEMV and the gated activation of its rows;
+    - a routed GEMV, the combine of its ranks and the residual add (with the
+      activation's, 3.6 µs less a step of two experts of 1024, 6.2 of four).
+
+    None where a value that one of them stores is another's operand by
+    another route (a step's stored values have buffers of their own)."""
+    found, i, launches = [], 0, out.launches
+    while i < len(launches):
+        got = _fused_router(launches[i:i + 3]) or _fused_routed(launches[i:i + 2])
+        if got is not None:
+            found.append((i, *got))
+        i += got[0] if got is not None else 1
+    return found
+
+
+def _apart(inputs, outputs) -> bool:
+    """Whether no output is an input or another output."""
+    outputs = list(outputs)
+    return len(set(outputs)) == len(outputs) and not set(outputs) & set(inputs)
+
+
+def _fused_router(run: list) -> Optional[tuple]:
+    if [L.entry for L in run[::2]] != ["fk_rmsnorm_f32", "fk_step_route"]:
+        return None
+    norm, gm, route = run
+    p = gm.params
+    wt = gm.meta.get("wtype")
+    if gm.entry not in (f"fk_step_gemv_{wt}_k2048_r{r}_p0_e0" for r in (1, 2)) or wt not in ("f16", "bf16"):
+        return None
+    width, experts = norm.params["width"], p["rows"][0]
+    if norm.params["rows"] != 1 or norm.params["seg"] != width or p["k"] != width or width % 8 or \
+            width > ROUTER_WIDTH or p["n_anchors"] != 1 or not p["store_tile"] or experts > ROUTER_EXPERTS or \
+            gm.bind["src"] != norm.bind["y"] or route.bind["x"] != gm.bind["y0"] or route.params["n"] != experts:
+        return None
+    gamma = norm.bind["gamma"] if norm.params["has_gamma"] else None
+    scale = route.bind["scale"] if route.params["has_scale"] else None
+    bind = {"x": norm.bind["x"], "gamma": gamma, "y": norm.bind["y"], "w": gm.bind["w0"], "logits": gm.bind["y0"],
+            "scale": scale, "ids": route.bind["ids"], "ws": route.bind["ws"]}
+    if not _apart([bind[b] for b in ("x", "gamma", "w", "scale")], [bind[b] for b in ("y", "logits", "ids", "ws")]):
+        return None
+    params = {"width": width, "experts": experts, "k": route.params["k"], "has_gamma": norm.params["has_gamma"],
+              "has_scale": route.params["has_scale"], "eps": norm.params["eps"], "factor": norm.params["factor"]}
+    return 3, Launch(f"{gm.step}+{route.step}", f"fk_step_router_{wt}", 1, 1024, bind, params)
+
+
+def _fused_routed(run: list) -> Optional[tuple]:
+    if len(run) < 2 or not run[0].entry.startswith("fk_gemv_routed_"):
+        return None
+    gm, then = run
+    p = gm.params
+    wt = gm.entry.split("_")[3]
+    packs = p["k"] // (4 if wt == "f32" else 8)
+    step = f"{gm.step}+{then.step}"
+    operands = [gm.bind[b] for b in ("table", "ids", "x")]
+    if then.entry == "fk_step_act_mul":
+        half = p["n"] // 2
+        segment = then.params.get("half", 0) or (then.params["b_off"] if p["ranks"] == 1 else 0)
+        if {then.bind["a"], then.bind["b"]} != {gm.bind["y"]} or p["n"] != 2 * half or segment != half or \
+                then.params["n"] != p["ranks"] * half or packs > 512 or \
+                not _apart(operands, [gm.bind["y"], then.bind["y"]]):
+            return None
+        per_rank = -(-half // 4)
+        return 2, Launch(step, f"fk_gemv_routed_act_{wt}", p["ranks"] * per_rank, 256,
+                         dict(gm.bind, out=then.bind["y"]),
+                         dict(p, groups_per_rank=per_rank, act=then.params["act"]))
+    if then.entry == "fk_step_combine_ranks":
+        q = then.params
+        if then.bind["x"] != gm.bind["y"] or q["seg"] != p["n"] or q["ranks"] != p["ranks"] or p["ranks"] > 4 or \
+                packs > (128 if p["ranks"] > 2 else 256) or \
+                not _apart(operands + [then.bind["w"]], [gm.bind["y"], then.bind["y"]]) or \
+                (q["residual"] and then.bind["res"] == gm.bind["y"]):
+            return None
+        params = {f: p[f] for f in ("n", "k", "ranks", "shared", "entries")}
+        return 2, Launch(step, f"fk_gemv_routed_combine_{wt}", -(-p["n"] // 4), 256,
+                         dict(gm.bind, w=then.bind["w"], res=then.bind["res"] if q["residual"] else None,
+                              out=then.bind["y"]), dict(params, residual=q["residual"]))
+    return None
+
+
 GEMV_THREADS = 512
 
 

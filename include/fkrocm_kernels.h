@@ -222,6 +222,42 @@ typedef struct fk_step_combine_ranks_params {
   uint32_t residual;
 } fk_step_combine_ranks_params;
 
+/* A routed step's launches as fewer (fk_routed.h), each value as the kernels
+ * they replace store it.  The RMSNorm of one row of `width` (a multiple of 8,
+ * at most 2048), the logits of `experts` rows (at most 32) and their route. */
+typedef struct fk_step_router_params {
+  uint32_t width;
+  uint32_t experts;
+  uint32_t k; /* 1 to 8, at most experts */
+  uint32_t has_gamma;
+  uint32_t has_scale;
+  float eps;
+  float factor;
+} fk_step_router_params;
+
+/* LinearRouted of 2 half rows a rank and out[rank half + i] = act(y[i]) *
+ * y[half + i] of each rank's rows (n = 2 half; k at most 512 packs). */
+typedef struct fk_gemv_routed_act_params {
+  uint32_t n;
+  uint32_t k;
+  uint32_t ranks;
+  uint32_t shared;
+  uint32_t entries;
+  uint32_t groups_per_rank;
+  uint32_t act;
+} fk_gemv_routed_act_params;
+
+/* LinearRouted, CombineRanks of its ranks and, with `residual`, the add after
+ * it: rows of at most 256 packs of up to 2 ranks, 128 of up to 4. */
+typedef struct fk_gemv_routed_combine_params {
+  uint32_t n;
+  uint32_t k;
+  uint32_t ranks;
+  uint32_t shared;
+  uint32_t entries;
+  uint32_t residual;
+} fk_gemv_routed_combine_params;
+
 /* A light step's elementwise value of stored rows, one thread an element of
  * the n = rows * width elements (Eval.hs:336-355, 536-544):
  *   FK_ELT_ADD          y = a + b                      (Add)
