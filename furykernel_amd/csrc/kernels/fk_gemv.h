@@ -333,44 +333,64 @@ __device__ __forceinline__ void gemv_wave_inflight(const WT *__restrict__ w, con
   }
 }
 
-// The int8 weights' full rows (k = 64 KPL 16) with x (f16) staged once a
-// threadgroup of T threads in LDS, where every wavefront would otherwise read
-// the whole 16 KB x row from memory beside its own 8 KB of weights: the x
-// loads first (T into 16-byte chunks), then the rows' weights, then the
-// chunks into LDS transposed (chunk u of lane l's pack it at (2 it + u) 64 +
-// l, so a wavefront's reads meet distinct banks) and one barrier.  The same
-// sums as gemv_wave_inflight: each product of an int8 and an f16 is exact in
-// binary32, so a pair's sum p0 + p1 is one fused multiply-add of the second
-// product onto the first (one rounding either way), the chain of four
-// (p0 + p1) + (p2 + p3).  Every wavefront reaches the barrier: rows past n
-// read row n - 1 and store nothing.
-template <int T, int R, int KPL>
-__device__ __forceinline__ void gemv_i8_xlds(const int8_t *__restrict__ w, const _Float16 *__restrict__ x,
-                                             const float *__restrict__ scale, float *__restrict__ y, uint32_t n,
-                                             uint32_t row0) {
-  constexpr int P = 16, C = 4;
-  constexpr uint32_t K = 64 * KPL * P;
-  constexpr uint32_t CH = K * 2 / 16;  // x's 16-byte chunks
-  constexpr int PER = CH / T;
-  static_assert(CH % T == 0, "x's chunks divide among the threads");
-  __shared__ uint4 xs[CH];
-  const uint32_t tid = threadIdx.x;
-  const uint32_t lane = tid & (FK_WAVE - 1);
+// One pack's products into its chains where each is exact in binary32 (int8 by
+// f16): a pair's sum p0 + p1 is one fused multiply-add of the second product
+// onto the first, one rounding either way.
+template <int P>
+__device__ __forceinline__ void add_pack_exact(float (&acc)[P / 4], const float (&xf)[P], const float (&wf)[P],
+                                               bool live) {
+#pragma unroll
+  for (int c = 0; c < P / 4; c++) {
+    const float s01 = __builtin_fmaf(xf[4 * c + 1], wf[4 * c + 1], xf[4 * c] * wf[4 * c]);
+    const float s23 = __builtin_fmaf(xf[4 * c + 3], wf[4 * c + 3], xf[4 * c + 2] * wf[4 * c + 2]);
+    const float sum = acc[c] + (s01 + s23);
+    acc[c] = live ? sum : acc[c];
+  }
+}
+
+// R rows of y = W x (times a per-row scale if given) by one wavefront, for
+// rows of at most 64 KPL packs: their loads all in flight, and x staged once a
+// threadgroup in `xs` (64 KPL XW chunks of 16 bytes, at least 256): read by
+// every wavefront from memory, x is as much traffic through a CU's L1 as f32
+// weights, and twice f16 ones.  The x loads first, then the rows' weights,
+// then x's chunks into LDS transposed (chunk u of lane l's pack it at
+// (XW it + u) 64 + l, so a wavefront's reads meet distinct banks) and one
+// barrier.  Every wavefront reaches it: rows past n read row n - 1 and store
+// nothing.  FULL: the row fills every lane's packs (k = 64 KPL P).  T: the
+// threadgroup's threads, 0 any.  (Wider rows a segment at a time lose to the
+// loop, whose wavefronts need not meet: f16 8192 x 8192 36 µs against 27.)
+template <typename WT, typename XT, int P, int R, int KPL, bool FULL, uint32_t T>
+__device__ __forceinline__ void gemv_xlds(const WT *__restrict__ w, const XT *__restrict__ x,
+                                          const float *__restrict__ scale, float *__restrict__ y, uint32_t n,
+                                          uint32_t k, uint32_t row0, uint4 *xs) {
+  constexpr int C = P / 4, XW = P * (int)sizeof(XT) / 16;
+  constexpr uint32_t PER = KPL * XW >= 4 ? KPL * XW / 4 : 1;  // a thread's chunks of x, of 256 threads
+  static_assert(P * sizeof(WT) == 16, "a W pack is one 16-byte load");
+  const uint32_t tid = threadIdx.x, threads = T ? T : blockDim.x, lane = tid & (FK_WAVE - 1);
+  const uint32_t packs = FULL ? FK_WAVE * KPL : k / P, chunks = packs * XW, width = packs * P;
+  const uint4 *const src = reinterpret_cast<const uint4 *>(x);
   uint4 xc[PER];
 #pragma unroll
-  for (int i = 0; i < PER; i++) xc[i] = reinterpret_cast<const uint4 *>(x)[tid + i * T];
+  for (uint32_t i = 0; i < PER; i++) xc[i] = src[FULL && T ? tid + i * T : min(tid + i * threads, chunks - 1)];
   uint4 wv[R][KPL];
 #pragma unroll
   for (int q = 0; q < R; q++) {
-    const int8_t *wr = w + (size_t)min(row0 + q, n - 1) * K;
+    const WT *const wr = w + (size_t)min(row0 + q, n - 1) * width;
 #pragma unroll
-    for (int it = 0; it < KPL; it++) wv[q][it] = load16<true>(wr + (size_t)(lane + FK_WAVE * it) * P);
+    for (int it = 0; it < KPL; it++) {
+      const uint32_t j = lane + FK_WAVE * (uint32_t)it;
+      wv[q][it] = load16<true>(wr + (size_t)(FULL ? j : min(j, packs - 1)) * P);
+    }
   }
+  auto put = [&](uint32_t j, const uint4 &v) {
+    const uint32_t pack = j / XW;
+    xs[(pack / FK_WAVE * XW + j % XW) * FK_WAVE + pack % FK_WAVE] = v;
+  };
+  // (Chunks past the row repeat its last one, where nothing is added.)
 #pragma unroll
-  for (int i = 0; i < PER; i++) {
-    const uint32_t j = tid + i * T, pack = j / 2;
-    xs[((pack / FK_WAVE) * 2 + j % 2) * FK_WAVE + pack % FK_WAVE] = xc[i];
-  }
+  for (uint32_t i = 0; i < PER; i++) put(tid + i * threads, xc[i]);
+  if constexpr (T == 0)
+    for (uint32_t j = tid + PER * threads; j < chunks; j += threads) put(j, src[j]);
   __syncthreads();
   float acc[R][C];
 #pragma unroll
@@ -379,19 +399,19 @@ __device__ __forceinline__ void gemv_i8_xlds(const int8_t *__restrict__ w, const
     for (int c = 0; c < C; c++) acc[q][c] = 0.0f;
 #pragma unroll
   for (int it = 0; it < KPL; it++) {
-    const uint4 xu[2] = {xs[(2 * it) * FK_WAVE + lane], xs[(2 * it + 1) * FK_WAVE + lane]};
+    // A pack past the row is computed from what LDS holds there and not added.
+    const bool live = FULL || lane + FK_WAVE * (uint32_t)it < packs;
+    uint4 xu[XW];
+#pragma unroll
+    for (int u = 0; u < XW; u++) xu[u] = xs[(XW * it + u) * FK_WAVE + lane];
     float xf[P];
-    unpack<P>(xu, xf, _Float16{});
+    unpack<P>(xu, xf, XT{});
 #pragma unroll
     for (int q = 0; q < R; q++) {
       float wf[P];
-      unpack_w<P>(wv[q][it], wf, int8_t{});
-#pragma unroll
-      for (int c = 0; c < C; c++) {
-        const float s01 = __builtin_fmaf(xf[4 * c + 1], wf[4 * c + 1], xf[4 * c] * wf[4 * c]);
-        const float s23 = __builtin_fmaf(xf[4 * c + 3], wf[4 * c + 3], xf[4 * c + 2] * wf[4 * c + 2]);
-        acc[q][c] = acc[q][c] + (s01 + s23);
-      }
+      unpack_w<P>(wv[q][it], wf, WT{});
+      if constexpr (sizeof(WT) == 1) add_pack_exact<P>(acc[q], xf, wf, live);
+      else add_pack<P>(acc[q], xf, wf, live);
     }
   }
   float t[R];
@@ -409,41 +429,131 @@ __device__ __forceinline__ void gemv_i8_xlds(const int8_t *__restrict__ w, const
   }
 }
 
+// The rows of a threadgroup: full rows, or by the fewest packs a lane that hold
+// the row (a pack past the row costs its products all the same); wider rows,
+// and int8 rows of up to two packs a lane (whose x is no more than the weights'
+// bytes), by the loop.  MI355X, µs, by the loads of KPL packs with x from
+// memory (int8: by the loop) and so:
+//
+//   f32 4096 x 256      6.3  2.7    f16 4096 x 256      5.1  2.6
+//       4096 x 1040     7.5  5.0        16384 x 512    15.1  6.2
+//       16384 x 2048   27.6 21.0        16384 x 2048   18.0 11.7
+//       5000 x 3088    12.7 12.1        5000 x 3088     9.2  8.5
+//       4096 x 4096    12.3 12.0        4096 x 4096     8.3  7.3
+//   i8  5000 x 3088     8.4  5.7    i8  4096 x 4096     7.7  5.0
+//       16384 x 512     6.2  6.8 (so the loop)
+template <typename WT, typename XT, int P, int R, int KPL>
+__device__ __forceinline__ void gemv_rows(const WT *__restrict__ w, const XT *__restrict__ x,
+                                          const float *__restrict__ scale, float *__restrict__ y, uint32_t n,
+                                          uint32_t k) {
+  __shared__ uint4 xs[FK_WAVE * KPL * P * sizeof(XT) / 16];
+  static_assert(sizeof xs >= 256 * 16, "a chunk a thread");
+  const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * R;
+  const uint32_t lanes = (k / P + FK_WAVE - 1) / FK_WAVE;  // packs a lane
+  if (lanes > KPL || (sizeof(WT) == 1 && lanes <= 2)) {
+    if (row0 < n) gemv_wave<WT, XT, P, R>(w, x, scale, y, n, k, row0);
+  } else if (blockDim.x != 256) {
+    gemv_xlds<WT, XT, P, R, KPL, false, 0>(w, x, scale, y, n, k, row0, xs);
+  } else if (k == FK_WAVE * KPL * P) {
+    gemv_xlds<WT, XT, P, R, KPL, true, 256>(w, x, scale, y, n, k, row0, xs);
+  } else if (lanes <= 1) {
+    gemv_xlds<WT, XT, P, R, 1, false, 256>(w, x, scale, y, n, k, row0, xs);
+  } else if (lanes <= 2) {
+    gemv_xlds<WT, XT, P, R, 2, false, 256>(w, x, scale, y, n, k, row0, xs);
+  } else if (lanes <= 4) {
+    gemv_xlds<WT, XT, P, R, 4, false, 256>(w, x, scale, y, n, k, row0, xs);
+  } else if (KPL > 8 && lanes <= 8) {
+    gemv_xlds<WT, XT, P, R, KPL < 8 ? KPL : 8, false, 256>(w, x, scale, y, n, k, row0, xs);
+  } else {
+    gemv_xlds<WT, XT, P, R, KPL, false, 256>(w, x, scale, y, n, k, row0, xs);
+  }
+}
+
+// A wavefront's row of more packs than gemv_xlds holds: the whole of x staged
+// once a threadgroup in `xs`, as there, then the row 8 packs a lane at a time,
+// the next 8 loaded before the last ones' products.
+template <typename WT, int P>
+__device__ __forceinline__ void gemv_wide(const WT *__restrict__ w, const float *__restrict__ x, float *__restrict__ y,
+                                          uint32_t n, uint32_t k, uint4 *xs) {
+  constexpr int C = P / 4, XW = P / 4, B = 8;
+  const uint32_t tid = threadIdx.x, lane = tid & (FK_WAVE - 1);
+  const uint32_t row = blockIdx.x * 4 + tid / FK_WAVE;
+  const uint32_t packs = k / P, chunks = packs * XW;
+  const WT *const wr = w + (size_t)min(row, n - 1) * k;
+  uint4 cur[B], nxt[B];
+#pragma unroll
+  for (int it = 0; it < B; it++) cur[it] = load16<true>(wr + (size_t)min(lane + FK_WAVE * (uint32_t)it, packs - 1) * P);
+#pragma unroll 4
+  for (uint32_t j = tid; j < chunks; j += 256) {
+    const uint32_t pack = j / XW;
+    xs[(pack / FK_WAVE * XW + j % XW) * FK_WAVE + pack % FK_WAVE] = reinterpret_cast<const uint4 *>(x)[j];
+  }
+  __syncthreads();
+  float acc[C];
+#pragma unroll
+  for (int c = 0; c < C; c++) acc[c] = 0.0f;
+  for (uint32_t base = 0; base < packs; base += B * FK_WAVE) {
+#pragma unroll
+    for (int it = 0; it < B; it++)
+      nxt[it] = load16<true>(wr + (size_t)min(base + lane + FK_WAVE * (uint32_t)(B + it), packs - 1) * P);
+#pragma unroll
+    for (int it = 0; it < B; it++) {
+      const uint32_t j = base + lane + FK_WAVE * (uint32_t)it, at = min(j, packs - 1);
+      uint4 xu[XW];
+#pragma unroll
+      for (int u = 0; u < XW; u++) xu[u] = xs[(at / FK_WAVE * XW + u) * FK_WAVE + at % FK_WAVE];
+      float xf[P], wf[P];
+      unpack<P>(xu, xf, float{});
+      unpack_w<P>(cur[it], wf, WT{});
+      add_pack<P>(acc, xf, wf, j < packs);
+    }
+#pragma unroll
+    for (int it = 0; it < B; it++) cur[it] = nxt[it];
+  }
+  float t = acc[0];
+#pragma unroll
+  for (int c = 1; c < C; c++) t = t + acc[c];
+  t = wave_sum(t);
+  if (lane == 0 && row < n) y[row] = t;
+}
+
 }  // namespace fk
 
-// Entry points: a threadgroup of W wavefronts takes W * R consecutive rows;
-// rows of at most 64 KPL packs take the all-in-flight form.
+// Entry points: a threadgroup of W wavefronts takes W * R consecutive rows.
 // Kernargs: the buffers in binding order, then the parameter struct.
 
-#define FK_GEMV_ENTRY(NAME, WT, XT, P, R, KPL)                                                                 \
+#define FK_GEMV_ENTRY(NAME, WT, XT, P, R, KPL)                                                               \
   extern "C" __global__ void __launch_bounds__(256) NAME(const WT *__restrict__ w, const XT *__restrict__ x, \
                                                          float *__restrict__ y, fk_gemv_params p) {         \
-    const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * (R);             \
-    if (row0 >= p.n) return;                                                                                 \
-    if (p.k / (P) == FK_WAVE * (KPL))                                                                        \
-      fk::gemv_wave_inflight<WT, XT, P, R, KPL, true>(w, x, nullptr, y, p.n, p.k, row0);                    \
-    else if (p.k / (P) < FK_WAVE * (KPL))                                                                    \
-      fk::gemv_wave_inflight<WT, XT, P, R, KPL, false>(w, x, nullptr, y, p.n, p.k, row0);                   \
-    else                                                                                                     \
-      fk::gemv_wave<WT, XT, P, R>(w, x, nullptr, y, p.n, p.k, row0);                                         \
+    fk::gemv_rows<WT, XT, P, R, KPL>(w, x, nullptr, y, p.n, p.k);                                            \
   }
 
-// The int8 entries: full rows of 64 KPL packs in threadgroups of 256 with x
-// staged in LDS (gemv_i8_xlds); other widths and threadgroups by the loop
-// form (which keeps the kernel's registers to what the staged form needs,
-// so that as many wavefronts as its LDS allows are resident).
-#define FK_GEMV_SCALED_ENTRY(NAME, WT, XT, P, R, KPL)                                                      \
-  extern "C" __global__ void __launch_bounds__(256)                                                        \
+// (WAVES a SIMD: int8 rows that the loop takes are short, and many at once.)
+#define FK_GEMV_SCALED_ENTRY(NAME, WT, XT, P, R, KPL, WAVES)                                               \
+  extern "C" __global__ void __launch_bounds__(256, WAVES)                                                 \
       NAME(const WT *__restrict__ w, const float *__restrict__ scale, const XT *__restrict__ x,            \
            float *__restrict__ y, fk_gemv_params p) {                                                      \
-    const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * (R);           \
-    if (p.k / (P) == FK_WAVE * (KPL) && blockDim.x == 256) {                                               \
-      fk::gemv_i8_xlds<256, R, KPL>(w, x, scale, y, p.n, row0);                                            \
-      return;                                                                                              \
-    }                                                                                                      \
-    if (row0 >= p.n) return;                                                                               \
-    fk::gemv_wave<WT, XT, P, R>(w, x, scale, y, p.n, p.k, row0);                                           \
+    fk::gemv_rows<WT, XT, P, R, KPL>(w, x, scale, y, p.n, p.k);                                            \
   }
+
+// f16 rows of more than 4096 columns, a row a wavefront, four a threadgroup.
+// Of 4096 rows or more, with x whole in LDS (its lanes of packs rounded up to
+// 64): through the L1 it is twice the weights' bytes.  Fewer leave the chip to
+// their latency, and x is met sooner where it lies.  MI355X, µs, by the loop
+// and so: 16384 x 8192 50.3, 43.8; 8192 x 6000 25.1, 21.0; 2048 x 8192 8.1,
+// 9.3; f32, whose weights are as wide as x: 83.
+extern "C" __global__ void __launch_bounds__(256)
+    fk_gemv_f16_f32_wide(const _Float16 *__restrict__ w, const float *__restrict__ x, float *__restrict__ y,
+                         fk_gemv_params p) {
+  extern __shared__ uint4 gemv_wide_xs[];
+  fk::gemv_wide<_Float16, 8>(w, x, y, p.n, p.k, gemv_wide_xs);
+}
+extern "C" __global__ void __launch_bounds__(256)
+    fk_gemv_f16_f32_loop(const _Float16 *__restrict__ w, const float *__restrict__ x, float *__restrict__ y,
+                         fk_gemv_params p) {
+  const uint32_t row = blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE;
+  if (row < p.n) fk::gemv_wave<_Float16, float, 8, 1>(w, x, nullptr, y, p.n, p.k, row);
+}
 
 // Rows whose width is a multiple of 4 but not of a 16-byte pack (the small
 // programs' linear layers): packs of 4 elements, the loop form.
@@ -495,6 +605,6 @@ FK_GEMV_ENTRY(fk_gemv_f32_f32_r4, float, float, 4, 4, 4)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r1, _Float16, float, 8, 1, 8)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r2, _Float16, float, 8, 2, 8)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r4, _Float16, float, 8, 4, 4)
-FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r1, int8_t, _Float16, 16, 1, 8)
-FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r2, int8_t, _Float16, 16, 2, 8)
-FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r4, int8_t, _Float16, 16, 4, 4)
+FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r1, int8_t, _Float16, 16, 1, 8, 8)
+FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r2, int8_t, _Float16, 16, 2, 8, 1)
+FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r4, int8_t, _Float16, 16, 4, 4, 1)

@@ -444,6 +444,7 @@ NORM_PACK_HELD = (512, 1024, 2048, 4096)
 
 ABIS: dict[str, KernelAbi] = {
     **_gemv_abis(),
+    **{e: KernelAbi(e, ("w", "x", "y"), GemvParams, 256) for e in ("fk_gemv_f16_f32_wide", "fk_gemv_f16_f32_loop")},
     "fk_rmsnorm_f32": KernelAbi("fk_rmsnorm_f32", ("x", "gamma", "y"), RmsNormParams),
     "fk_softmax_f32": KernelAbi("fk_softmax_f32", ("x", "y"), SoftmaxParams),
     "fk_fill_u32": KernelAbi("fk_fill_u32", ("dst",), FillParams),
@@ -520,6 +521,10 @@ ABIS: dict[str, KernelAbi] = {
     "fk_stream_read": KernelAbi("fk_stream_read", ("src", "out"), StreamReadParams),
 }
 
+# f16 matvecs (fk_gemv.h): the columns that a wavefront holds, the x that a
+# threadgroup holds whole in LDS, and the rows from which that pays.
+GEMV_HELD, GEMV_WIDE, GEMV_WIDE_ROWS = 4096, 16384, 4096
+
 # Elements a lane loads at once, by weight type: one 16-byte load of W.
 GEMV_PACK = {"f32": 4, "f16": 8, "i8": 16}
 ELEM_BYTES = {"f32": 4, "f16": 2, "i8": 1}
@@ -584,9 +589,20 @@ class Kernels:
                 raise LaunchError(f"{entry}: the int8 layer needs its per-row scales")
             _need(scale, n * 4, "scale", entry)
             bound["scale"] = scale.ptr
+        if wtype != "i8" and k <= GEMV_HELD:
+            # x is staged once a threadgroup: smaller ones than 256 stage it
+            # more often for the same sums (f16 4096 x 4096: of 64 threads
+            # 11.8 µs, of 256 7.5)
+            threads = 256
         rows_per_group = threads // WAVE * rows_per_wave
         groups = (n + rows_per_group - 1) // rows_per_group
-        self.launch(entry, groups, threads, bound, GemvParams(n, k), stream)
+        lds = 0
+        if wtype == "f16" and rows_per_wave == 1 and threads == 256 and k > GEMV_HELD:
+            if n >= GEMV_WIDE_ROWS and k <= GEMV_WIDE:
+                entry, lds = "fk_gemv_f16_f32_wide", -(-k // (64 * pack)) * 64 * pack * 4
+            else:
+                entry = "fk_gemv_f16_f32_loop"
+        self.launch(entry, groups, threads, bound, GemvParams(n, k), stream, lds)
 
     # C = A Bᵀ on the matrix cores (fk_gemm.h): the prefill GEMM.  256 × 256
     # tiles, K steps of 32 taken in pairs; LDS: a ring of 4 stages of A's and
