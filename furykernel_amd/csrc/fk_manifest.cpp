@@ -179,6 +179,8 @@ std::vector<Entry> build() {
          FK_P(S, factor, "f32"), FK_P(S, has_gamma, "u32")},
         sizeof(S));
   }
+  add("fk_softmax_f32_wide", 1024, {buf("x", "read", "f32"), buf("y", "write", "f32")},
+      {FK_P(fk_softmax_params, rows, "u32"), FK_P(fk_softmax_params, n, "u32")}, sizeof(fk_softmax_params));
   add("fk_softmax_f32", 0, {buf("x", "read", "f32"), buf("y", "write", "f32")},
       {FK_P(fk_softmax_params, rows, "u32"), FK_P(fk_softmax_params, n, "u32")}, sizeof(fk_softmax_params));
   add("fk_fill_u32", 0, {buf("dst", "write", "u32")},

@@ -13,6 +13,19 @@
 
 namespace fk {
 
+// block_reduce where `slots` is used once: its first round, one barrier, and
+// the second round by every wavefront for itself.
+template <bool IsMax>
+__device__ __forceinline__ float block_reduce_once(float v, float *slots) {
+  const uint32_t lane = threadIdx.x & (FK_WAVE - 1), waves = blockDim.x / FK_WAVE;
+  const float s = IsMax ? wave_max(v) : wave_sum(v);
+  if (lane == 0) slots[threadIdx.x / FK_WAVE] = s;
+  __syncthreads();
+  float acc = IsMax ? -__builtin_inff() : -0.0f;
+  if (lane < waves) acc = IsMax ? max_number(acc, slots[lane]) : acc + slots[lane];
+  return IsMax ? wave_max(acc) : wave_sum(acc);
+}
+
 // Segments of at most H packs a thread: the thread's packs (t, t + T, ...)
 // loaded into registers at once — every load issued before any is used, its
 // index clamped into the segment — and both passes made on the registers,
@@ -39,7 +52,7 @@ __device__ __forceinline__ void rmsnorm_held(const float *__restrict__ xs, const
     a = a + v[i].w * v[i].w;
     acc = t + i * T < packs ? a : acc;
   }
-  const float total = block_reduce<false>(acc, slots);
+  const float total = block_reduce_once<false>(acc, slots);
   const float scale = rsqrt_once(total / (float)p.seg + p.eps);
 #pragma unroll
   for (int i = 0; i < H; i++) {
@@ -85,7 +98,7 @@ extern "C" __global__ void __launch_bounds__(1024)
     acc = acc + v.z * v.z;
     acc = acc + v.w * v.w;
   }
-  const float total = fk::block_reduce<false>(acc, slots);
+  const float total = fk::block_reduce_once<false>(acc, slots);
   const float scale = fk::rsqrt_once(total / (float)p.seg + p.eps);
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
@@ -114,7 +127,7 @@ namespace fk {
 // sum in the loop's order, and the stores of e / sum.
 template <int H>
 __device__ __forceinline__ void softmax_held(const float *__restrict__ xs, float *__restrict__ ys, uint32_t packs,
-                                             float *slots) {
+                                             float *tops, float *slots) {
   const uint32_t T = blockDim.x, t = threadIdx.x;
   float4 v[H];
 #pragma unroll
@@ -128,7 +141,7 @@ __device__ __forceinline__ void softmax_held(const float *__restrict__ xs, float
     a = max_number(a, v[i].w);
     m = t + i * T < packs ? a : m;
   }
-  const float top = block_reduce<true>(m, slots);
+  const float top = block_reduce_once<true>(m, tops);
   float acc = -0.0f;
   float4 e[H];
 #pragma unroll
@@ -141,7 +154,7 @@ __device__ __forceinline__ void softmax_held(const float *__restrict__ xs, float
     a = a + e[i].w;
     acc = t + i * T < packs ? a : acc;
   }
-  const float total = block_reduce<false>(acc, slots);
+  const float total = block_reduce_once<false>(acc, slots);
 #pragma unroll
   for (int i = 0; i < H; i++) {
     if (t + i * T >= packs) break;
@@ -154,17 +167,17 @@ __device__ __forceinline__ void softmax_held(const float *__restrict__ xs, float
 
 extern "C" __global__ void __launch_bounds__(1024)
     fk_softmax_f32(const float *__restrict__ x, float *__restrict__ y, fk_softmax_params p) {
-  __shared__ float slots[16];
+  __shared__ float tops[16], slots[16];
   const uint32_t row = blockIdx.x;
   if (row >= p.rows) return;
   const float *xs = x + (size_t)row * p.n;
   float *ys = y + (size_t)row * p.n;
   const uint32_t packs = p.n / 4;
   const uint32_t held = (packs + blockDim.x - 1) / blockDim.x;  // packs a thread holds
-  if (held <= 1) return fk::softmax_held<1>(xs, ys, packs, slots);
-  if (held <= 2) return fk::softmax_held<2>(xs, ys, packs, slots);
-  if (held <= 4) return fk::softmax_held<4>(xs, ys, packs, slots);
-  if (held <= 8) return fk::softmax_held<8>(xs, ys, packs, slots);
+  if (held <= 1) return fk::softmax_held<1>(xs, ys, packs, tops, slots);
+  if (held <= 2) return fk::softmax_held<2>(xs, ys, packs, tops, slots);
+  if (held <= 4) return fk::softmax_held<4>(xs, ys, packs, tops, slots);
+  if (held <= 8) return fk::softmax_held<8>(xs, ys, packs, tops, slots);
   float m = -__builtin_inff();
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
@@ -173,7 +186,7 @@ extern "C" __global__ void __launch_bounds__(1024)
     m = fk::max_number(m, v.z);
     m = fk::max_number(m, v.w);
   }
-  const float top = fk::block_reduce<true>(m, slots);
+  const float top = fk::block_reduce_once<true>(m, tops);
   float acc = -0.0f;
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
@@ -182,11 +195,79 @@ extern "C" __global__ void __launch_bounds__(1024)
     acc = acc + fk::exp_once(v.z - top);
     acc = acc + fk::exp_once(v.w - top);
   }
-  const float total = fk::block_reduce<false>(acc, slots);
+  const float total = fk::block_reduce_once<false>(acc, slots);
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
     float4 o = make_float4(fk::exp_once(v.x - top) / total, fk::exp_once(v.y - top) / total,
                            fk::exp_once(v.z - top) / total, fk::exp_once(v.w - top) / total);
     *reinterpret_cast<float4 *>(ys + 4 * (size_t)j) = o;
   }
+}
+
+// The same rows, of up to 16384 elements, where they are few: 4 of the threads make what one of fk_softmax_f32's 256 does
+// (pack t + 256 i by thread t + 256 (i mod 4)), its exps meet in LDS and
+// threads 0 .. 255 sum theirs in the loop's order.  A row of 4096 alone on a
+// CU is bound by its own chain: 16 exps in binary64 a thread one wavefront a
+// SIMD, and their straight-line code, fetched once.  MI355X, µs, before and
+// so: 64 rows of 4096 4.9, 4.1; of 8192 7.2, 5.5; 4 of 16384 20.8, 8.2.
+#define FK_SOFTMAX_WIDE 16384
+
+namespace fk {
+
+template <int H>
+__device__ __forceinline__ void softmax_wide(const float *__restrict__ xs, float *__restrict__ ys, uint32_t packs,
+                                             float4 *es, float *tops, float *slots) {
+  constexpr uint32_t T = 256, N = 1024;
+  const uint32_t p = threadIdx.x, lane = p & (FK_WAVE - 1);
+  float4 v[H];
+#pragma unroll
+  for (int h = 0; h < H; h++) v[h] = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)min(p + h * N, packs - 1));
+  float m = -__builtin_inff();
+#pragma unroll
+  for (int h = 0; h < H; h++)  // (a pack past the row repeats its last one)
+    m = max_number(max_number(max_number(max_number(m, v[h].x), v[h].y), v[h].z), v[h].w);
+  const float top = block_reduce_once<true>(m, tops);
+#pragma unroll
+  for (int h = 0; h < H; h++) {
+    v[h] = make_float4(exp_once(v[h].x - top), exp_once(v[h].y - top), exp_once(v[h].z - top), exp_once(v[h].w - top));
+    es[p + h * N] = v[h];
+  }
+  __syncthreads();
+  if (p < T) {
+    float acc = -0.0f;
+#pragma unroll
+    for (int i = 0; i < 4 * H; i++) {
+      const float4 e = es[p + i * T];
+      float a = acc + e.x;
+      a = a + e.y;
+      a = a + e.z;
+      a = a + e.w;
+      acc = p + i * T < packs ? a : acc;
+    }
+    const float s = wave_sum(acc);
+    if (lane == 0) slots[p / FK_WAVE] = s;
+  }
+  __syncthreads();
+  const float total = wave_sum(lane < T / FK_WAVE ? -0.0f + slots[lane] : -0.0f);
+#pragma unroll
+  for (int h = 0; h < H; h++) {
+    if (p + h * N >= packs) break;
+    *reinterpret_cast<float4 *>(ys + 4 * (size_t)(p + h * N)) =
+        make_float4(v[h].x / total, v[h].y / total, v[h].z / total, v[h].w / total);
+  }
+}
+
+}  // namespace fk
+
+extern "C" __global__ void __launch_bounds__(1024)
+    fk_softmax_f32_wide(const float *__restrict__ x, float *__restrict__ y, fk_softmax_params p) {
+  __shared__ float4 es[FK_SOFTMAX_WIDE / 4];
+  __shared__ float tops[16], slots[4];
+  if (blockIdx.x >= p.rows) return;
+  const float *xs = x + (size_t)blockIdx.x * p.n;
+  float *ys = y + (size_t)blockIdx.x * p.n;
+  const uint32_t packs = p.n / 4;
+  if (packs <= 1024) fk::softmax_wide<1>(xs, ys, packs, es, tops, slots);
+  else if (packs <= 2048) fk::softmax_wide<2>(xs, ys, packs, es, tops, slots);
+  else fk::softmax_wide<4>(xs, ys, packs, es, tops, slots);
 }

@@ -447,6 +447,7 @@ ABIS: dict[str, KernelAbi] = {
     **{e: KernelAbi(e, ("w", "x", "y"), GemvParams, 256) for e in ("fk_gemv_f16_f32_wide", "fk_gemv_f16_f32_loop")},
     "fk_rmsnorm_f32": KernelAbi("fk_rmsnorm_f32", ("x", "gamma", "y"), RmsNormParams),
     "fk_softmax_f32": KernelAbi("fk_softmax_f32", ("x", "y"), SoftmaxParams),
+    "fk_softmax_f32_wide": KernelAbi("fk_softmax_f32_wide", ("x", "y"), SoftmaxParams, 1024),
     "fk_fill_u32": KernelAbi("fk_fill_u32", ("dst",), FillParams),
     **{e: KernelAbi(e, STEP_GEMV_BUFFERS, StepGemvParams, 512) for e in STEP_GEMV_ENTRIES},
     "fk_step_token": KernelAbi("fk_step_token", ("arg", "out", "token", "position"), StepTokenParams, 64),
@@ -524,6 +525,12 @@ ABIS: dict[str, KernelAbi] = {
 # f16 matvecs (fk_gemv.h): the columns that a wavefront holds, the x that a
 # threadgroup holds whole in LDS, and the rows from which that pays.
 GEMV_HELD, GEMV_WIDE, GEMV_WIDE_ROWS = 4096, 16384, 4096
+
+# Softmax rows that four times the threads make, in the same order (fk_rows.h):
+# more than 2048 elements (64 rows of 2048: 3.65 µs, so 3.73; of 4096 4.9, 4.1),
+# up to what LDS holds, and at most 512 rows, past which the chip is full
+# without (512 of 16384 31.8, 18.6; 1024 of 4096 10.4, 10.1).
+SOFTMAX_WIDE_FROM, SOFTMAX_WIDE, SOFTMAX_WIDE_ROWS = 2048, 16384, 512
 
 # Elements a lane loads at once, by weight type: one 16-byte load of W.
 GEMV_PACK = {"f32": 4, "f16": 8, "i8": 16}
@@ -788,6 +795,8 @@ class Kernels:
             raise LaunchError(f"{entry}: {threads} threads is not 1 to 16 wavefronts")
         _need(x, rows * n * 4, "x", entry)
         _need(y, rows * n * 4, "y", entry)
+        if threads == 256 and SOFTMAX_WIDE_FROM < n <= SOFTMAX_WIDE and rows <= SOFTMAX_WIDE_ROWS:
+            entry, threads = "fk_softmax_f32_wide", 1024
         self.launch(entry, rows, threads, {"x": x.ptr, "y": y.ptr}, SoftmaxParams(rows, n), stream)
 
 
