@@ -450,12 +450,12 @@ __device__ __forceinline__ void gemv_rows(const WT *__restrict__ w, const XT *__
   static_assert(sizeof xs >= 256 * 16, "a chunk a thread");
   const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * R;
   const uint32_t lanes = (k / P + FK_WAVE - 1) / FK_WAVE;  // packs a lane
-  if (lanes > KPL || (sizeof(WT) == 1 && lanes <= 2)) {
+  if (k == FK_WAVE * KPL * P && blockDim.x == 256) {
+    gemv_xlds<WT, XT, P, R, KPL, true, 256>(w, x, scale, y, n, k, row0, xs);
+  } else if (lanes > KPL || (sizeof(WT) == 1 && lanes <= 2)) {
     if (row0 < n) gemv_wave<WT, XT, P, R>(w, x, scale, y, n, k, row0);
   } else if (blockDim.x != 256) {
     gemv_xlds<WT, XT, P, R, KPL, false, 0>(w, x, scale, y, n, k, row0, xs);
-  } else if (k == FK_WAVE * KPL * P) {
-    gemv_xlds<WT, XT, P, R, KPL, true, 256>(w, x, scale, y, n, k, row0, xs);
   } else if (lanes <= 1) {
     gemv_xlds<WT, XT, P, R, 1, false, 256>(w, x, scale, y, n, k, row0, xs);
   } else if (lanes <= 2) {
