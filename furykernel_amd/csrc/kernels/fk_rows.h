@@ -204,9 +204,10 @@ extern "C" __global__ void __launch_bounds__(1024)
   }
 }
 
-// The same rows, of up to 16384 elements, where they are few: 4 of the threads make what one of fk_softmax_f32's 256 does
-// (pack t + 256 i by thread t + 256 (i mod 4)), its exps meet in LDS and
-// threads 0 .. 255 sum theirs in the loop's order.  A row of 4096 alone on a
+// The same rows, of up to 16384 elements, where they are few: 4 of the
+// threads make what one of fk_softmax_f32's 256 does (pack t + 256 i by
+// thread t + 256 (i mod 4)), its exps meet in LDS and threads 0 .. 255 sum
+// theirs in the loop's order.  A row of 4096 alone on a
 // CU is bound by its own chain: 16 exps in binary64 a thread one wavefront a
 // SIMD, and their straight-line code, fetched once.  MI355X, µs, before and
 // so: 64 rows of 4096 4.9, 4.1; of 8192 7.2, 5.5; 4 of 16384 20.8, 8.2.
