@@ -41,7 +41,7 @@ the sequence rows of a step).
 from __future__ import annotations
 
 from collections import defaultdict
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import Optional
 
 import numpy as np
@@ -96,13 +96,28 @@ def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Opti
     _Prefill(out, run_rows, scratch_slot).run()
     _fuse_qkv_rope(out)
     _fuse_argmax(out)
-    live = live or LiveRows(rows // 16, rows // 16, rows)
+    live = _whole_blocks(out, live or LiveRows(rows // 16, rows // 16, rows))
     _skinny_gemms(out, live)
     _rows_norms(out, live)
     _row_attention(out, live)
     _split_attention(out, live)
     _compact(out, live)
     return out
+
+
+def _whole_blocks(out: Lowered, live: LiveRows) -> LiveRows:
+    """The rows a step has to make: the live ones, and where its KV stores are
+    staged the rest of their query blocks too.  The attention loads its run's
+    staging rows up to a block's last query; the rows past the live ones are
+    masked, but a probability of 0 times what was never written there may be
+    NaN.  (In place those rows' positions lie in the ring, which holds what it
+    held before the step.)"""
+    if not any(L.entry in ATTEND_FORMS and L.params.get("staged") for L in out.launches):
+        return live
+    if live.apart != 1:
+        return LiveRows(out.rows // 16, out.rows // 16, out.rows)
+    run_chunks = -(-live.run_chunks * 16 // QBLOCK) * QBLOCK // 16
+    return replace(live, chunks=-(-live.chunks // live.run_chunks) * run_chunks, run_chunks=run_chunks)
 
 
 def attend_parts(pairs: int, length: int) -> int:
