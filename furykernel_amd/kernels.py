@@ -407,36 +407,73 @@ ATTEND_FORMS.update({f"fk_split_attend_{form}h{h}k{k}": 64 * h * k for form in (
                      for h, k in ATTEND_SPLITS})
 
 
-def attend_launch(form: str, rows: int, heads: int, kv_heads: int, keys: int) -> tuple[str, int, int]:
+# Where each split form is taken, by the query heads a kv head, tried in order:
+# (heads a group, groups), the most pairs of a block of 32 rows and a head, and
+# with a window the most pairs and the least window.  See attend_launch.
+ATTEND_RULE = {1: (((1, 4), 511, 256, 128), ((1, 2), 1024, 512, 256)),
+               2: (((1, 4), 256, 256, 128), ((2, 4), 767, 512, 128), ((2, 2), 2559, 1024, 256)),
+               4: (((1, 4), 256, 256, 128), ((2, 4), 767, 512, 128), ((2, 2), 1279, 1024, 512))}
+ATTEND_RULE_BF16 = {1: (((1, 4), 767, 256, 1), ((1, 2), 1024, 512, 1)),
+                    2: (((2, 4), 767, 512, 1), ((2, 2), 2559, 1024, 1)),
+                    4: (((2, 4), 767, 512, 128), ((4, 2), 1279, 1024, 256))}
+ATTEND_RULE_MANY = ((4, 2), 2559, 2048, 1024)  # 4 heads, past those
+
+
+def attend_launch(form: str, rows: int, heads: int, kv_heads: int, keys: int, window: int = 0, bf16: bool = False,
+                  prompts: bool = False) -> tuple[str, int, int]:
     """The entry, threadgroups and threads of the prefill attention of `rows`
     rows ("", "f16_", "paged_", "paged_f16_": where its keys come from), the
-    rows' positions below `keys`.
+    rows' positions below `keys`, over `bf16` caches or f16 ones; `prompts`:
+    the rows are taken to be sequences' first `keys` ones.
 
     A wavefront takes a block of 32 rows and a query head and walks the
     block's keys, 64 at a time; few such pairs leave SIMDs idle (1024 on the
     chip, and up to four wavefronts a SIMD to hide a block's latency), so
-    below 2560 their keys are split among groups of wavefronts
-    (fk_split_attend_*): in two, below 768 in four (all the LDS of a CU); and
-    below 1280 the heads of a kv head go to threadgroups of their own, for
-    256 or more.  MI355X, f16, 8 kv heads of 4, µs unsplit and split:
+    their keys are split among groups of wavefronts (fk_split_attend_*), 32
+    KB of LDS a group: in four while a threadgroup a CU holds the pairs, in
+    two while two a CU do; and the heads of a kv head go to threadgroups of
+    their own, for 256 or more.  MI355X, f16, 8 kv heads of 4, µs unsplit and
+    split:
 
     - 256 rows from position 3000 (256 pairs): 48.0, h1k4 22.9, h4k2 36.4;
     - 512 from 3072: 52.1, h2k4 25.9, h1k4 43.2; from 0: 11.0, h2k4 8.7;
     - 1024 from 0: 18.5, h2k2 13.6, h4k2 15.8; from 3072: 59.5, 46.9, 46.7;
     - 2048 from 0 (2048 pairs): 36.6, h4k2 31.3, h2k2 34.7;
-    - 2 x 1536 (3072 pairs): 32.0, h4k2 33.5.
+    - 2 x 1536 (3072 pairs): 32.0, h4k2 33.5;
+    - 8 kv heads of one, 2 x 1792 from 2048 (896 pairs): 55.5, h1k2 55.3; 4
+      of one, 2048 pairs, h1k2 at 0.80 to 0.93 of unsplit's speed.
+
+    The blocks of a sequence's first rows differ in their keys and fill in
+    behind each other, so there a second round costs little; those of a
+    window are all the same, so a form has to hold them at once, and a window
+    of few blocks leaves nothing to split.  From 2048, 512 rows: window 64
+    6.4, h2k4 6.3; 256 8.9, 8.2; 512 12.2, 9.5.  2048 rows: window 256 12.4,
+    h4k2 13.0; 512 17.6, 17.6; 1024 28.1, 26.5.  1536 rows of 4 kv heads of 2
+    (384 pairs), window 256: 8.5, h1k4 14.2, h2k4 7.9.
+
+    Rows that go through registers (bf16 ones, converted by the group that
+    takes them; f16 ones of staged steps) share the work of a group's heads:
+    bf16, 512 rows from 2048, 54.1, h2k4 31.4, h1k4 63.3.  Their h4k2 holds a
+    threadgroup a CU, so past 1280 pairs it is for `prompts` alone (bf16, 2 x
+    768 from 0 20.7, h4k2 17.5; from 2048 73.1, 76.5).
 
     Fewer than eight blocks of keys stay: their merge would cost what the
-    split saves (256 rows from 0: 7.8, at best 6.7).  The rule is the same
-    for every place that the keys come from, so that staged, paged and ring
+    split saves (256 rows from 0: 7.8, at best 6.7); past 1280 pairs eight do
+    too (4 x 512 from 0: 12.4, h4k2 12.8).  The rule is the same for every
+    place that a session's keys come from, so that its staged, paged and ring
     steps of one shape agree bit for bit."""
     g = heads // kv_heads
     pairs = rows // 32 * heads
-    if pairs >= 2560 or keys < 8 * ATTEND_KEYS:
-        return f"fk_prefill_attend_{form}g{g}", rows // 32 * kv_heads, 64 * g
-    h = g if pairs >= 1280 else min(g, 2) if pairs >= 512 else 1
-    k = 2 if pairs >= 768 else 4
-    return f"fk_split_attend_{form}h{h}k{k}", pairs // h, 64 * h * k
+    rule = (ATTEND_RULE_BF16 if bf16 else ATTEND_RULE)[g]
+    if g == 4 and keys > 8 * ATTEND_KEYS and (prompts or "f16" in form):
+        rule += (ATTEND_RULE_MANY,)
+    if keys >= 8 * ATTEND_KEYS:
+        for (h, k), most, most_windowed, least in rule:
+            if pairs <= (most_windowed if window else most):
+                if window and window < least:
+                    break
+                return f"fk_split_attend_{form}h{h}k{k}", pairs // h, 64 * h * k
+    return f"fk_prefill_attend_{form}g{g}", rows // 32 * kv_heads, 64 * g
 
 
 # Row widths the one-pass RMSNorm-to-tiles holds in registers (fk_prefill.h).
@@ -745,7 +782,7 @@ class Kernels:
         _need(out, rows * heads * 64 * 2, "out", entry)
         bound = {"qr": qr.ptr, "kc": kc.ptr, "vc": vc.ptr, "position": position.ptr, "slot": slot.ptr, "out": out.ptr,
                  "ks": 0, "vs": 0}
-        entry, groups, threads = attend_launch(form, rows, heads, kv_heads, length)
+        entry, groups, threads = attend_launch(form, rows, heads, kv_heads, length, window, cache_bf16)
         self.launch(entry, groups, threads, bound,
                     PrefillAttendParams(rows, heads, kv_heads, length, slots, window, int(cache_bf16), scale), stream)
 

@@ -73,7 +73,10 @@ class LiveRows:
     run: int
     apart: int = 1
     count: Optional[int] = None  # the rows themselves, where the last chunk is not whole
-    keys: Optional[int] = None   # their positions are below it, where that is known
+    # Where they are sequences' runs of rows: the run's.  The attention's form is
+    # picked as for a run's first positions, also for a step that is moved to
+    # later ones, so that it is the same whatever their bound.
+    keys: Optional[int] = None
 
 
 def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Optional[int] = None,
@@ -170,8 +173,10 @@ def _split_attention(out: Lowered, live: LiveRows) -> None:
         if at.entry in ATTEND_FORMS:
             p = at.params
             form = at.entry[len("fk_prefill_attend_"):at.entry.rindex("g")]
-            at.entry, at.groups, at.threads = attend_launch(form, p["rows"], p["heads"], p["kv_heads"],
-                                                            min(live.keys or p["length"], p["length"]))
+            keys = min(live.keys or p["length"], p["length"])
+            at.entry, at.groups, at.threads = attend_launch(form, p["rows"], p["heads"], p["kv_heads"], keys,
+                                                            p["window"], bool(p["cache_bf16"]),
+                                                            prompts=live.keys is not None)
 
 
 # What a tile of each form of fk_skinny costs a CU: µs a tile and a step of 32
