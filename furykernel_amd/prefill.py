@@ -77,6 +77,13 @@ class LiveRows:
     # picked as for a run's first positions, also for a step that is moved to
     # later ones, so that it is the same whatever their bound.
     keys: Optional[int] = None
+    # Where a step makes more rows than are read (_whole_blocks): the chunks
+    # that its forms are picked by, those that are.
+    picks: Optional[int] = None
+
+    @property
+    def picked(self) -> int:
+        return self.chunks if self.picks is None else self.picks
 
 
 def lower_prefill(checked: CheckedProgram, plan: Plan, rows: int, run_rows: Optional[int] = None,
@@ -114,13 +121,15 @@ def _whole_blocks(out: Lowered, live: LiveRows) -> LiveRows:
     staging rows up to a block's last query; the rows past the live ones are
     masked, but a probability of 0 times what was never written there may be
     NaN.  (In place those rows' positions lie in the ring, which holds what it
-    held before the step.)"""
+    held before the step.)  The forms stay those of the live rows, so that a
+    staged step is the in-place one of the same rows bit for bit."""
     if not any(L.entry in ATTEND_FORMS and L.params.get("staged") for L in out.launches):
         return live
     if live.apart != 1:
         return LiveRows(out.rows // 16, out.rows // 16, out.rows)
     run_chunks = -(-live.run_chunks * 16 // QBLOCK) * QBLOCK // 16
-    return replace(live, chunks=-(-live.chunks // live.run_chunks) * run_chunks, run_chunks=run_chunks)
+    return replace(live, chunks=-(-live.chunks // live.run_chunks) * run_chunks, run_chunks=run_chunks,
+                   picks=live.chunks)
 
 
 def attend_parts(pairs: int, length: int) -> int:
@@ -251,7 +260,7 @@ def _skinny_gemms(out: Lowered, live: LiveRows) -> None:
         norm = out.launches[i + 1] if mode == "add" and i + 1 < len(out.launches) else None
         if norm is not None and not (_rows_norm_of(norm, live) and norm.bind["x"] == gm.bind["c0"]):
             norm = None
-        picked = skinny_form(live.chunks, p["m"], n, p["k"], mode, (1, 2, 4, 8) if norm else (1,))
+        picked = skinny_form(live.picked, p["m"], n, p["k"], mode, (1, 2, 4, 8) if norm else (1,))
         if picked is None:
             continue
         form, split = picked
@@ -290,7 +299,7 @@ ROWS_NORM_CHUNKS = 128
 
 def _rows_norm_of(launch: Launch, live: LiveRows) -> bool:
     """Whether fk_rows_norm can take the place of `launch`."""
-    return live.chunks <= ROWS_NORM_CHUNKS and launch.entry.startswith("fk_prefill_norm_pack_w") and \
+    return live.picked <= ROWS_NORM_CHUNKS and launch.entry.startswith("fk_prefill_norm_pack_w") and \
         launch.params["width"] in ROWS_NORM_THREADS
 
 
@@ -328,7 +337,7 @@ def _rows_norms(out: Lowered, live: LiveRows) -> None:
                 gone.append(before)
             else:
                 _to_rows_norm(norm, live, norm.params["rows"], {"x": x}, source=ROWS_STORED)
-        elif norm.entry == "fk_prefill_argmax_keys" and live.chunks <= ROWS_NORM_CHUNKS:
+        elif norm.entry == "fk_prefill_argmax_keys" and live.picked <= ROWS_NORM_CHUNKS:
             made = next(L for L in reversed(out.launches[:i]) if L.bind.get("keys") == norm.bind["keys"])
             if made.entry.startswith("fk_skinny_"):
                 norm.entry, norm.groups, norm.threads = "fk_rows_token", live.chunks * 16, 256

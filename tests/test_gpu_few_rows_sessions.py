@@ -80,24 +80,22 @@ def test_staged_prefills_read_only_rows_they_made(device, kernels, seqs, rows):
         s.close()
 
 
-def test_a_staged_prefill_is_the_in_place_one_bit_for_bit(device, kernels):
-    """100 rows staged, and in place the same 100 and 28 more of token 0
-    (what fills the staged step's query blocks): the same rows made by the
-    same forms."""
-    tokens = np.zeros(128, np.int64)
-    tokens[:100] = np.random.default_rng(1).integers(0, DIMS.vocab, 100)
+@pytest.mark.parametrize("seqs,rows", [(1, 100), (1, 9), (2, 70), (1, 400)])
+def test_a_staged_prefill_is_the_in_place_one_bit_for_bit(device, kernels, seqs, rows):
+    """The rows that a staged step makes past the live ones change no form."""
+    tokens = np.random.default_rng(rows).integers(0, DIMS.vocab, seqs * rows)
     got = []
-    for rows, bound in ((100, DIMS.context), (128, None)):
-        s = open_session(device, kernels, 1, rows, bound=bound)
+    for bound in (DIMS.context, None):
+        s = open_session(device, kernels, seqs, rows, bound=bound)
         try:
             assert s.staged == (bound is not None)
-            s.set_tokens(tokens[:rows])
-            print(f"prefill 1 x {rows}, staged {s.staged}", flush=True)
+            s.set_tokens(tokens)
+            print(f"prefill {seqs} x {rows}, staged {s.staged}", flush=True)
             s.run()
             device.sync()
             held = caches_of(s, s.dims)
-            got.append((s.logits()[:100], s.tokens()[:100],
-                        [held[n][0].reshape(8, -1, 64)[:, :100] for n in sorted(held)]))
+            got.append((s.logits(), s.tokens(),
+                        [held[n][u].reshape(8, -1, 64)[:, :rows] for n in sorted(held) for u in range(seqs)]))
         finally:
             s.close()
     (la, ta, ca), (lb, tb, cb) = got

@@ -83,7 +83,7 @@ def prefill(dims, seqs, seq_rows, layers, **kw):
     chunks = -(-seq_rows // 16)
     c = check_program(decoder_step(dims, layers=layers, **kw))
     return lower_prefill(c, plan(PlanOptions(sequence_rows=seq_rows), c), rows, run, True,
-                         LiveRows(seqs * chunks, chunks, run)), real, rows
+                         LiveRows(seqs * chunks, chunks, run, keys=run)), real, rows
 
 
 # Every count up to past a run of 256 rows' query blocks, and rows on both
@@ -131,3 +131,15 @@ def test_in_place_steps_make_their_real_rows():
             low, real, rows = prefill(ONE_B, seqs, seq_rows, 2, position_bound=seq_rows, **kw)
             made, staged = made_rows(low, rows)
             assert staged == 0 and made["value:logits"][real].all()
+
+
+@pytest.mark.parametrize("seqs", [1, 2])
+def test_a_staged_step_takes_the_in_place_ones_forms(seqs):
+    """Whatever the rows that it makes beside the live ones, so that the two
+    agree bit for bit: the same launches but for where keys and values go."""
+    for seq_rows in ROWS:
+        steps = [prefill(ONE_B, seqs, seq_rows, 2, position_bound=bound)[0] for bound in (seq_rows, 4096)]
+        entries = [[L.entry.replace("_attend_f16_", "_attend_") for L in low.launches if L.entry != "fk_prefill_land"]
+                   for low in steps]
+        parts = [[L.params.get("parts") for L in low.launches if L.entry.startswith("fk_skinny")] for low in steps]
+        assert entries[0] == entries[1] and parts[0] == parts[1], seq_rows
