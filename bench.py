@@ -469,9 +469,10 @@ def main_kernels(args) -> int:
     best = None
     for r, t in gemv_variants("f32", n, k):
         us = timed([lambda w=w, r=r, t=t: ks.gemv(w, x, y, n, k, "f32", rows_per_wave=r, threads=t) for w in ws], 20)
-        log(f"fk_gemv_f32_f32_r{r} 4096 x 4096, {t} threads: {us:.2f} us a launch, {nbytes / us / 1e3:.1f} GB/s")
+        entry = kernels.gemv_launch("f32", n, k, r, t)[0]
+        log(f"{entry} 4096 x 4096, {t} threads: {us:.2f} us a launch, {nbytes / us / 1e3:.1f} GB/s")
         if best is None or us < best[1]:
-            best = (f"fk_gemv_f32_f32_r{r}", us)
+            best = (entry, us)
     table["matvec_f32_4096x4096"] = {"kernel": best[0], "avg_us": round(best[1], 3), "bytes": nbytes,
                                      "gbps": round(nbytes / best[1] / 1e3, 1),
                                      "frac": round(nbytes / best[1] / 1e3 / HBM_PEAK_GBPS, 4)}
@@ -485,18 +486,19 @@ def main_kernels(args) -> int:
         normal(b, 300 + i, False)
     normal(gamma, 298, False)
     bufs += xs + [gamma, out]
-    for name, entry, run, nb in (
-            ("rmsnorm_64x4096", "fk_rmsnorm_f32", lambda b, t: ks.rmsnorm(b, gamma, out, rows, width, threads=t),
-             2 * rows * width * 4 + width * 4),
-            ("softmax_64x4096", "fk_softmax_f32", lambda b, t: ks.softmax(b, out, rows, width, threads=t),
-             2 * rows * width * 4)):
+    for name, launched, run, nb in (
+            ("rmsnorm_64x4096", lambda t: ("fk_rmsnorm_f32", t),
+             lambda b, t: ks.rmsnorm(b, gamma, out, rows, width, threads=t), 2 * rows * width * 4 + width * 4),
+            ("softmax_64x4096", lambda t: kernels.softmax_launch(rows, width, t),
+             lambda b, t: ks.softmax(b, out, rows, width, threads=t), 2 * rows * width * 4)):
         best = None
         for t in (256, 512, 1024):
             us = timed([lambda b=b, t=t: run(b, t) for b in xs], 20)
+            entry, t = launched(t)
             log(f"{entry} 64 x 4096, {t} threads a row: {us:.2f} us a launch, {nb / us / 1e3:.1f} GB/s")
-            if best is None or us < best[1]:
-                best = (t, us)
-        t, us = best
+            if best is None or us < best[2]:
+                best = (entry, t, us)
+        entry, t, us = best
         table[name] = {"kernel": entry, "threads": t, "avg_us": round(us, 3), "bytes": nb,
                        "gbps": round(nb / us / 1e3, 1), "frac": round(nb / us / 1e3 / HBM_PEAK_GBPS, 4)}
 
@@ -515,9 +517,10 @@ def main_kernels(args) -> int:
     for r, t in gemv_variants("i8", n, k):
         us = timed([lambda w=w, r=r, t=t: ks.gemv(w, xh, yi, n, k, "i8", rows_per_wave=r, threads=t, scale=scale)
                     for w in wi], 20)
-        log(f"fk_gemv_i8_f16_r{r} 8192 x 8192, {t} threads: {us:.2f} us a launch, {nbytes / us / 1e3:.1f} GB/s")
+        entry = kernels.gemv_launch("i8", n, k, r, t)[0]
+        log(f"{entry} 8192 x 8192, {t} threads: {us:.2f} us a launch, {nbytes / us / 1e3:.1f} GB/s")
         if best is None or us < best[1]:
-            best = (f"fk_gemv_i8_f16_r{r}", us)
+            best = (entry, us)
     table["matvec_i8_8192x8192"] = {"kernel": best[0], "avg_us": round(best[1], 3), "bytes": nbytes,
                                     "gbps": round(nbytes / best[1] / 1e3, 1),
                                     "frac": round(nbytes / best[1] / 1e3 / HBM_PEAK_GBPS, 4)}

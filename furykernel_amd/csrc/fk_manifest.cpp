@@ -162,9 +162,13 @@ std::vector<Entry> build() {
       add(std::string("fk_gemv_") + wt + "_f32_r" + std::to_string(r), 0,
           {buf("w", "read", wt), buf("x", "read", "f32"), buf("y", "write", "f32")},
           {FK_P(fk_gemv_params, n, "u32"), FK_P(fk_gemv_params, k, "u32")}, sizeof(fk_gemv_params));
-  for (const char *name : {"fk_gemv_f16_f32_wide", "fk_gemv_f16_f32_loop"})
-    add(name, 256, {buf("w", "read", "f16"), buf("x", "read", "f32"), buf("y", "write", "f32")},
-        {FK_P(fk_gemv_params, n, "u32"), FK_P(fk_gemv_params, k, "u32")}, sizeof(fk_gemv_params));
+  for (const char *wt : {"f32", "f16"})
+    for (int r : {1, 2, 4})
+      add(std::string("fk_gemv_") + wt + "_f32_staged_r" + std::to_string(r), 256,
+          {buf("w", "read", wt), buf("x", "read", "f32"), buf("y", "write", "f32")},
+          {FK_P(fk_gemv_params, n, "u32"), FK_P(fk_gemv_params, k, "u32")}, sizeof(fk_gemv_params));
+  add("fk_gemv_f16_f32_wide", 256, {buf("w", "read", "f16"), buf("x", "read", "f32"), buf("y", "write", "f32")},
+      {FK_P(fk_gemv_params, n, "u32"), FK_P(fk_gemv_params, k, "u32")}, sizeof(fk_gemv_params));
   for (const char *wt : {"f32", "f16", "bf16"})
     add(std::string("fk_gemv_p4_") + wt, 0, {buf("w", "read", wt), buf("x", "read", "f32"), buf("y", "write", "f32")},
         {FK_P(fk_gemv_params, n, "u32"), FK_P(fk_gemv_params, k, "u32")}, sizeof(fk_gemv_params));
@@ -809,16 +813,25 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
                  threads);
     need = {{"w", (uint64_t)p.ranks * 4}, {"x", (uint64_t)p.ranks * p.seg * 4}, {"y", (uint64_t)p.seg * 4}};
     if (p.residual) need.push_back({"res", (uint64_t)p.seg * 4});
-  } else if (std::strcmp(entry, "fk_gemv_f16_f32_wide") == 0 || std::strcmp(entry, "fk_gemv_f16_f32_loop") == 0) {
+  } else if (std::strcmp(entry, "fk_gemv_f16_f32_wide") == 0) {
     fk_gemv_params p;
     std::memcpy(&p, params, sizeof p);
-    // a wavefront a row, four a threadgroup; wide: x's lanes of packs in LDS
-    const bool wide = std::strcmp(entry + 16, "wide") == 0;
-    if (p.n == 0 || p.k == 0 || p.k % 8 || (uint64_t)groups * 4 < p.n ||
-        (wide && (p.k > 16384 || lds_bytes < (p.k + 511) / 512 * 512 * 4)))
+    // a wavefront a row, four a threadgroup; x's lanes of packs in LDS
+    if (p.n == 0 || p.k == 0 || p.k % 8 || (uint64_t)groups * 4 < p.n || p.k > 16384 ||
+        lds_bytes < (p.k + 511) / 512 * 512 * 4)
       return bad(err, cap, FK_ERR_ARG, "%s: %u rows of %u in %u groups, %u bytes of LDS", entry, p.n, p.k, groups,
                  lds_bytes);
     need = {{"w", (uint64_t)p.n * p.k * 2}, {"x", (uint64_t)p.k * 4}, {"y", (uint64_t)p.n * 4}};
+  } else if (std::strncmp(entry, "fk_gemv_f32_f32_staged_r", 24) == 0 ||
+             std::strncmp(entry, "fk_gemv_f16_f32_staged_r", 24) == 0) {
+    fk_gemv_params p;
+    std::memcpy(&p, params, sizeof p);
+    // r rows a wavefront, four wavefronts; a row's packs held by its lanes
+    const bool f16 = entry[9] == '1';
+    const uint32_t r = (uint32_t)(entry[24] - '0'), pack = f16 ? 8 : 4, held = r == 4 ? (f16 ? 2048 : 1024) : 4096;
+    if (p.n == 0 || p.k == 0 || p.k % pack || p.k > held || groups * 4ull * r < p.n)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u rows of %u in %u groups", entry, p.n, p.k, groups);
+    need = {{"w", (uint64_t)p.n * p.k * (f16 ? 2 : 4)}, {"x", (uint64_t)p.k * 4}, {"y", (uint64_t)p.n * 4}};
   } else if (std::strncmp(entry, "fk_gemv_p4_", 11) == 0) {
     fk_gemv_params p;
     std::memcpy(&p, params, sizeof p);

@@ -477,11 +477,10 @@ __device__ __forceinline__ void gemv_xlds(const WT *__restrict__ w, const XT *__
   }
 }
 
-// The rows of a threadgroup: full rows, or by the fewest packs a lane that hold
-// the row (a pack past the row costs its products all the same); wider rows,
-// and int8 rows of up to two packs a lane (whose x is no more than the weights'
-// bytes), by the loop.  MI355X, µs, by the loads of KPL packs with x from
-// memory (int8: by the loop) and so:
+// The rows of a threadgroup of 256 threads, at most 64 KPL packs each: full
+// rows, or by the fewest packs a lane that hold the row (a pack past the row
+// costs its products all the same).  MI355X, µs, by the loads of KPL packs with
+// x from memory (int8: by the loop) and so:
 //
 //   f32 4096 x 256      6.3  2.7    f16 4096 x 256      5.1  2.6
 //       4096 x 1040     7.5  5.0        16384 x 512    15.1  6.2
@@ -489,21 +488,13 @@ __device__ __forceinline__ void gemv_xlds(const WT *__restrict__ w, const XT *__
 //       5000 x 3088    12.7 12.1        5000 x 3088     9.2  8.5
 //       4096 x 4096    12.3 12.0        4096 x 4096     8.3  7.3
 //   i8  5000 x 3088     8.4  5.7    i8  4096 x 4096     7.7  5.0
-//       16384 x 512     6.2  6.8 (so the loop)
 template <typename WT, typename XT, int P, int R, int KPL>
-__device__ __forceinline__ void gemv_rows(const WT *__restrict__ w, const XT *__restrict__ x,
-                                          const float *__restrict__ scale, float *__restrict__ y, uint32_t n,
-                                          uint32_t k) {
-  __shared__ uint4 xs[FK_WAVE * KPL * P * sizeof(XT) / 16];
-  static_assert(sizeof xs >= 256 * 16, "a chunk a thread");
-  const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * R;
+__device__ __forceinline__ void gemv_staged(const WT *__restrict__ w, const XT *__restrict__ x,
+                                            const float *__restrict__ scale, float *__restrict__ y, uint32_t n,
+                                            uint32_t k, uint32_t row0, uint4 *xs) {
   const uint32_t lanes = (k / P + FK_WAVE - 1) / FK_WAVE;  // packs a lane
-  if (k == FK_WAVE * KPL * P && blockDim.x == 256) {
+  if (k == FK_WAVE * KPL * P) {
     gemv_xlds<WT, XT, P, R, KPL, true, 256>(w, x, scale, y, n, k, row0, xs);
-  } else if (lanes > KPL || (sizeof(WT) == 1 && lanes <= 2)) {
-    if (row0 < n) gemv_wave<WT, XT, P, R>(w, x, scale, y, n, k, row0);
-  } else if (blockDim.x != 256) {
-    gemv_xlds<WT, XT, P, R, KPL, false, 0>(w, x, scale, y, n, k, row0, xs);
   } else if (lanes <= 1) {
     gemv_xlds<WT, XT, P, R, 1, false, 256>(w, x, scale, y, n, k, row0, xs);
   } else if (lanes <= 2) {
@@ -570,37 +561,68 @@ __device__ __forceinline__ void gemv_wide(const WT *__restrict__ w, const float 
 // Entry points: a threadgroup of W wavefronts takes W * R consecutive rows.
 // Kernargs: the buffers in binding order, then the parameter struct.
 
+// Any threadgroup: rows of at most 64 KPL packs in flight at once, wider ones
+// by the loop.
 #define FK_GEMV_ENTRY(NAME, WT, XT, P, R, KPL)                                                               \
   extern "C" __global__ void __launch_bounds__(256) NAME(const WT *__restrict__ w, const XT *__restrict__ x, \
                                                          float *__restrict__ y, fk_gemv_params p) {         \
-    fk::gemv_rows<WT, XT, P, R, KPL>(w, x, nullptr, y, p.n, p.k);                                            \
+    const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * (R);             \
+    if (row0 >= p.n) return;                                                                                 \
+    if (p.k / (P) == FK_WAVE * (KPL))                                                                        \
+      fk::gemv_wave_inflight<WT, XT, P, R, KPL, true>(w, x, nullptr, y, p.n, p.k, row0);                    \
+    else if (p.k / (P) < FK_WAVE * (KPL))                                                                    \
+      fk::gemv_wave_inflight<WT, XT, P, R, KPL, false>(w, x, nullptr, y, p.n, p.k, row0);                   \
+    else                                                                                                     \
+      fk::gemv_wave<WT, XT, P, R>(w, x, nullptr, y, p.n, p.k, row0);                                         \
   }
 
-// (WAVES a SIMD: int8 rows that the loop takes are short, and many at once.)
+// Threadgroups of 256 with x staged in LDS, rows of at most 64 KPL packs: the
+// same sums.  (Entries of their own: beside the form above, the f16 row would
+// keep 110 registers where it needs 80.  Smaller threadgroups stage x more
+// often than they read it: f16 4096 x 4096 of 64 threads 11.6 µs, by the form
+// above 7.9, of 256 7.2 and 7.9.)
+#define FK_GEMV_STAGED_ENTRY(NAME, WT, XT, P, R, KPL)                                                        \
+  extern "C" __global__ void __launch_bounds__(256) NAME(const WT *__restrict__ w, const XT *__restrict__ x, \
+                                                         float *__restrict__ y, fk_gemv_params p) {         \
+    __shared__ uint4 xs[FK_WAVE * (KPL) * (P) * sizeof(XT) / 16];                                           \
+    static_assert(sizeof xs >= 256 * 16, "a chunk a thread");                                               \
+    const uint32_t row0 = (blockIdx.x * 4 + threadIdx.x / FK_WAVE) * (R);                                   \
+    fk::gemv_staged<WT, XT, P, R, KPL>(w, x, nullptr, y, p.n, p.k, row0, xs);                               \
+  }
+
+// The int8 entries: x staged in any threadgroup (64 threads, 8192 x 8192 by the
+// loop 35.9 µs, so 24.0; 128, 22.7 and 18.1), but rows of up to two packs a
+// lane, whose x is no more than the weights' bytes, and wider ones by the loop
+// (16384 x 512 6.2, staged 6.8).  (WAVES a SIMD: rows that the loop takes are
+// short, and many at once.)
 #define FK_GEMV_SCALED_ENTRY(NAME, WT, XT, P, R, KPL, WAVES)                                               \
   extern "C" __global__ void __launch_bounds__(256, WAVES)                                                 \
       NAME(const WT *__restrict__ w, const float *__restrict__ scale, const XT *__restrict__ x,            \
            float *__restrict__ y, fk_gemv_params p) {                                                      \
-    fk::gemv_rows<WT, XT, P, R, KPL>(w, x, scale, y, p.n, p.k);                                            \
+    __shared__ uint4 xs[FK_WAVE * (KPL) * (P) * sizeof(XT) / 16];                                         \
+    static_assert(sizeof xs >= 256 * 16, "a chunk a thread");                                             \
+    const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * (R);           \
+    const uint32_t lanes = (p.k / (P) + FK_WAVE - 1) / FK_WAVE;                                           \
+    if (lanes > (KPL) || lanes <= 2) {                                                                     \
+      if (row0 < p.n) fk::gemv_wave<WT, XT, P, R>(w, x, scale, y, p.n, p.k, row0);                        \
+    } else if (blockDim.x == 256) {                                                                        \
+      fk::gemv_staged<WT, XT, P, R, KPL>(w, x, scale, y, p.n, p.k, row0, xs);                             \
+    } else {                                                                                               \
+      fk::gemv_xlds<WT, XT, P, R, KPL, false, 0>(w, x, scale, y, p.n, p.k, row0, xs);                     \
+    }                                                                                                      \
   }
 
-// f16 rows of more than 4096 columns, a row a wavefront, four a threadgroup.
-// Of 4096 rows or more, with x whole in LDS (its lanes of packs rounded up to
-// 64): through the L1 it is twice the weights' bytes.  Fewer leave the chip to
+// f16 rows of more than 4096 columns, a row a wavefront, four a threadgroup, with
+// x whole in LDS (its lanes of packs rounded up to 64): through the L1 it is
+// twice the weights' bytes.  For 4096 rows or more; fewer leave the chip to
 // their latency, and x is met sooner where it lies.  MI355X, µs, by the loop
-// and so: 16384 x 8192 50.3, 43.8; 8192 x 6000 25.1, 21.0; 2048 x 8192 8.1,
+// and so: 16384 x 8192 51.5, 45.3; 8192 x 6000 24.4, 21.2; 2048 x 8192 7.8,
 // 9.3; f32, whose weights are as wide as x: 83.
 extern "C" __global__ void __launch_bounds__(256)
     fk_gemv_f16_f32_wide(const _Float16 *__restrict__ w, const float *__restrict__ x, float *__restrict__ y,
                          fk_gemv_params p) {
   extern __shared__ uint4 gemv_wide_xs[];
   fk::gemv_wide<_Float16, 8>(w, x, y, p.n, p.k, gemv_wide_xs);
-}
-extern "C" __global__ void __launch_bounds__(256)
-    fk_gemv_f16_f32_loop(const _Float16 *__restrict__ w, const float *__restrict__ x, float *__restrict__ y,
-                         fk_gemv_params p) {
-  const uint32_t row = blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE;
-  if (row < p.n) fk::gemv_wave<_Float16, float, 8, 1>(w, x, nullptr, y, p.n, p.k, row);
 }
 
 // Rows whose width is a multiple of 4 but not of a 16-byte pack (the small
@@ -653,6 +675,12 @@ FK_GEMV_ENTRY(fk_gemv_f32_f32_r4, float, float, 4, 4, 4)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r1, _Float16, float, 8, 1, 8)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r2, _Float16, float, 8, 2, 8)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r4, _Float16, float, 8, 4, 4)
+FK_GEMV_STAGED_ENTRY(fk_gemv_f32_f32_staged_r1, float, float, 4, 1, 16)
+FK_GEMV_STAGED_ENTRY(fk_gemv_f32_f32_staged_r2, float, float, 4, 2, 16)
+FK_GEMV_STAGED_ENTRY(fk_gemv_f32_f32_staged_r4, float, float, 4, 4, 4)
+FK_GEMV_STAGED_ENTRY(fk_gemv_f16_f32_staged_r1, _Float16, float, 8, 1, 8)
+FK_GEMV_STAGED_ENTRY(fk_gemv_f16_f32_staged_r2, _Float16, float, 8, 2, 8)
+FK_GEMV_STAGED_ENTRY(fk_gemv_f16_f32_staged_r4, _Float16, float, 8, 4, 4)
 FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r1, int8_t, _Float16, 16, 1, 8, 8)
 FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r2, int8_t, _Float16, 16, 2, 8, 1)
 FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r4, int8_t, _Float16, 16, 4, 4, 1)

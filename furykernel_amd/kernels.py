@@ -481,7 +481,9 @@ NORM_PACK_HELD = (512, 1024, 2048, 4096)
 
 ABIS: dict[str, KernelAbi] = {
     **_gemv_abis(),
-    **{e: KernelAbi(e, ("w", "x", "y"), GemvParams, 256) for e in ("fk_gemv_f16_f32_wide", "fk_gemv_f16_f32_loop")},
+    **{e: KernelAbi(e, ("w", "x", "y"), GemvParams, 256)
+       for e in ("fk_gemv_f16_f32_wide",
+                 *(f"fk_gemv_{t}_f32_staged_r{r}" for t in ("f32", "f16") for r in (1, 2, 4)))},
     "fk_rmsnorm_f32": KernelAbi("fk_rmsnorm_f32", ("x", "gamma", "y"), RmsNormParams),
     "fk_softmax_f32": KernelAbi("fk_softmax_f32", ("x", "y"), SoftmaxParams),
     "fk_softmax_f32_wide": KernelAbi("fk_softmax_f32_wide", ("x", "y"), SoftmaxParams, 1024),
@@ -559,9 +561,14 @@ ABIS: dict[str, KernelAbi] = {
     "fk_stream_read": KernelAbi("fk_stream_read", ("src", "out"), StreamReadParams),
 }
 
-# f16 matvecs (fk_gemv.h): the columns that a wavefront holds, the x that a
-# threadgroup holds whole in LDS, and the rows from which that pays.
-GEMV_HELD, GEMV_WIDE, GEMV_WIDE_ROWS = 4096, 16384, 4096
+# Matvecs (fk_gemv.h): the columns up to which a row takes x staged in LDS, by
+# the weights and the rows a wavefront takes: what it holds, of four f16 rows
+# (2048) a little less (16384 x 1800 12.7 µs, staged 11.2; x 2040 14.1, 14.9).
+# Of wider f16 rows the x that a threadgroup holds whole in LDS, and the rows
+# from which that pays.
+GEMV_HELD = {("f32", 1): 4096, ("f32", 2): 4096, ("f32", 4): 1024,
+             ("f16", 1): 4096, ("f16", 2): 4096, ("f16", 4): 1800}
+GEMV_WIDE, GEMV_WIDE_ROWS = 16384, 4096
 
 # Softmax rows that four times the threads make, in the same order (fk_rows.h):
 # more than 2048 elements (64 rows of 2048: 3.65 µs, so 3.73; of 4096 4.9, 4.1),
@@ -572,6 +579,27 @@ SOFTMAX_WIDE_FROM, SOFTMAX_WIDE, SOFTMAX_WIDE_ROWS = 2048, 16384, 512
 # Elements a lane loads at once, by weight type: one 16-byte load of W.
 GEMV_PACK = {"f32": 4, "f16": 8, "i8": 16}
 ELEM_BYTES = {"f32": 4, "f16": 2, "i8": 1}
+
+
+def gemv_launch(wtype: str, n: int, k: int, rows_per_wave: int, threads: int) -> tuple[str, int, int]:
+    """The entry, threadgroups and LDS bytes of a standalone matvec in
+    threadgroups of `threads`: of 256, x is staged in LDS (fk_gemv.h says
+    where that pays); the sums are the same in any."""
+    entry, lds = f"fk_gemv_{wtype}_{'f16' if wtype == 'i8' else 'f32'}_r{rows_per_wave}", 0
+    if threads == 256 and wtype != "i8":
+        if k <= GEMV_HELD[wtype, rows_per_wave]:
+            entry = f"fk_gemv_{wtype}_f32_staged_r{rows_per_wave}"
+        elif wtype == "f16" and rows_per_wave == 1 and n >= GEMV_WIDE_ROWS and k <= GEMV_WIDE:
+            entry, lds = "fk_gemv_f16_f32_wide", -(-k // (64 * GEMV_PACK["f16"])) * 64 * GEMV_PACK["f16"] * 4
+    return entry, -(-n // (threads // WAVE * rows_per_wave)), lds
+
+
+def softmax_launch(rows: int, n: int, threads: int) -> tuple[str, int]:
+    """The entry and threads of a softmax in the order of `threads` threads:
+    of 256, four for one where the rows are few and long, bit for bit."""
+    if threads == 256 and SOFTMAX_WIDE_FROM < n <= SOFTMAX_WIDE and rows <= SOFTMAX_WIDE_ROWS:
+        return "fk_softmax_f32_wide", 1024
+    return "fk_softmax_f32", threads
 
 
 def _need(buf: runtime.Buffer, nbytes: int, what: str, entry: str) -> None:
@@ -633,19 +661,7 @@ class Kernels:
                 raise LaunchError(f"{entry}: the int8 layer needs its per-row scales")
             _need(scale, n * 4, "scale", entry)
             bound["scale"] = scale.ptr
-        if wtype != "i8" and k <= GEMV_HELD:
-            # x is staged once a threadgroup: smaller ones than 256 stage it
-            # more often for the same sums (f16 4096 x 4096: of 64 threads
-            # 11.8 µs, of 256 7.5)
-            threads = 256
-        rows_per_group = threads // WAVE * rows_per_wave
-        groups = (n + rows_per_group - 1) // rows_per_group
-        lds = 0
-        if wtype == "f16" and rows_per_wave == 1 and threads == 256 and k > GEMV_HELD:
-            if n >= GEMV_WIDE_ROWS and k <= GEMV_WIDE:
-                entry, lds = "fk_gemv_f16_f32_wide", -(-k // (64 * pack)) * 64 * pack * 4
-            else:
-                entry = "fk_gemv_f16_f32_loop"
+        entry, groups, lds = gemv_launch(wtype, n, k, rows_per_wave, threads)
         self.launch(entry, groups, threads, bound, GemvParams(n, k), stream, lds)
 
     # C = A Bᵀ on the matrix cores (fk_gemm.h): the prefill GEMM.  256 × 256
@@ -825,6 +841,8 @@ class Kernels:
 
     def softmax(self, x: runtime.Buffer, y: runtime.Buffer, rows: int, n: int, threads: int = 256,
                 stream: runtime.Stream | None = None) -> None:
+        """The softmax of each row in the order of `threads` threads (of 256
+        maybe by more of them, softmax_launch)."""
         entry = "fk_softmax_f32"
         if rows <= 0 or n <= 0 or n % 4:
             raise LaunchError(f"{entry}: rows of {n} are not packs of 4")
@@ -832,8 +850,7 @@ class Kernels:
             raise LaunchError(f"{entry}: {threads} threads is not 1 to 16 wavefronts")
         _need(x, rows * n * 4, "x", entry)
         _need(y, rows * n * 4, "y", entry)
-        if threads == 256 and SOFTMAX_WIDE_FROM < n <= SOFTMAX_WIDE and rows <= SOFTMAX_WIDE_ROWS:
-            entry, threads = "fk_softmax_f32_wide", 1024
+        entry, threads = softmax_launch(rows, n, threads)
         self.launch(entry, rows, threads, {"x": x.ptr, "y": y.ptr}, SoftmaxParams(rows, n), stream)
 
 

@@ -5,10 +5,10 @@ src/FuryKernel/Selection.hs; the GEMV axes of test/Test/FuryKernel/Gemv.hs:
 
 Families:
 
-* ``gemv_f32``, ``gemv_f16``, ``gemv_i8`` — the standalone matvec
-  (``fk_gemv_<w>_<x>_r<R>``): axes rows a wavefront (r: 1, 2, 4) and
-  threads (t: 64, 128, 256); classes n × k × m (m the batch, 1).  Pack and
-  split-K, the reference's order axes, are fixed by these kernels (a pack of
+* ``gemv_f32``, ``gemv_f16``, ``gemv_i8`` — the standalone matvec (the
+  launch that ``kernels.gemv_launch`` makes of them): axes rows a wavefront
+  (r: 1, 2, 4) and threads (t: 64, 128, 256); classes n × k × m (m the batch,
+  1).  Pack and split-K, the reference's order axes, are fixed by these kernels (a pack of
   4 f32, 8 f16 or 16 i8 elements a lane load; no split), so no axis here
   decides a reduction's order: every variant of a class gives the same bits.
 * ``step_gemv_f16``, ``step_gemv_bf16`` — the decode step's GEMV
@@ -69,13 +69,11 @@ def gemv_space(wtype: str, classes: Optional[list] = None) -> Space:
     def kernel(name, shape, point):
         n, k = shape_dim("n", shape), shape_dim("k", shape)
         r, t = point_value("r", point), point_value("t", point)
-        entry = f"fk_gemv_{wtype}_{xtype}_r{r}"
-        if entry not in K.ABIS:
-            raise Illegal([f"{name}: no kernel {entry}."])
-        per_group = t // 64 * r
-        groups = -(-n // per_group)
+        if f"fk_gemv_{wtype}_{xtype}_r{r}" not in K.ABIS:
+            raise Illegal([f"{name}: no kernel of {r} rows a wavefront."])
+        entry, groups, lds = K.gemv_launch(wtype, n, k, r, t)
         sizes = {"w": n * k * welt, "x": k * xelt, "y": n * 4, "scale": n * 4}
-        return Launch(entry, groups, t, 0, bytes(K.GemvParams(n, k)),
+        return Launch(entry, groups, t, lds, bytes(K.GemvParams(n, k)),
                       tuple(sizes[b] for b in K.ABIS[entry].buffers))
 
     def divides(shape, point):
