@@ -813,6 +813,13 @@ int fk_launch_check(const char *entry, uint32_t groups, uint32_t threads, uint32
                  threads);
     need = {{"w", (uint64_t)p.ranks * 4}, {"x", (uint64_t)p.ranks * p.seg * 4}, {"y", (uint64_t)p.seg * 4}};
     if (p.residual) need.push_back({"res", (uint64_t)p.seg * 4});
+  } else if (std::strcmp(entry, "fk_softmax_f32_wide") == 0) {
+    fk_softmax_params p;
+    std::memcpy(&p, params, sizeof p);
+    // a row a threadgroup, held whole: at most 16 elements a thread
+    if (p.rows == 0 || p.n == 0 || p.n % 4 || p.n > 16384 || groups < p.rows)
+      return bad(err, cap, FK_ERR_ARG, "%s: %u rows of %u in %u groups", entry, p.rows, p.n, groups);
+    need = {{"x", (uint64_t)p.rows * p.n * 4}, {"y", (uint64_t)p.rows * p.n * 4}};
   } else if (std::strcmp(entry, "fk_gemv_f16_f32_wide") == 0) {
     fk_gemv_params p;
     std::memcpy(&p, params, sizeof p);

@@ -74,3 +74,16 @@ def test_softmax_threads():
     assert K.softmax_launch(64, 4096, 256) == ("fk_softmax_f32_wide", 1024)
     assert K.softmax_launch(64, 4096, 512) == ("fk_softmax_f32", 512)
     assert K.softmax_launch(64, 2048, 256) == ("fk_softmax_f32", 256) == K.softmax_launch(513, 4096, 256)
+
+
+def test_the_wide_softmax_refuses_rows_it_cannot_hold():
+    """It holds 16 elements a thread; a longer row would be summed and stored
+    short."""
+    def check(rows, n, groups, threads=1024, short=0):
+        spans = [(1 << 40, rows * n * 4), (2 << 40, rows * n * 4 - short)]
+        runtime.launch_check("fk_softmax_f32_wide", groups, threads, 0, spans, K.SoftmaxParams(rows, n))
+    check(3, 16384, 3)
+    check(3, 4, 3)
+    for bad in ((3, 16388, 3), (3, 32768, 3), (3, 4098, 3), (3, 4096, 2), (3, 4096, 3, 512), (3, 4096, 3, 1024, 4)):
+        with pytest.raises(runtime.FkError):
+            check(*bad)
