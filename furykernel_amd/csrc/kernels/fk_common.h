@@ -128,28 +128,19 @@ __device__ __forceinline__ float wave_max(float x) {
 }
 
 // tgReduceSum / tgReduceMax (src/FuryKernel/Reduce.hs:55-85): each wave's
-// reduction in its slot; after a barrier the first wave's lane l folds slots
-// l, l + 64, ... from the identity (-0 for the sum, -inf for the maximum) and
-// reduces once more; every thread gets the result.  `slots` holds one float per
-// wave and is reusable when this returns.
+// reduction in its slot; after a barrier lane l folds slot l onto the identity
+// (-0 for the sum, -inf for the maximum) and the wave reduces once more, every
+// wavefront for itself, so that each thread has the result at one barrier.
+// `slots` holds one float per wave and is used once.
 template <bool IsMax>
 __device__ __forceinline__ float block_reduce(float v, float *slots) {
-  const int lane = threadIdx.x & (FK_WAVE - 1);
-  const int wave = threadIdx.x / FK_WAVE;
-  const int waves = blockDim.x / FK_WAVE;
-  float s = IsMax ? wave_max(v) : wave_sum(v);
-  if (lane == 0) slots[wave] = s;
+  const uint32_t lane = threadIdx.x & (FK_WAVE - 1), waves = blockDim.x / FK_WAVE;
+  const float s = IsMax ? wave_max(v) : wave_sum(v);
+  if (lane == 0) slots[threadIdx.x / FK_WAVE] = s;
   __syncthreads();
-  if (wave == 0) {
-    float acc = IsMax ? -__builtin_inff() : -0.0f;
-    for (int k = lane; k < waves; k += FK_WAVE) acc = IsMax ? max_number(acc, slots[k]) : acc + slots[k];
-    float t = IsMax ? wave_max(acc) : wave_sum(acc);
-    if (lane == 0) slots[0] = t;
-  }
-  __syncthreads();
-  float total = slots[0];
-  __syncthreads();
-  return total;
+  float acc = IsMax ? -__builtin_inff() : -0.0f;
+  if (lane < waves) acc = IsMax ? max_number(acc, slots[lane]) : acc + slots[lane];
+  return IsMax ? wave_max(acc) : wave_sum(acc);
 }
 
 // rsqrt, exp: binary64's, rounded once to binary32 (src/FuryKernel/Interp.hs:828-854).

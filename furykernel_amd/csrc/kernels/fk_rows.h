@@ -13,19 +13,6 @@
 
 namespace fk {
 
-// block_reduce where `slots` is used once: its first round, one barrier, and
-// the second round by every wavefront for itself.
-template <bool IsMax>
-__device__ __forceinline__ float block_reduce_once(float v, float *slots) {
-  const uint32_t lane = threadIdx.x & (FK_WAVE - 1), waves = blockDim.x / FK_WAVE;
-  const float s = IsMax ? wave_max(v) : wave_sum(v);
-  if (lane == 0) slots[threadIdx.x / FK_WAVE] = s;
-  __syncthreads();
-  float acc = IsMax ? -__builtin_inff() : -0.0f;
-  if (lane < waves) acc = IsMax ? max_number(acc, slots[lane]) : acc + slots[lane];
-  return IsMax ? wave_max(acc) : wave_sum(acc);
-}
-
 // Segments of at most H packs a thread: the thread's packs (t, t + T, ...)
 // loaded into registers at once — every load issued before any is used, its
 // index clamped into the segment — and both passes made on the registers,
@@ -52,7 +39,7 @@ __device__ __forceinline__ void rmsnorm_held(const float *__restrict__ xs, const
     a = a + v[i].w * v[i].w;
     acc = t + i * T < packs ? a : acc;
   }
-  const float total = block_reduce_once<false>(acc, slots);
+  const float total = block_reduce<false>(acc, slots);
   const float scale = rsqrt_once(total / (float)p.seg + p.eps);
 #pragma unroll
   for (int i = 0; i < H; i++) {
@@ -98,7 +85,7 @@ extern "C" __global__ void __launch_bounds__(1024)
     acc = acc + v.z * v.z;
     acc = acc + v.w * v.w;
   }
-  const float total = fk::block_reduce_once<false>(acc, slots);
+  const float total = fk::block_reduce<false>(acc, slots);
   const float scale = fk::rsqrt_once(total / (float)p.seg + p.eps);
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
@@ -141,7 +128,7 @@ __device__ __forceinline__ void softmax_held(const float *__restrict__ xs, float
     a = max_number(a, v[i].w);
     m = t + i * T < packs ? a : m;
   }
-  const float top = block_reduce_once<true>(m, tops);
+  const float top = block_reduce<true>(m, tops);
   float acc = -0.0f;
   float4 e[H];
 #pragma unroll
@@ -154,7 +141,7 @@ __device__ __forceinline__ void softmax_held(const float *__restrict__ xs, float
     a = a + e[i].w;
     acc = t + i * T < packs ? a : acc;
   }
-  const float total = block_reduce_once<false>(acc, slots);
+  const float total = block_reduce<false>(acc, slots);
 #pragma unroll
   for (int i = 0; i < H; i++) {
     if (t + i * T >= packs) break;
@@ -186,7 +173,7 @@ extern "C" __global__ void __launch_bounds__(1024)
     m = fk::max_number(m, v.z);
     m = fk::max_number(m, v.w);
   }
-  const float top = fk::block_reduce_once<true>(m, tops);
+  const float top = fk::block_reduce<true>(m, tops);
   float acc = -0.0f;
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
@@ -195,7 +182,7 @@ extern "C" __global__ void __launch_bounds__(1024)
     acc = acc + fk::exp_once(v.z - top);
     acc = acc + fk::exp_once(v.w - top);
   }
-  const float total = fk::block_reduce_once<false>(acc, slots);
+  const float total = fk::block_reduce<false>(acc, slots);
   for (uint32_t j = threadIdx.x; j < packs; j += blockDim.x) {
     float4 v = *reinterpret_cast<const float4 *>(xs + 4 * (size_t)j);
     float4 o = make_float4(fk::exp_once(v.x - top) / total, fk::exp_once(v.y - top) / total,
@@ -227,7 +214,7 @@ __device__ __forceinline__ void softmax_wide(const float *__restrict__ xs, float
 #pragma unroll
   for (int h = 0; h < H; h++)  // (a pack past the row repeats its last one)
     m = max_number(max_number(max_number(max_number(m, v[h].x), v[h].y), v[h].z), v[h].w);
-  const float top = block_reduce_once<true>(m, tops);
+  const float top = block_reduce<true>(m, tops);
 #pragma unroll
   for (int h = 0; h < H; h++) {
     v[h] = make_float4(exp_once(v[h].x - top), exp_once(v[h].y - top), exp_once(v[h].z - top), exp_once(v[h].w - top));
