@@ -23,9 +23,13 @@
 // 64) once there are many (64 rows, 185 MB: 36.6 µs, 5.1 TB/s), and below that
 // a launch's latency (one row of 4096 positions, 8.4 MB: 5.9 µs).  8 rows of
 // 256 to 4095 positions: 58 µs in blocks of 32 queries, 10.6 here and 2.3 for
-// the combine; 41 rows of up to 700: 18 µs, now 8.9 and 2.1.  The arithmetic is fk_prefill_attend's:
-// f16 operands, binary32 scores, probabilities rounded to f16 and summed as
-// rounded, exp2 of scores in log2 units.
+// the combine; 41 rows of up to 700: 18 µs, now 8.9 and 2.1.
+//
+// The arithmetic is fk_prefill_attend's: f16 operands, binary32 scores,
+// probabilities rounded to f16 and summed as rounded, exp2 of scores in log2
+// units.  A wavefront's reference lies 8 below its running maximum, so that
+// its probabilities reach 2^8 and small ones keep f16's bits at least as long
+// as with that kernel's reference, which may lag its maximum by up to 8.
 #pragma once
 
 #include "fk_common.h"
@@ -169,9 +173,9 @@ __device__ __forceinline__ void rows_attend(const uint16_t *__restrict__ qr, con
         sc[s][r] = k <= ks.pos && k >= ks.first ? sc[s][r] * c : -__builtin_inff();
         mt = __builtin_fmaxf(mt, sc[s][r]);
       }
-    mt = fk::rows_max(mt);
+    mt = fk::rows_max(mt) - 8.0f;
     // (a head whose scores are all -inf, or NaN, keeps nothing: 0 in place
-    // of its maximum)
+    // of its reference)
     const float mn = __builtin_fmaxf(m, mt);
     const float mc = mn == -__builtin_inff() ? 0.0f : mn;
     const float alpha = __builtin_amdgcn_exp2f(m - mc);
