@@ -105,7 +105,7 @@ struct SkinnyForm {
 };
 const SkinnyForm skinny_forms[] = {{"m1n1", 1, 1, 8}, {"m1n2", 1, 2, 8}, {"m2n1", 2, 1, 8}, {"m2n2", 2, 2, 8},
                                    {"m2n4", 2, 4, 4}, {"m4n2", 4, 2, 8}, {"m4n4", 4, 4, 4}, {"m4n8", 4, 8, 4},
-                                   {"m8n4", 8, 4, 4}, {"m8n8", 8, 8, 4}};
+                                   {"m8n8", 8, 8, 4}};
 // The forms of the prefill attention whose keys are split among groups of
 // wavefronts: heads (wavefronts) a group, groups.
 struct SplitForm {

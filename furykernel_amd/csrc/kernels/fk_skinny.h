@@ -22,19 +22,20 @@
 //   fk_gemm.h).
 //
 // What bounds it: up to 16 live rows the weights' stream from HBM (gate and
-// up, 67 MB, in 13.9 µs: 4.8 TB/s; the logits, 131 MB, in 25.9: 5.1) or, of
+// up, 67 MB, in 13.6 µs: 4.9 TB/s; the logits, 131 MB, in 25.5: 5.1) or, of
 // fewer than 256 tiles, what one CU draws through its L1 (about 75 GB/s: the
-// down projection's 128 tiles read 512 KB each in 12.2 µs); from 64 rows on
-// the operands' reads through the L1s (a tile reads (MB + NB) KB for MB · NB
-// matrix operations), which is why tiles grow with the rows.  Measured on
-// MI355X, f16, µs (fk_gemm's tiles in brackets):
+// down projection's 128 tiles read 512 KB each); from 64 rows on the operands'
+// reads through the L1s (a tile reads (MB + NB) KB for MB · NB matrix
+// operations), which is why tiles grow with the rows.  Measured on MI355X, f16,
+// each launch on weights of its own out of HBM, µs, the forms that
+// prefill.py's skinny_form picks (fk_gemm's tiles in brackets):
 //
 //   live rows            16          64         112         208         704        1408
-//   QKV  3072 x 2048    7.1 [49]    8.7 [49]  10.9 [49]   12.9 [49]   26.0 [51]   42.7 [57]
-//   O    2048 x 2048    5.4 [50]    6.4 [50]   7.4 [50]    9.1 [50]   18.2 [55]   26.4 [55]
-//   gate/up 2 x 8192   13.6 [45]   17.9 [45]  20.8 [44]   28.0 [44]    -  [51]     -  [98]
-//   down 2048 x 8192   12.5 [160] 15.6 [160]  18.2 [161]  23.3 [161]  45.9 [160]  65.2 [160]
-//   head 32000 x 2048  26.7 [62]   31.0 [56]  38.5 [57]     -  [57]    -  [125]    -  [200]
+//   QKV  3072 x 2048    7.6 [49]    9.0 [49]  11.3 [49]   11.2 [49]   23.4 [51]   38.7 [57]
+//   O    2048 x 2048    5.9 [50]    6.8 [50]   6.5 [50]    8.2 [50]   16.3 [55]   25.6 [55]
+//   gate/up 2 x 8192   13.6 [45]   17.7 [45]  21.1 [44]   30.3 [44]    -  [51]     -  [98]
+//   down 2048 x 8192   12.9 [160] 15.9 [160]  16.9 [161]  21.7 [161]  46.9 [160]  64.4 [160]
+//   head 32000 x 2048  25.5 [62]   36.6 [56]  42.7 [57]     -  [57]    -  [125]    -  [200]
 //
 // The forms (MB, NB, W, D) and where each is taken: prefill.py's skinny_form.
 //
@@ -238,9 +239,9 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
       if (x + s < count) FK_SKINNY_STEP(s, x + s);
   };
   // Weights that one or two tiles of rows read are streamed past the caches
-  // (the down projection of 16 rows 12.2 µs against 13.0, gate and up 13.9
-  // against 15.7); read by more, they are kept (the down projection of 112
-  // rows, four tiles: 18.3 against 19.5).
+  // (the down projection of 16 rows in 6 % less time, gate and up in 11 %);
+  // read by more, they are kept (the down projection of 112 rows, four tiles,
+  // in 6 % less).
   if constexpr (MB * NB >= 64) loop(fk_bool_tag<false>{});
   else if (tiles_m <= 2) loop(fk_bool_tag<true>{});
   else loop(fk_bool_tag<false>{});
@@ -408,7 +409,10 @@ __device__ __forceinline__ void skinny_tile(const _Float16 *__restrict__ a, cons
   }
 
 // S: the ring's steps in the modes that stream many tiles (gate and up, the
-// logits), D in the rest.
+// logits), D in the rest.  m8n8's rings take 64 KB a step and its sums 128 KB,
+// so a second step costs no LDS, but gate and up are slower with it (112 rows
+// 30.9 µs, two steps 33.4; 208, 30.3 and 32.8), the logits about the same (112
+// rows 42.7 and 42.0).
 #define FK_SKINNY_FORM(FORM, MB, NB, W, D, S)                                   \
   FK_SKINNY_ENTRY(fk_skinny_part_##FORM, FK_GEMM_PART, MB, NB, W, D)            \
   FK_SKINNY_ENTRY(fk_skinny_store_##FORM, FK_GEMM_STORE, MB, NB, W, D)          \
@@ -430,6 +434,5 @@ FK_SKINNY_PAIR_FORM(m2n4, 2, 4, 4, 2, 2)
 FK_SKINNY_PAIR_FORM(m4n2, 4, 2, 8, 2, 2)
 FK_SKINNY_PAIR_FORM(m4n4, 4, 4, 4, 2, 2)
 FK_SKINNY_PAIR_FORM(m4n8, 4, 8, 4, 2, 2)
-FK_SKINNY_PAIR_FORM(m8n4, 8, 4, 4, 2, 2)
 FK_SKINNY_PAIR_FORM(m8n8, 8, 8, 4, 2, 1)
 #endif

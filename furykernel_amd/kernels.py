@@ -370,7 +370,7 @@ STEP_GEMV_BUFFERS = ("w0", "w1", "w2", "y0", "y1", "y2", "src", "src2", "gamma",
 # among; forms of one column block have no pairs of columns (gate and up, a
 # head's RoPE pairs).
 SKINNY_FORMS = {"m1n1": (1, 1, 8), "m1n2": (1, 2, 8), "m2n1": (2, 1, 8), "m2n2": (2, 2, 8), "m2n4": (2, 4, 4),
-                "m4n2": (4, 2, 8), "m4n4": (4, 4, 4), "m4n8": (4, 8, 4), "m8n4": (8, 4, 4), "m8n8": (8, 8, 4)}
+                "m4n2": (4, 2, 8), "m4n4": (4, 4, 4), "m4n8": (4, 8, 4), "m8n8": (8, 8, 4)}
 SKINNY_PAIR_MODES = ("silu_mul", "qkv_rope", "qkv_rope_paged")
 SKINNY_MODES = ("store", "add", "part", "store_keys") + SKINNY_PAIR_MODES
 SKINNY_BUFFERS = ("a", "b0", "b1", "b2", "c0", "c1", "c2", "r0", "position", "slot", "rope", "keys")

@@ -194,7 +194,7 @@ def _split_attention(out: Lowered, live: LiveRows) -> None:
 # several.
 SKINNY_COST = {"m1n1": (1.1, 0.037, False), "m1n2": (1.4, 0.054, False), "m2n1": (1.4, 0.047, False),
                "m2n2": (1.9, 0.056, False), "m2n4": (2.3, 0.089, False), "m4n2": (2.4, 0.074, True),
-               "m4n4": (3.3, 0.110, False), "m4n8": (7.0, 0.150, True), "m8n4": (7.0, 0.150, True),
+               "m4n4": (3.3, 0.110, False), "m4n8": (7.0, 0.150, True),
                "m8n8": (11.5, 0.202, True)}
 
 
@@ -213,11 +213,14 @@ def skinny_form(chunks: int, m: int, n: int, k: int, mode: str, splits: tuple = 
       at 4 TB/s.
 
     So, measured: O and down (n 2048) of 1408 rows take m8n8's 176 tiles (26
-    against 55, 65 against 160 at k 8192); gate and up (n 16384) of 208 rows
-    its 256 (28 against 44), but of 352 rows, two rounds, fk_gemm (49 against
-    47).  Among forms, down: 16 rows m1n1 (12.5), 112 rows m2n2 (18.2; m4n2,
-    half as many tiles, 25.6), 352 rows m4n4 (33.7; m4n2 43), 704 rows m8n4
-    (45.9; m4n4 60).  A k shorter than 1024 leaves a wavefront under four
+    against 55, 64 against 160 at k 8192); gate and up (n 16384) of 208 rows
+    its 256 (30 against 44), but of 352 rows, two rounds, fk_gemm (47; m4n4
+    49, m8n8 56).  Among forms, down: 16 rows m1n1 (12.9), 112 rows m2n2
+    (16.9; m4n2, half as many tiles, 27.3), 352 rows m4n4 (32.7; m4n2 40.6),
+    704 rows m4n8 (46.9; m4n4 60).  The picks were the fastest forms, or
+    within 2 %, but for QKV of 64 and 112 rows (9.0, m1n2 8.5; 11.3, m2n4
+    8.4), O and down of 64 (6.8, m1n2 5.9; 15.9, 15.3) and the head of 64
+    (36.6, m4n4 33.9).  A k shorter than 1024 leaves a wavefront under four
     steps to overlap and stays."""
     if k < 1024 or m * k * 2 >= 0xfffffff0:
         return None
