@@ -403,6 +403,17 @@ def gemv_variants(wtype: str, n: int, k: int) -> list:
     return [pick] if pick else [(r, 256) for r in (1, 2, 4)]
 
 
+def launched(ks, run) -> tuple:
+    """(entry, threads) of the launch that a call makes, not made."""
+    seen = []
+    ks.launch = lambda entry, groups, threads, *rest: seen.append((entry, threads))
+    try:
+        run()
+    finally:
+        del ks.launch
+    return seen[0]
+
+
 def main_kernels(args) -> int:
     """The standalone kernels at their configurations' sizes: f32 matvec
     W[4096 × 4096]·x, RMSNorm and row softmax over [64 × 4096] f32, and the
@@ -469,7 +480,7 @@ def main_kernels(args) -> int:
     best = None
     for r, t in gemv_variants("f32", n, k):
         us = timed([lambda w=w, r=r, t=t: ks.gemv(w, x, y, n, k, "f32", rows_per_wave=r, threads=t) for w in ws], 20)
-        entry = kernels.gemv_launch("f32", n, k, r, t)[0]
+        entry, _ = launched(ks, lambda r=r, t=t: ks.gemv(ws[0], x, y, n, k, "f32", rows_per_wave=r, threads=t))
         log(f"{entry} 4096 x 4096, {t} threads: {us:.2f} us a launch, {nbytes / us / 1e3:.1f} GB/s")
         if best is None or us < best[1]:
             best = (entry, us)
@@ -486,15 +497,14 @@ def main_kernels(args) -> int:
         normal(b, 300 + i, False)
     normal(gamma, 298, False)
     bufs += xs + [gamma, out]
-    for name, launched, run, nb in (
-            ("rmsnorm_64x4096", lambda t: ("fk_rmsnorm_f32", t),
-             lambda b, t: ks.rmsnorm(b, gamma, out, rows, width, threads=t), 2 * rows * width * 4 + width * 4),
-            ("softmax_64x4096", lambda t: kernels.softmax_launch(rows, width, t),
-             lambda b, t: ks.softmax(b, out, rows, width, threads=t), 2 * rows * width * 4)):
+    for name, run, nb in (
+            ("rmsnorm_64x4096", lambda b, t: ks.rmsnorm(b, gamma, out, rows, width, threads=t),
+             2 * rows * width * 4 + width * 4),
+            ("softmax_64x4096", lambda b, t: ks.softmax(b, out, rows, width, threads=t), 2 * rows * width * 4)):
         best = None
         for t in (256, 512, 1024):
             us = timed([lambda b=b, t=t: run(b, t) for b in xs], 20)
-            entry, t = launched(t)
+            entry, t = launched(ks, lambda t=t: run(xs[0], t))
             log(f"{entry} 64 x 4096, {t} threads a row: {us:.2f} us a launch, {nb / us / 1e3:.1f} GB/s")
             if best is None or us < best[2]:
                 best = (entry, t, us)
@@ -517,7 +527,8 @@ def main_kernels(args) -> int:
     for r, t in gemv_variants("i8", n, k):
         us = timed([lambda w=w, r=r, t=t: ks.gemv(w, xh, yi, n, k, "i8", rows_per_wave=r, threads=t, scale=scale)
                     for w in wi], 20)
-        entry = kernels.gemv_launch("i8", n, k, r, t)[0]
+        entry, _ = launched(ks, lambda r=r, t=t: ks.gemv(wi[0], xh, yi, n, k, "i8", rows_per_wave=r, threads=t,
+                                                         scale=scale))
         log(f"{entry} 8192 x 8192, {t} threads: {us:.2f} us a launch, {nbytes / us / 1e3:.1f} GB/s")
         if best is None or us < best[1]:
             best = (entry, us)

@@ -417,6 +417,11 @@ ATTEND_RULE_BF16 = {1: (((1, 4), 767, 256, 1), ((1, 2), 1024, 512, 1)),
                     2: (((2, 4), 767, 512, 1), ((2, 2), 2559, 1024, 1)),
                     4: (((2, 4), 767, 512, 128), ((4, 2), 1279, 1024, 256))}
 ATTEND_RULE_MANY = ((4, 2), 2559, 2048, 1024)  # 4 heads, past those
+# (form, heads a kv head or (heads a group, groups)) -> entry
+ATTEND_ENTRIES = {(form, g): f"fk_prefill_attend_{form}g{g}" for form in ("", "f16_", "paged_", "paged_f16_")
+                  for g in (1, 2, 4)}
+ATTEND_ENTRIES.update({(form, hk): f"fk_split_attend_{form}h{hk[0]}k{hk[1]}"
+                       for form in ("", "f16_", "paged_", "paged_f16_") for hk in ATTEND_SPLITS})
 
 
 def attend_launch(form: str, rows: int, heads: int, kv_heads: int, keys: int, window: int = 0, bf16: bool = False,
@@ -462,18 +467,17 @@ def attend_launch(form: str, rows: int, heads: int, kv_heads: int, keys: int, wi
     too (4 x 512 from 0: 12.4, h4k2 12.8).  The rule is the same for every
     place that a session's keys come from, so that its staged, paged and ring
     steps of one shape agree bit for bit."""
-    g = heads // kv_heads
-    pairs = rows // 32 * heads
-    rule = (ATTEND_RULE_BF16 if bf16 else ATTEND_RULE)[g]
-    if g == 4 and keys > 8 * ATTEND_KEYS and (prompts or "f16" in form):
-        rule += (ATTEND_RULE_MANY,)
-    if keys >= 8 * ATTEND_KEYS:
-        for (h, k), most, most_windowed, least in rule:
+    g, pairs = heads // kv_heads, rows // 32 * heads
+    if keys >= 512 and pairs < 2560:
+        rule = (ATTEND_RULE_BF16 if bf16 else ATTEND_RULE)[g]
+        if g == 4 and keys > 512 and (prompts or "f16" in form):
+            rule += (ATTEND_RULE_MANY,)
+        for split, most, most_windowed, least in rule:
             if pairs <= (most_windowed if window else most):
                 if window and window < least:
                     break
-                return f"fk_split_attend_{form}h{h}k{k}", pairs // h, 64 * h * k
-    return f"fk_prefill_attend_{form}g{g}", rows // 32 * kv_heads, 64 * g
+                return ATTEND_ENTRIES[form, split], pairs // split[0], 64 * split[0] * split[1]
+    return ATTEND_ENTRIES[form, g], rows // 32 * kv_heads, 64 * g
 
 
 # Row widths the one-pass RMSNorm-to-tiles holds in registers (fk_prefill.h).
@@ -561,6 +565,10 @@ ABIS: dict[str, KernelAbi] = {
     "fk_stream_read": KernelAbi("fk_stream_read", ("src", "out"), StreamReadParams),
 }
 
+# Elements a lane loads at once, by weight type: one 16-byte load of W.
+GEMV_PACK = {"f32": 4, "f16": 8, "i8": 16}
+ELEM_BYTES = {"f32": 4, "f16": 2, "i8": 1}
+
 # Matvecs (fk_gemv.h): the columns up to which a row takes x staged in LDS, by
 # the weights and the rows a wavefront takes: what it holds, of four f16 rows
 # (2048) a little less (16384 x 1800 12.7 µs, staged 11.2; x 2040 14.1, 14.9).
@@ -568,6 +576,12 @@ ABIS: dict[str, KernelAbi] = {
 # from which that pays.
 GEMV_HELD = {("f32", 1): 4096, ("f32", 2): 4096, ("f32", 4): 1024,
              ("f16", 1): 4096, ("f16", 2): 4096, ("f16", 4): 1800}
+# (weights, rows a wavefront) -> the entry of any threads, the staged one and
+# the columns up to which it is taken; the elements of a pack, the bytes of an
+# element of W and of x.
+GEMV_ENTRIES = {(t, r): (f"fk_gemv_{t}_f32_r{r}", f"fk_gemv_{t}_f32_staged_r{r}", held, GEMV_PACK[t], ELEM_BYTES[t], 4)
+                for (t, r), held in GEMV_HELD.items()}
+GEMV_ENTRIES.update({("i8", r): (f"fk_gemv_i8_f16_r{r}", "", 0, 16, 1, 2) for r in (1, 2, 4)})
 GEMV_WIDE, GEMV_WIDE_ROWS = 16384, 4096
 
 # Softmax rows that four times the threads make, in the same order (fk_rows.h):
@@ -576,30 +590,19 @@ GEMV_WIDE, GEMV_WIDE_ROWS = 16384, 4096
 # without (512 of 16384 31.8, 18.6; 1024 of 4096 10.4, 10.1).
 SOFTMAX_WIDE_FROM, SOFTMAX_WIDE, SOFTMAX_WIDE_ROWS = 2048, 16384, 512
 
-# Elements a lane loads at once, by weight type: one 16-byte load of W.
-GEMV_PACK = {"f32": 4, "f16": 8, "i8": 16}
-ELEM_BYTES = {"f32": 4, "f16": 2, "i8": 1}
-
 
 def gemv_launch(wtype: str, n: int, k: int, rows_per_wave: int, threads: int) -> tuple[str, int, int]:
     """The entry, threadgroups and LDS bytes of a standalone matvec in
     threadgroups of `threads`: of 256, x is staged in LDS (fk_gemv.h says
     where that pays); the sums are the same in any."""
-    entry, lds = f"fk_gemv_{wtype}_{'f16' if wtype == 'i8' else 'f32'}_r{rows_per_wave}", 0
-    if threads == 256 and wtype != "i8":
-        if k <= GEMV_HELD[wtype, rows_per_wave]:
-            entry = f"fk_gemv_{wtype}_f32_staged_r{rows_per_wave}"
-        elif wtype == "f16" and rows_per_wave == 1 and n >= GEMV_WIDE_ROWS and k <= GEMV_WIDE:
-            entry, lds = "fk_gemv_f16_f32_wide", -(-k // (64 * GEMV_PACK["f16"])) * 64 * GEMV_PACK["f16"] * 4
+    entry, staged, held, _, _, _ = GEMV_ENTRIES[wtype, rows_per_wave]
+    lds = 0
+    if threads == 256:
+        if k <= held:
+            entry = staged
+        elif rows_per_wave == 1 and wtype == "f16" and n >= GEMV_WIDE_ROWS and k <= GEMV_WIDE:
+            entry, lds = "fk_gemv_f16_f32_wide", -(-k // 512) * 512 * 4
     return entry, -(-n // (threads // WAVE * rows_per_wave)), lds
-
-
-def softmax_launch(rows: int, n: int, threads: int) -> tuple[str, int]:
-    """The entry and threads of a softmax in the order of `threads` threads:
-    of 256, four for one where the rows are few and long, bit for bit."""
-    if threads == 256 and SOFTMAX_WIDE_FROM < n <= SOFTMAX_WIDE and rows <= SOFTMAX_WIDE_ROWS:
-        return "fk_softmax_f32_wide", 1024
-    return "fk_softmax_f32", threads
 
 
 def _need(buf: runtime.Buffer, nbytes: int, what: str, entry: str) -> None:
@@ -643,17 +646,15 @@ class Kernels:
     def gemv(self, w: runtime.Buffer, x: runtime.Buffer, y: runtime.Buffer, n: int, k: int, wtype: str = "f32",
              rows_per_wave: int = 1, threads: int = 256, scale: runtime.Buffer | None = None,
              stream: runtime.Stream | None = None) -> None:
-        xtype = "f16" if wtype == "i8" else "f32"
-        entry = f"fk_gemv_{wtype}_{xtype}_r{rows_per_wave}"
-        if entry not in ABIS:
-            raise LaunchError(f"no GEMV kernel {entry}")
-        pack = GEMV_PACK[wtype]
+        if (wtype, rows_per_wave) not in GEMV_ENTRIES:
+            raise LaunchError(f"no GEMV kernel fk_gemv_{wtype}_{'f16' if wtype == 'i8' else 'f32'}_r{rows_per_wave}")
+        entry, _, _, pack, w_bytes, x_bytes = GEMV_ENTRIES[wtype, rows_per_wave]
         if n <= 0 or k <= 0 or k % pack:
             raise LaunchError(f"{entry}: k = {k} is not a positive multiple of the pack width {pack}")
         if threads % WAVE or not 0 < threads <= 256:
             raise LaunchError(f"{entry}: {threads} threads is not 1 to 4 wavefronts")
-        _need(w, n * k * ELEM_BYTES[wtype], "W", entry)
-        _need(x, k * ELEM_BYTES[xtype], "x", entry)
+        _need(w, n * k * w_bytes, "W", entry)
+        _need(x, k * x_bytes, "x", entry)
         _need(y, n * 4, "y", entry)
         bound = {"w": w.ptr, "x": x.ptr, "y": y.ptr}
         if wtype == "i8":
@@ -778,10 +779,10 @@ class Kernels:
         f16): an element beyond f16's range (|x| > 65504) becomes infinite and
         one below 2^-24 flushes to zero, so bf16 caches are for values inside
         f16's range, as the prefill's own stores of f16-range rows are."""
-        g = heads // kv_heads if kv_heads and heads % kv_heads == 0 else 0
         form = "" if cache_bf16 else "f16_"
-        entry = f"fk_prefill_attend_{form}g{g}"
-        if rows <= 0 or rows % 256 or kv_heads <= 0 or heads % kv_heads or heads // kv_heads not in (1, 2, 4):
+        g = heads // kv_heads if kv_heads > 0 and heads % kv_heads == 0 else 0
+        entry = ATTEND_ENTRIES.get((form, g), "fk_prefill_attend")
+        if rows <= 0 or rows % 256 or g not in ATTEND_RULE:
             raise LaunchError(f"{entry}: {rows} rows, {heads} heads over {kv_heads}")
         if length <= 0 or length % ATTEND_KEYS:
             raise LaunchError(f"{entry}: a ring of {length}; keys go by blocks of {ATTEND_KEYS} that must not wrap")
@@ -790,12 +791,13 @@ class Kernels:
             check_rows(positions, seqs)
             if np.max(np.asarray(positions)) >= length:
                 raise LaunchError(f"{entry}: positions past the ring's {length}")
-        _need(qr, rows * heads * 64 * 2, "q", entry)
-        for b, what in ((kc, "K cache"), (vc, "V cache")):
-            _need(b, slots * kv_heads * length * 64 * 2, what, entry)
+        q_bytes, cache_bytes = rows * heads * 128, slots * kv_heads * length * 128
+        _need(qr, q_bytes, "q", entry)
+        _need(kc, cache_bytes, "K cache", entry)
+        _need(vc, cache_bytes, "V cache", entry)
         _need(position, rows * 4, "position", entry)
         _need(slot, rows * 4, "slot", entry)
-        _need(out, rows * heads * 64 * 2, "out", entry)
+        _need(out, q_bytes, "out", entry)
         bound = {"qr": qr.ptr, "kc": kc.ptr, "vc": vc.ptr, "position": position.ptr, "slot": slot.ptr, "out": out.ptr,
                  "ks": 0, "vs": 0}
         entry, groups, threads = attend_launch(form, rows, heads, kv_heads, length, window, cache_bf16)
@@ -841,8 +843,9 @@ class Kernels:
 
     def softmax(self, x: runtime.Buffer, y: runtime.Buffer, rows: int, n: int, threads: int = 256,
                 stream: runtime.Stream | None = None) -> None:
-        """The softmax of each row in the order of `threads` threads (of 256
-        maybe by more of them, softmax_launch)."""
+        """The softmax of each row in the order of `threads` threads; of 256,
+        four make what one of them would where the rows are few and long, bit
+        for bit."""
         entry = "fk_softmax_f32"
         if rows <= 0 or n <= 0 or n % 4:
             raise LaunchError(f"{entry}: rows of {n} are not packs of 4")
@@ -850,7 +853,8 @@ class Kernels:
             raise LaunchError(f"{entry}: {threads} threads is not 1 to 16 wavefronts")
         _need(x, rows * n * 4, "x", entry)
         _need(y, rows * n * 4, "y", entry)
-        entry, threads = softmax_launch(rows, n, threads)
+        if threads == 256 and SOFTMAX_WIDE_FROM < n <= SOFTMAX_WIDE and rows <= SOFTMAX_WIDE_ROWS:
+            entry, threads = "fk_softmax_f32_wide", 1024
         self.launch(entry, rows, threads, {"x": x.ptr, "y": y.ptr}, SoftmaxParams(rows, n), stream)
 
 

@@ -1,6 +1,6 @@
-"""The launch of a standalone matvec or row softmax (kernels.gemv_launch,
-softmax_launch), on the CPU: in threadgroups of the caller's threads, its
-entry one that holds its rows, covering every row once."""
+"""The launch of a standalone matvec (kernels.gemv_launch), on the CPU: in
+threadgroups of the caller's threads, its entry one that holds its rows,
+covering every row once; and what the launch check refuses."""
 
 import ctypes
 
@@ -68,12 +68,6 @@ def test_staged_entries_refuse_rows_they_cannot_hold():
                 with pytest.raises(runtime.FkError):
                     runtime.launch_check(*args)
     assert ctypes.sizeof(K.GemvParams) == 8
-
-
-def test_softmax_threads():
-    assert K.softmax_launch(64, 4096, 256) == ("fk_softmax_f32_wide", 1024)
-    assert K.softmax_launch(64, 4096, 512) == ("fk_softmax_f32", 512)
-    assert K.softmax_launch(64, 2048, 256) == ("fk_softmax_f32", 256) == K.softmax_launch(513, 4096, 256)
 
 
 def test_the_wide_softmax_refuses_rows_it_cannot_hold():
