@@ -477,9 +477,9 @@ __device__ __forceinline__ void gemv_xlds(const WT *__restrict__ w, const XT *__
   }
 }
 
-// The rows of a threadgroup of 256 threads, at most 64 KPL packs each: full
-// rows, or by the fewest packs a lane that hold the row (a pack past the row
-// costs its products all the same).  MI355X, µs, by the loads of KPL packs with
+// The rows of a threadgroup of 256 threads, under 64 KPL packs each, by the
+// fewest packs a lane that hold the row (a pack past the row costs its products
+// all the same; a full row is gemv_xlds's own form).  MI355X, µs, by the loads of KPL packs with
 // x from memory (int8: by the loop) and so:
 //
 //   f32 4096 x 256      6.3  2.7    f16 4096 x 256      5.1  2.6
@@ -493,9 +493,7 @@ __device__ __forceinline__ void gemv_staged(const WT *__restrict__ w, const XT *
                                             const float *__restrict__ scale, float *__restrict__ y, uint32_t n,
                                             uint32_t k, uint32_t row0, uint4 *xs) {
   const uint32_t lanes = (k / P + FK_WAVE - 1) / FK_WAVE;  // packs a lane
-  if (k == FK_WAVE * KPL * P) {
-    gemv_xlds<WT, XT, P, R, KPL, true, 256>(w, x, scale, y, n, k, row0, xs);
-  } else if (lanes <= 1) {
+  if (lanes <= 1) {
     gemv_xlds<WT, XT, P, R, 1, false, 256>(w, x, scale, y, n, k, row0, xs);
   } else if (lanes <= 2) {
     gemv_xlds<WT, XT, P, R, 2, false, 256>(w, x, scale, y, n, k, row0, xs);
@@ -576,20 +574,6 @@ __device__ __forceinline__ void gemv_wide(const WT *__restrict__ w, const float 
       fk::gemv_wave<WT, XT, P, R>(w, x, nullptr, y, p.n, p.k, row0);                                         \
   }
 
-// Threadgroups of 256 with x staged in LDS, rows of at most 64 KPL packs: the
-// same sums.  (Entries of their own: beside the form above, the f16 row would
-// keep 110 registers where it needs 80.  Smaller threadgroups stage x more
-// often than they read it: f16 4096 x 4096 of 64 threads 11.6 µs, by the form
-// above 7.9, of 256 7.2 and 7.9.)
-#define FK_GEMV_STAGED_ENTRY(NAME, WT, XT, P, R, KPL)                                                        \
-  extern "C" __global__ void __launch_bounds__(256) NAME(const WT *__restrict__ w, const XT *__restrict__ x, \
-                                                         float *__restrict__ y, fk_gemv_params p) {         \
-    __shared__ uint4 xs[FK_WAVE * (KPL) * (P) * sizeof(XT) / 16];                                           \
-    static_assert(sizeof xs >= 256 * 16, "a chunk a thread");                                               \
-    const uint32_t row0 = (blockIdx.x * 4 + threadIdx.x / FK_WAVE) * (R);                                   \
-    fk::gemv_staged<WT, XT, P, R, KPL>(w, x, nullptr, y, p.n, p.k, row0, xs);                               \
-  }
-
 // The int8 entries: x staged in any threadgroup (64 threads, 8192 x 8192 by the
 // loop 35.9 µs, so 24.0; 128, 22.7 and 18.1), but rows of up to two packs a
 // lane, whose x is no more than the weights' bytes, and wider ones by the loop
@@ -603,7 +587,9 @@ __device__ __forceinline__ void gemv_wide(const WT *__restrict__ w, const float 
     static_assert(sizeof xs >= 256 * 16, "a chunk a thread");                                             \
     const uint32_t row0 = (blockIdx.x * (blockDim.x / FK_WAVE) + threadIdx.x / FK_WAVE) * (R);           \
     const uint32_t lanes = (p.k / (P) + FK_WAVE - 1) / FK_WAVE;                                           \
-    if (lanes > (KPL) || lanes <= 2) {                                                                     \
+    if (p.k == FK_WAVE * (KPL) * (P) && blockDim.x == 256) {                                               \
+      fk::gemv_xlds<WT, XT, P, R, KPL, true, 256>(w, x, scale, y, p.n, p.k, row0, xs);                    \
+    } else if (lanes > (KPL) || lanes <= 2) {                                                              \
       if (row0 < p.n) fk::gemv_wave<WT, XT, P, R>(w, x, scale, y, p.n, p.k, row0);                        \
     } else if (blockDim.x == 256) {                                                                        \
       fk::gemv_staged<WT, XT, P, R, KPL>(w, x, scale, y, p.n, p.k, row0, xs);                             \
@@ -675,12 +661,6 @@ FK_GEMV_ENTRY(fk_gemv_f32_f32_r4, float, float, 4, 4, 4)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r1, _Float16, float, 8, 1, 8)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r2, _Float16, float, 8, 2, 8)
 FK_GEMV_ENTRY(fk_gemv_f16_f32_r4, _Float16, float, 8, 4, 4)
-FK_GEMV_STAGED_ENTRY(fk_gemv_f32_f32_staged_r1, float, float, 4, 1, 16)
-FK_GEMV_STAGED_ENTRY(fk_gemv_f32_f32_staged_r2, float, float, 4, 2, 16)
-FK_GEMV_STAGED_ENTRY(fk_gemv_f32_f32_staged_r4, float, float, 4, 4, 4)
-FK_GEMV_STAGED_ENTRY(fk_gemv_f16_f32_staged_r1, _Float16, float, 8, 1, 8)
-FK_GEMV_STAGED_ENTRY(fk_gemv_f16_f32_staged_r2, _Float16, float, 8, 2, 8)
-FK_GEMV_STAGED_ENTRY(fk_gemv_f16_f32_staged_r4, _Float16, float, 8, 4, 4)
 FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r1, int8_t, _Float16, 16, 1, 8, 8)
 FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r2, int8_t, _Float16, 16, 2, 8, 1)
 FK_GEMV_SCALED_ENTRY(fk_gemv_i8_f16_r4, int8_t, _Float16, 16, 4, 4, 1)

@@ -12,3 +12,4 @@
 #include "fk_rows_norm.h"
 #include "fk_skinny.h"
 #include "fk_split_attend.h"
+#include "fk_gemv_staged.h"
