@@ -632,7 +632,7 @@ def paged_routed_table(dev, ks, eager: bool = False, reps: int = 50) -> dict:
     import numpy as np
 
     from furykernel_amd.engine import Engine
-    from furykernel_amd.lower import lower_plan
+    from furykernel_amd.lower import lower_plan, routed_fusions
     from furykernel_amd.program.build import program
     from furykernel_amd.program.check import check_program
     from furykernel_amd.program.graph import CACHE_F16, F16, F32, AttnSpec, Paged, Ring, RopeSpec, Shape, whole_row
@@ -733,7 +733,10 @@ def paged_routed_table(dev, ks, eager: bool = False, reps: int = 50) -> dict:
         us = timed(eng, low)
     finally:
         eng.close()
+    # the launches queued: each run that one launch does as that one
     entries = [l.entry for l in low.launches]
+    for first, n, l in reversed(routed_fusions(low)):
+        entries[first:first + n] = [l.entry]
     log(f"moe_step_2048_e16_f1024_k2: {entries}, {us:.2f} us a step, {nbytes / us / 1e3:.1f} GB/s")
     out["moe_step_2048_e16_f1024_k2"] = {"launches": entries, "avg_us": round(us, 3), "bytes": nbytes,
                                          "gbps": round(nbytes / us / 1e3, 1),
