@@ -196,6 +196,14 @@ SKINNY_COST = {"m1n1": (1.1, 0.037, False), "m1n2": (1.4, 0.054, False), "m2n1":
                "m2n2": (1.9, 0.056, False), "m2n4": (2.3, 0.089, False), "m4n2": (2.4, 0.074, True),
                "m4n4": (3.3, 0.110, False), "m4n8": (7.0, 0.150, True),
                "m8n8": (11.5, 0.202, True)}
+# Where it is another for a mode: m8n8's ring has one step for gate and up and
+# for the logits.  At k 4096 and more the cost above took m8n8, at 0.81 to 0.98
+# of fk_gemm's speed, for 2048 rows by 2 x 2048 (93 µs against 75) or 1408 by
+# 4096 logits (95 against 80), and m4n8 for gate and up at 0.93 of it (256 rows by
+# 2 x 12288: 91 against 84).  With these no pick was more than 2 % behind
+# fk_gemm at k 1024 to 16384, n 1536 to 16384 and 16 to 2048 rows.
+SKINNY_COST_OF = {"silu_mul": {"m4n8": (7.0, 0.155, True), "m8n8": (11.5, 0.275, True)},
+                  "store_keys": {"m8n8": (11.5, 0.275, True)}}
 
 
 def skinny_form(chunks: int, m: int, n: int, k: int, mode: str, splits: tuple = (1,)) -> Optional[tuple]:
@@ -208,7 +216,7 @@ def skinny_form(chunks: int, m: int, n: int, k: int, mode: str, splits: tuple = 
     - fk_gemm: its tiles in rounds of 256 (one a CU), 0.55 µs a step of 32
       columns and 11 a round, 17 with the residual's or QKV's epilogue (46
       and 52 at k 2048, 158 for down, whatever the rows);
-    - a form: 2 µs, and SKINNY_COST's for as many tiles as a CU takes, of a
+    - a form: 2 µs, and SKINNY_COST's (or SKINNY_COST_OF's) for as many tiles as a CU takes, of a
       split's share of the steps; and its partial sums' way to HBM and back
       at 4 TB/s.
 
@@ -226,13 +234,14 @@ def skinny_form(chunks: int, m: int, n: int, k: int, mode: str, splits: tuple = 
         return None
     steps = k / 32
     pairs = mode in SKINNY_PAIR_MODES
+    costs = {**SKINNY_COST, **SKINNY_COST_OF.get(mode, {})}
     ends = 11 if mode in ("store", "silu_mul", "store_keys") else 17
     least = -(-(m // SLAB) * (n // SLAB) // 256) * (ends + 0.55 * steps)
     best = None
     for form, (mb, nb, _) in SKINNY_FORMS.items():
         if mb >= 2 * chunks or (pairs and nb == 1):
             continue
-        tile, step, one = SKINNY_COST[form]
+        tile, step, one = costs[form]
         for parts in splits:
             share = -(-chunks // mb) * (n // (16 * nb)) * parts / 256
             share = max(1.0, float(np.ceil(share))) if one else (share + 0.25 if share > 1 else 1.0)
