@@ -200,8 +200,8 @@ SKINNY_COST = {"m1n1": (1.1, 0.037, False), "m1n2": (1.4, 0.054, False), "m2n1":
 # for the logits.  At k 4096 and more the cost above took m8n8, at 0.81 to 0.98
 # of fk_gemm's speed, for 2048 rows by 2 x 2048 (93 µs against 75) or 1408 by
 # 4096 logits (95 against 80), and m4n8 for gate and up at 0.93 of it (256 rows by
-# 2 x 12288: 91 against 84).  With these no pick was more than 2 % behind
-# fk_gemm at k 1024 to 16384, n 1536 to 16384 and 16 to 2048 rows.
+# 2 x 12288: 91 against 84).  With these the worst pick was 2.1 %
+# behind fk_gemm (k 1024 to 16384, n 256 to 16384, 16 to 2048 rows).
 SKINNY_COST_OF = {"silu_mul": {"m4n8": (7.0, 0.155, True), "m8n8": (11.5, 0.275, True)},
                   "store_keys": {"m8n8": (11.5, 0.275, True)}}
 
