@@ -106,8 +106,8 @@ def test_gemv_i8_ragged_rows_full_width(device, kernels, n, r, threads):
     """Full rows of 8192 with fewer rows than the last threadgroup holds: in
     256-thread groups x goes through LDS and every wavefront reaches its
     barrier (rows past n read row n - 1 and store nothing); smaller groups
-    take the loop form.  Bit for bit against the oracle, and y past n left
-    as it was."""
+    stage it too, by the general form.  Bit for bit against the oracle, and
+    y past n left as it was."""
     k = 8192
     rng = np.random.default_rng(n * 10 + r)
     w = rng.integers(-128, 128, (n, k)).astype(np.int8)
